@@ -129,7 +129,7 @@ size_t forward_workspace_fast(int B, int T, int H, int N, int dtype, int flags) 
 size_t backward_workspace(int B, int T, int H, int N, int dtype, int flags) {
     if (chunk_ok(B, T, H, N, dtype, flags)) return chunk_backward_workspace(B, T, H, cu_count());
     if (rec_shape(B, T, H, N, dtype, flags)) return wkv7_rec_bwd_workspace(B, T, H);
-    return seq_backward_workspace(B, H, N);
+    return seq_backward_workspace(B, T, H, N);
 }
 
 }  // namespace wkv7

@@ -51,7 +51,7 @@ struct Dec {
 
 void launch_seq_forward(const Fwd& p);
 void launch_seq_backward(const Bwd& p);
-size_t seq_backward_workspace(int B, int H, int N);
+size_t seq_backward_workspace(int B, int T, int H, int N);
 void launch_decode(const Dec& p);
 // bf16, N == 64; `cus` = CUs the schedule spreads the heads over
 void launch_chunk_forward(const Fwd& p, int cus);
