@@ -141,6 +141,10 @@ long long theseus_wkv7_checkpoint_count(int T);
  * shared by calls that may run at the same time. */
 size_t theseus_wkv7_forward_workspace_size(int B, int T, int H, int N, int dtype);
 size_t theseus_wkv7_backward_workspace_size(int B, int T, int H, int N, int dtype);
+/* The workspace with which a forward runs fastest, at least theseus_wkv7_forward_workspace_size:
+ * more for calls whose few heads leave CUs idle.  saved_states: whether ckpt is given.
+ *  - bf16, N = 128: the buffers of up to 9 time segments. */
+size_t theseus_wkv7_forward_best_workspace_size(int B, int T, int H, int N, int dtype, int saved_states);
 
 /* Forward recurrence.  Replaces wkv_forward (kernels/wkv7_state.cpp:16-25)
  * and launch_forward (kernels/wkv7_state.cu:81-86).

@@ -37,10 +37,10 @@
 // it, X_{c+1} = X_c M_c + U_c, so each head's chunks form k segments scanned at once.
 // Segment 0 starts from s0; segment s >= 1 carries two states in every wave, one from
 // zero (its output y0 and final U_s) and one from the identity with v = 0 (its output
-// z_t = Phi_t r_t and final Phi_s), both on the same record.  gdn_split_fixup then
-// chains X_{s+1} = X_s Phi_s + U_s and forms y_t = y0_t + X_s z_t.
-#include "wkv7_io.h"
+// z_t = Phi_t r_t and final Phi_s), both on the same record.  scan_chain then chains
+// X_{s+1} = X_s Phi_s + U_s and gdn_split_y forms y_t = y0_t + X_s z_t.
 #include "wkv7_launch.h"
+#include "wkv7_scan.h"
 
 namespace wkv7 {
 namespace {
@@ -62,7 +62,8 @@ struct GdnRec {
     static constexpr size_t BYTES = EL + (PK ? ((size_t)NK * 4 + 255) / 256 * 256 : 256);
     static constexpr int DMA_BLOCKS = (int)((BYTES + 1023) / 1024);  // 1 KB LDS DMA blocks
 };
-static_assert(GdnRec<128>::BYTES % 256 == 0 && GdnRec<64>::BYTES % 256 == 0 && GdnRec<128, true>::BYTES % 256 == 0,
+static_assert(GdnRec<128>::BYTES % 256 == 0 && GdnRec<64>::BYTES % 256 == 0 && GdnRec<128, true>::BYTES % 256 == 0 &&
+                  GdnRec<64, true>::BYTES % 256 == 0,
               "record alignment");
 
 // ---------------------------------------------------------------------------
@@ -229,16 +230,16 @@ __global__ __launch_bounds__(64) void gdn_prep(int Tn, int H, int qk_norm, const
             for (int e = 0; e < 4; e++) rt[e] = qr[ks][4 * u + e] * egam;  // R~[t][16tj + 4q4 + e]
             pP2T[u] = pk(rt + mm16s(pk(Pt), pBrbT));  // P2^T = R~^T + P^T Brb^T
             const Pk pb = pk(bhat), pkh = pk(khat);
-            uint4* uf = reinterpret_cast<uint4*>(rec + R::UF) + (size_t)(2 * tj) * 64 + lane;
-            uf[0] = cat(pb.h, pkh.h);
-            uf[64] = cat(pb.l, pkh.l);
+            uint8_t* uf = rec + R::UF + (size_t)(2 * tj) * 1024;
+            put_frag(uf, lane, cat(pb.h, pkh.h));
+            put_frag(uf + 1024, lane, cat(pb.l, pkh.l));
         }
-        uint4* pf = reinterpret_cast<uint4*>(rec + R::PF) + (size_t)(2 * ks) * 64 + lane;
-        pf[0] = cat(pPT[0].h, pPT[1].h);
-        pf[64] = cat(pPT[0].l, pPT[1].l);
-        uint4* p2 = reinterpret_cast<uint4*>(rec + R::P2F) + (size_t)(2 * ks) * 64 + lane;
-        p2[0] = cat(pP2T[0].h, pP2T[1].h);
-        p2[64] = cat(pP2T[0].l, pP2T[1].l);
+        uint8_t* pf = rec + R::PF + (size_t)(2 * ks) * 1024;
+        put_frag(pf, lane, cat(pPT[0].h, pPT[1].h));
+        put_frag(pf + 1024, lane, cat(pPT[0].l, pPT[1].l));
+        uint8_t* p2 = rec + R::P2F + (size_t)(2 * ks) * 1024;
+        put_frag(p2, lane, cat(pP2T[0].h, pP2T[1].h));
+        put_frag(p2 + 1024, lane, cat(pP2T[0].l, pP2T[1].l));
     }
 }
 
@@ -375,16 +376,16 @@ __global__ __launch_bounds__(64) void wkv7_rec_prep(int Tn, int H, const bf16_t*
             for (int e = 0; e < 4; e++) rr4[e] = rt[ks][4 * u + e];
             pP2T[u] = pk(rr4 + mm16s(pk(Pt), pBrbT));  // P2^T = R~^T + P^T Brb^T
             const Pk pb4 = pk(bhat), pk4 = pk(khat);
-            uint4* uf = reinterpret_cast<uint4*>(rec + R::UF) + (size_t)(2 * tj) * 64 + lane;
-            uf[0] = cat(pb4.h, pk4.h);
-            uf[64] = cat(pb4.l, pk4.l);
+            uint8_t* uf = rec + R::UF + (size_t)(2 * tj) * 1024;
+            put_frag(uf, lane, cat(pb4.h, pk4.h));
+            put_frag(uf + 1024, lane, cat(pb4.l, pk4.l));
         }
-        uint4* pf = reinterpret_cast<uint4*>(rec + R::PF) + (size_t)(2 * ks) * 64 + lane;
-        pf[0] = cat(pPT[0].h, pPT[1].h);
-        pf[64] = cat(pPT[0].l, pPT[1].l);
-        uint4* p2 = reinterpret_cast<uint4*>(rec + R::P2F) + (size_t)(2 * ks) * 64 + lane;
-        p2[0] = cat(pP2T[0].h, pP2T[1].h);
-        p2[64] = cat(pP2T[0].l, pP2T[1].l);
+        uint8_t* pf = rec + R::PF + (size_t)(2 * ks) * 1024;
+        put_frag(pf, lane, cat(pPT[0].h, pPT[1].h));
+        put_frag(pf + 1024, lane, cat(pPT[0].l, pPT[1].l));
+        uint8_t* p2 = rec + R::P2F + (size_t)(2 * ks) * 1024;
+        put_frag(p2, lane, cat(pP2T[0].h, pP2T[1].h));
+        put_frag(p2 + 1024, lane, cat(pP2T[0].l, pP2T[1].l));
     }
 }
 
@@ -397,41 +398,38 @@ __global__ __launch_bounds__(64) void wkv7_rec_prep(int Tn, int H, const bf16_t*
 // double-buffered in LDS: chunk c + 1's comes in by DMA (each wave moves every NW-th
 // kilobyte) while chunk c's is read; one barrier per chunk.
 // ---------------------------------------------------------------------------
-// The time split's buffers (float32): X_1 [BH][N][N] (internal [value][key] layout), U_s
-// and Phi_s [k - 1][BH][N][N], and the y0 and z tiles [k - 1][BH][m][N/16 row blocks][64
-// lanes][4] (lane (q4, r16) of row block rb: y[4q4 + e][16rb + r16]).
-struct GdnSplit {
-    int m = 0, k = 0;  // chunks of each segment after the first, segments
-    int m0 = 0;        // chunks of segment 0
-    float *send0 = nullptr, *uend = nullptr, *phi = nullptr, *y0 = nullptr, *z = nullptr;
-};
-
+// MODE: SCAN_TILES cuts the chunks in segments 0 .. k-1 that run at once, the later ones in
+// two states whose y0 and z tiles ([k - 1][BH][m][N/16 row blocks][64 lanes][4], lane (q4, r16)
+// of row block rb: y[4q4 + e][16rb + r16]) gdn_split_y joins; SCAN_ENDS and SCAN_RESUME are the
+// two launches of the split with saved states (wkv7_scan.h).
 // PK: WKV7 records (a decay per key: the state's key columns scale by e^{g_L} each);
-// ckpt (not with SPLIT; may be null): the state at every chunk's start and the final one,
+// ckpt (not with SCAN_TILES; may be null): the state at every chunk's start and the final one,
 // [bh][count][value][key] as the step-serial kernels keep saved states.
-template <int NK, typename TO, bool SPLIT, bool PK = false>
-__global__ __launch_bounds__(256) void gdn_scan(int Tn, int H, int BH, int kv, const float* __restrict__ s0,
+template <int NK, typename TO, ScanMode MODE, bool PK = false>
+__global__ __launch_bounds__(4 * NK) void gdn_scan(int Tn, int H, int BH, int kv, const float* __restrict__ s0,
                                                    TO* __restrict__ o, float* __restrict__ sT,
-                                                   const uint8_t* __restrict__ ws, GdnSplit sp,
+                                                   const uint8_t* __restrict__ ws, ScanSplit sp,
                                                    float* __restrict__ ckpt) {
     using R = GdnRec<NK, PK>;
     constexpr int KS = R::KS, TJ = R::TJ;
     __shared__ __attribute__((aligned(1024))) uint8_t recs[2][R::DMA_BLOCKS * 1024];
-    // workgroup (segment * row groups + rg) * BH + bh (SPLIT; else rg * BH + bh)
-    constexpr int RGS = NK / 64;
-    const int bh = blockIdx.x % BH, rest = blockIdx.x / BH, rg = SPLIT ? rest % RGS : rest;
-    const int sgm = SPLIT ? rest / RGS : 0, bb = bh / H, h = bh - bb * H;
-    const bool dual = SPLIT && sgm > 0;  // the zero and identity runs
+    // workgroup (segment * row groups + rg) * BH + bh
+    // waves per workgroup (the host launches whole waves, at least one: the DMA loop steps by
+    // NW) and row groups per head
+    const int NW = max(1, __builtin_amdgcn_readfirstlane((int)(blockDim.x >> 6))), RGS = NK / 16 / NW;
+    constexpr bool DUALS = MODE == SCAN_TILES || MODE == SCAN_ENDS;
+    const int bh = blockIdx.x % BH, rest = blockIdx.x / BH, rg = rest % RGS, bb = bh / H, h = bh - bb * H;
+    const int sgm = DUALS ? rest / RGS : MODE == SCAN_RESUME ? 1 + rest / RGS : 0;
+    const bool dual = DUALS && sgm > 0;  // the zero and identity runs
+    const bool outs = MODE != SCAN_ENDS || !dual;  // forms y (and saves states)
     const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // waves per group (the host launches whole waves, at least one: the DMA loop steps by NW)
-    const int NW = max(1, __builtin_amdgcn_readfirstlane((int)(blockDim.x >> 6)));
     const int lane = tid & 63, q4 = lane >> 4, r16 = lane & 15;
     const int rb = rg * NW + wv, i_own = 16 * rb + r16;
     const long NN = (long)NK * NK, ei = kv ? 1 : NK, ej = kv ? NK : 1;
     const int nchunk = (Tn + GC - 1) / GC;
     // this segment's chunks (segment 0: m0, the others m)
-    const int c0 = SPLIT ? (sgm == 0 ? 0 : sp.m0 + (sgm - 1) * sp.m) : 0;
-    const int c1 = SPLIT ? min(nchunk, c0 + (sgm == 0 ? sp.m0 : sp.m)) : nchunk;
+    const int c0 = MODE == SCAN_ALL || sgm == 0 ? 0 : sp.m0 + (sgm - 1) * sp.m;
+    const int c1 = MODE == SCAN_ALL ? nchunk : min(nchunk, c0 + (sgm == 0 ? sp.m0 : sp.m));
     // this head's records (the host keeps them under 4 GB, so 32-bit offsets reach them)
     const i32x4_t rs = dma_rsrc(ws + (size_t)bh * nchunk * R::BYTES, (uint32_t)((size_t)nchunk * R::BYTES));
     auto fetch = [&](int c, int buf) {
@@ -446,7 +444,10 @@ __global__ __launch_bounds__(256) void gdn_scan(int Tn, int H, int BH, int kv, c
     for (int tj = 0; tj < TJ; tj++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            St[tj][e] = dual ? 0.f : s0[bh * NN + i_own * ei + (16 * tj + 4 * q4 + e) * ej];
+            if (MODE != SCAN_RESUME)
+                St[tj][e] = dual ? 0.f : s0[bh * NN + i_own * ei + (16 * tj + 4 * q4 + e) * ej];
+            else
+                St[tj][e] = seg_state(sp, BH, bh, sgm, NN)[(long)i_own * NK + 16 * tj + 4 * q4 + e];
             Sp[tj][e] = i_own == 16 * tj + 4 * q4 + e ? 1.f : 0.f;
         }
     vm_wait0();
@@ -456,9 +457,19 @@ __global__ __launch_bounds__(256) void gdn_scan(int Tn, int H, int BH, int kv, c
     // LDS, each of its TJ stores writes 1 KB of them (from the registers, each would write
     // 64-byte pieces of 16 rows)
     constexpr int SQ = NK + 4;  // padded row (floats)
-    __shared__ __attribute__((aligned(16))) float sq[SPLIT ? 1 : 4][SPLIT ? 4 : 16 * SQ];
+    // (the WKV7 operator's N = 64 states are kept in the chunked kernels' tiled order, which is
+    // the registers': whole KBs without the regrouping)
+    constexpr bool TILED = PK && NK == 64;
+    __shared__ __attribute__((aligned(16))) float sq[MODE == SCAN_TILES ? 1 : TJ][MODE == SCAN_TILES ? 4 : 16 * SQ];
     auto save = [&](int slot) {
-        if constexpr (!SPLIT) {
+        if (TILED && slot < nchunk) {
+            float* const dst = ckpt + ((long)bh * ncp + slot) * NN + (long)rb * TJ * 256 + 4 * lane;
+#pragma unroll
+            for (int tj = 0; tj < TJ; tj++)
+                *reinterpret_cast<float4*>(dst + 256 * tj) = make_float4(St[tj][0], St[tj][1], St[tj][2], St[tj][3]);
+            return;
+        }
+        if constexpr (MODE != SCAN_TILES) {
             float* const q = sq[wv];
 #pragma unroll
             for (int tj = 0; tj < TJ; tj++)
@@ -485,17 +496,18 @@ __global__ __launch_bounds__(256) void gdn_scan(int Tn, int H, int BH, int kv, c
                                  St[2 * ks + 1][0], St[2 * ks + 1][1], St[2 * ks + 1][2], St[2 * ks + 1][3]};
             uint4 sh, sl;
             pack8(sv, sh, sl);
-            const uint4* pf = reinterpret_cast<const uint4*>(rec + R::PF) + (2 * ks) * 64 + lane;
-            const uint4* p2 = reinterpret_cast<const uint4*>(rec + R::P2F) + (2 * ks) * 64 + lane;
-            const uint4 ph = pf[0], pl = pf[64], p2h = p2[0], p2l = p2[64];
+            const uint8_t* pf = rec + R::PF + (2 * ks) * 1024;
+            const uint8_t* p2 = rec + R::P2F + (2 * ks) * 1024;
+            const uint4 ph = get_frag(pf, lane), pl = get_frag(pf + 1024, lane);
+            const uint4 p2h = get_frag(p2, lane), p2l = get_frag(p2 + 1024, lane);
             sa = mma32(mma32(mma32(sa, ph, sh), ph, sl), pl, sh);
-            yy = mma32(mma32(mma32(yy, p2h, sh), p2h, sl), p2l, sh);
+            if (outs) yy = mma32(mma32(mma32(yy, p2h, sh), p2h, sl), p2l, sh);
             if (dual) {  // the identity run on the same record
                 const float sw[8] = {Sp[2 * ks][0], Sp[2 * ks][1], Sp[2 * ks][2], Sp[2 * ks][3],
                                      Sp[2 * ks + 1][0], Sp[2 * ks + 1][1], Sp[2 * ks + 1][2], Sp[2 * ks + 1][3]};
                 pack8(sw, sh, sl);
                 sa2 = mma32(mma32(mma32(sa2, ph, sh), ph, sl), pl, sh);
-                yy2 = mma32(mma32(mma32(yy2, p2h, sh), p2h, sl), p2l, sh);
+                if (MODE == SCAN_TILES) yy2 = mma32(mma32(mma32(yy2, p2h, sh), p2h, sl), p2l, sh);
             }
         }
         // + Q' V and Q2 V on the K=16 instruction, in their own accumulators
@@ -505,7 +517,7 @@ __global__ __launch_bounds__(256) void gdn_scan(int Tn, int H, int BH, int kv, c
             const uint2* qf = reinterpret_cast<const uint2*>(rec + R::QF) + lane;
             const uint2 q1h = qf[0], q1l = qf[64], q2h = qf[128], q2l = qf[192];
             sa += mma16(mma16(mma16(zero4(), q1h, vh), q1h, vl), q1l, vh);
-            yy += mma16(mma16(mma16(zero4(), q2h, vh), q2h, vl), q2l, vh);
+            if (outs) yy += mma16(mma16(mma16(zero4(), q2h, vh), q2h, vl), q2l, vh);
         }
         if (!dual) {
 #pragma unroll
@@ -513,7 +525,7 @@ __global__ __launch_bounds__(256) void gdn_scan(int Tn, int H, int BH, int kv, c
                 const int t = 4 * q4 + e;
                 if (t < L) io<TO>::st(o, ((tok0 + t) * H + h) * NK + i_own, yy[e]);
             }
-        } else {  // the tiles for gdn_split_fixup
+        } else if (MODE == SCAN_TILES) {  // the tiles for gdn_split_y
             const long f4 = ((((long)(sgm - 1) * BH + bh) * sp.m + (c - c0)) * TJ + rb) * 64 + lane;
             reinterpret_cast<float4*>(sp.y0)[f4] = make_float4(yy[0], yy[1], yy[2], yy[3]);
             reinterpret_cast<float4*>(sp.z)[f4] = make_float4(yy2[0], yy2[1], yy2[2], yy2[3]);
@@ -522,7 +534,7 @@ __global__ __launch_bounds__(256) void gdn_scan(int Tn, int H, int BH, int kv, c
         // below lets these TJ stores stay in flight (a vmcnt(0) there had waited for every
         // store to complete each chunk: 0.49 -> 0.23 ms of scan at B=4, T=2048, H=32, N=128
         // without them)
-        if (!SPLIT && ckpt) save(c);
+        if (MODE != SCAN_TILES && outs && ckpt) save(c);
         // X^T <- e^{gamma_L} X^T + [B^^T K^^T] [SA; V]   (K = 32: SA rows, then V rows;
         // the identity run has no V rows)
         uint2 sah, sal, sah2, sal2;
@@ -533,21 +545,31 @@ __global__ __launch_bounds__(256) void gdn_scan(int Tn, int H, int BH, int kv, c
         const float egL = *reinterpret_cast<const float*>(rec + R::EL);
 #pragma unroll
         for (int tj = 0; tj < TJ; tj++) {
-            const uint4* uf = reinterpret_cast<const uint4*>(rec + R::UF) + (2 * tj) * 64 + lane;
-            const uint4 ah = uf[0], al = uf[64];
+            const uint8_t* uf = rec + R::UF + (2 * tj) * 1024;
+            const uint4 ah = get_frag(uf, lane), al = get_frag(uf + 1024, lane);
             // the decay of the lane's keys 16 tj + 4 q4 + e (one for all keys unless PK)
             const f32x4_t eg = PK ? *reinterpret_cast<const f32x4_t*>(rec + R::EL + 4 * (16 * tj + 4 * q4))
                                   : f32x4_t{egL, egL, egL, egL};
             St[tj] = mma32(mma32(mma32(St[tj] * eg, ah, bhi), ah, blo), al, bhi);
             if (dual) Sp[tj] = mma32(mma32(mma32(Sp[tj] * eg, ah, bhi2), ah, blo2), al, bhi2);
         }
-        // this wave's part of the next record is in LDS (the DMA precedes the saved-state
-        // stores, and the memory counter completes in order)
-        if (!SPLIT && ckpt) vm_wait_n<TJ>();
-        else vm_wait0();
+        // this wave's part of the next record is in LDS.  The memory counter completes in
+        // order, so the stores issued after that DMA are counted out of the wait and stay in
+        // flight: a tile pair, or a full chunk's four y stores and the saved state's TJ
+        if (dual) {
+            if (MODE == SCAN_TILES) vm_wait_n<2>();
+            else vm_wait0();
+        } else if (MODE != SCAN_TILES && ckpt) {
+            if (L == GC) vm_wait_n<TJ + 4>();
+            else vm_wait_n<TJ>();
+        } else {
+            if (L == GC) vm_wait_n<4>();
+            else vm_wait0();
+        }
         __syncthreads();  // every wave's part is, and nobody still reads this one
     }
-    if (!SPLIT) {
+    if (!DUALS) {
+        if (c1 < nchunk) return;  // (only the last chunk's segment ends the head)
         if (ckpt) save(nchunk);
 #pragma unroll
         for (int tj = 0; tj < TJ; tj++)
@@ -559,22 +581,20 @@ __global__ __launch_bounds__(256) void gdn_scan(int Tn, int H, int BH, int kv, c
 #pragma unroll
         for (int tj = 0; tj < TJ; tj++) {
             *reinterpret_cast<float4*>(dst + o4 + 16 * tj + 4 * q4) = make_float4(St[tj][0], St[tj][1], St[tj][2], St[tj][3]);
-            if (dual)
-                *reinterpret_cast<float4*>(sp.phi + o4 + 16 * tj + 4 * q4) =
-                    make_float4(Sp[tj][0], Sp[tj][1], Sp[tj][2], Sp[tj][3]);
+            if (dual)  // (transposed, as scan_chain reads it)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    sp.phi[((long)(sgm - 1) * BH + bh) * NN + (long)(16 * tj + 4 * q4 + e) * NK + i_own] = Sp[tj][e];
         }
     }
 }
 
 // ---------------------------------------------------------------------------
-// The time split's fix-up, two kernels.  gdn_split_chain (one workgroup per head, N/16
-// waves, wave w on rows 16w .. 16w+15) chains X_{s+1} = X_s Phi_s + U_s in LDS on the
-// matrix cores (split-bf16 operands), storing X_{s+1} over U_s (which only it reads; the
-// same lane reads each U element before writing it) and X_k as sT in the caller's
-// layout.  Phi_s (as split B operands in LDS) and U_s (registers) come one step ahead.  gdn_split_y then forms y_t = y0_t + X_s z_t for every chunk of segments
-// 1 .. k-1: workgroup (chunk group, head), wave w keeps output columns 16w .. 16w+15
-// (rows of X_s as its B operand in registers); per chunk the z tile is turned into rows in
-// LDS, y0 comes in the accumulator layout, o leaves in whole rows through LDS.
+// The SCAN_TILES split's fix-up: scan_chain (wkv7_scan.h) forms every segment's true start
+// and sT, then gdn_split_y y_t = y0_t + X_s z_t for every chunk of segments 1 .. k-1:
+// workgroup (chunk group, head), wave w keeps output columns 16w .. 16w+15 (rows of X_s as
+// its B operand in registers); per chunk the z tile is turned into rows in LDS, y0 comes in
+// the accumulator layout, o leaves in whole rows through LDS.
 // ---------------------------------------------------------------------------
 constexpr int GFY = 8;  // chunks per gdn_split_y workgroup (2 measured slower: 21.6 against 19.3 us)
 __device__ __forceinline__ void op8f(const float* p, uint4& hi, uint4& lo) {  // 8 floats, split
@@ -582,105 +602,8 @@ __device__ __forceinline__ void op8f(const float* p, uint4& hi, uint4& lo) {  //
     const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
     pack8(v, hi, lo);
 }
-// X_s of segment s >= 1: X_1 in send0, X_s (s >= 2) in the U_{s-1} slot
-__device__ __forceinline__ const float* seg_state(const GdnSplit& sp, int BH, int bh, int s, long NN) {
-    return s == 1 ? sp.send0 + bh * NN : sp.uend + ((long)(s - 2) * BH + bh) * NN;
-}
-
-template <int NK>
-__global__ __launch_bounds__(64 * (NK / 16)) void gdn_split_chain(int BH, int kv, GdnSplit sp, float* __restrict__ sT) {
-    constexpr int KS = NK / 32, TJ = NK / 16, XR = NK + 4, NT = 64 * TJ;
-    __shared__ float st[NK * XR];              // X_s [i][j]
-    __shared__ uint4 fr[TJ * KS * 2 * 64];     // Phi_s as split B operands [n][t][hi, lo][lane]
-    const int bh = blockIdx.x, tid = threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-    const int q = lane >> 4, r16 = lane & 15;
-    const long NN = (long)NK * NK;
-    // Fragment entries (n, t, lane') = KS per thread, number v*NT + tid: Phi[32t + 8q' + e][16n + r']
-    // for e = 0..7, loaded a step ahead and split once here, not by every wave.  (Plain
-    // float arrays in macros: arrays behind lambdas end up in scratch memory.)
-    float pv[KS][8];
-    float uf[TJ][4];  // U_u[16w + 4q + e][16n + r16]
-#define GDN_CHAIN_LOAD(u_)                                                                                    \
-    do {                                                                                                      \
-        const long ol_ = ((long)((u_) - 1) * BH + bh) * NN;                                                   \
-        _Pragma("unroll") for (int v = 0; v < KS; v++) {                                                      \
-            const int x_ = v * NT + tid, l_ = x_ & 63, t_ = (x_ >> 6) % KS, n_ = (x_ >> 6) / KS;              \
-            _Pragma("unroll") for (int e = 0; e < 8; e++)                                                     \
-                pv[v][e] = sp.phi[ol_ + (32 * t_ + 8 * (l_ >> 4) + e) * NK + 16 * n_ + (l_ & 15)];            \
-        }                                                                                                     \
-        _Pragma("unroll") for (int n = 0; n < TJ; n++)                                                        \
-            _Pragma("unroll") for (int e = 0; e < 4; e++) uf[n][e] = sp.uend[ol_ + (16 * w + 4 * q + e) * NK + 16 * n + r16]; \
-    } while (0)
-#define GDN_CHAIN_STAGE()                                                                                     \
-    do {                                                                                                      \
-        _Pragma("unroll") for (int v = 0; v < KS; v++) {                                                      \
-            const int x_ = v * NT + tid, l_ = x_ & 63, f_ = x_ >> 6;                                          \
-            uint4 h_, lo_;                                                                                    \
-            pack8(pv[v], h_, lo_);                                                                            \
-            fr[(2 * f_) * 64 + l_] = h_;                                                                      \
-            fr[(2 * f_ + 1) * 64 + l_] = lo_;                                                                 \
-        }                                                                                                     \
-    } while (0)
-#pragma unroll
-    for (int u = 0; u < NK / 16; u++) {  // rows 16w .. 16w+15 of X_1 (float4 u*64 + lane of the strip)
-        const int f = 4 * (u * 64 + lane), r = 16 * w + f / NK, c = f % NK;
-        *reinterpret_cast<float4*>(&st[r * XR + c]) = *reinterpret_cast<const float4*>(sp.send0 + bh * NN + r * NK + c);
-    }
-    GDN_CHAIN_LOAD(1);
-    GDN_CHAIN_STAGE();
-    __syncthreads();
-    for (int u = 1; u < sp.k; u++) {  // X_{u+1} = X_u Phi_u + U_u, this wave's rows
-        const long ob = ((long)(u - 1) * BH + bh) * NN;
-        float acc0[TJ][4];
-#pragma unroll
-        for (int n = 0; n < TJ; n++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc0[n][e] = uf[n][e];
-        if (u + 1 < sp.k) GDN_CHAIN_LOAD(u + 1);  // the next step's operands, in flight during this one
-        uint4 ah[KS], al[KS];  // A operand X_u: lane (q, r16) holds X_u[16w + r16][32t + 8q .. +7]
-#pragma unroll
-        for (int t = 0; t < KS; t++) op8f(&st[(16 * w + r16) * XR + 32 * t + 8 * q], ah[t], al[t]);
-        wave_lds_fence();  // (the strip is overwritten below)
-        // the TJ output tiles' products interleaved (independent accumulator chains)
-        f32x4_t acc[TJ];
-#pragma unroll
-        for (int n = 0; n < TJ; n++) acc[n] = f32x4_t{acc0[n][0], acc0[n][1], acc0[n][2], acc0[n][3]};
-#pragma unroll
-        for (int t = 0; t < KS; t++)
-#pragma unroll
-            for (int n = 0; n < TJ; n++) {
-                const uint4 bhv = fr[(2 * (n * KS + t)) * 64 + lane], blv = fr[(2 * (n * KS + t) + 1) * 64 + lane];
-                acc[n] = mma32(acc[n], ah[t], bhv);
-                acc[n] = mma32(acc[n], ah[t], blv);
-                acc[n] = mma32(acc[n], al[t], bhv);
-            }
-#pragma unroll
-        for (int n = 0; n < TJ; n++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                st[(16 * w + 4 * q + e) * XR + 16 * n + r16] = acc[n][e];
-                if (u + 1 < sp.k) sp.uend[ob + (16 * w + 4 * q + e) * NK + 16 * n + r16] = acc[n][e];  // X_{u+1}
-            }
-        __syncthreads();  // everyone is done with Phi_u
-        if (u + 1 < sp.k) GDN_CHAIN_STAGE();
-        __syncthreads();  // (and, after the last step, every row of X_k is in st)
-    }
-#undef GDN_CHAIN_LOAD
-#undef GDN_CHAIN_STAGE
-    // sT = X_k in the caller's layout, whole rows: float4 number v*NT + tid of row a,
-    // columns c .. c+3 (kv: sT[a = j][c = i] = X[i][j], read down a column of st)
-#pragma unroll
-    for (int v = 0; v < NK * NK / 4 / NT; v++) {
-        const int f = 4 * (v * NT + tid), a = f / NK, c = f % NK;
-        const float4 x = kv ? make_float4(st[c * XR + a], st[(c + 1) * XR + a], st[(c + 2) * XR + a], st[(c + 3) * XR + a])
-                            : *reinterpret_cast<const float4*>(&st[a * XR + c]);
-        *reinterpret_cast<float4*>(sT + bh * NN + f) = x;
-    }
-}
-
 template <int NK, typename TO>
-__global__ __launch_bounds__(64 * (NK / 16)) void gdn_split_y(int Tn, int H, int BH, GdnSplit sp, TO* __restrict__ o) {
+__global__ __launch_bounds__(64 * (NK / 16)) void gdn_split_y(int Tn, int H, int BH, ScanSplit sp, TO* __restrict__ o) {
     constexpr int KS = NK / 32, TJ = NK / 16, XR = NK + 4, NT = 64 * TJ;
     __shared__ float zt[GC * XR];    // the chunk's z tile as rows [t][j]
     __shared__ TO yt[GC * NK];       // its o tile [t][i]
@@ -766,9 +689,9 @@ int gdn_split_segments(int B, int T, int H, int N, int cus) {
     if (n < 8 || per < 1) return 1;
     return max(1, min(min(4, cus / per), n));
 }
+// The records and the buffers of a split without saved states in k segments.
 template <bool PK>
-static size_t split_workspace(int B, int T, int H, int N, int cus) {
-    const int k = gdn_split_segments(B, T, H, N, cus);
+static size_t tiles_workspace(int B, int T, int H, int N, int k) {
     if (k < 2) return records<PK>(B, T, H, N);
     int m0, mi;
     gdn_split_lengths((T + GC - 1) / GC, k, m0, mi);
@@ -776,43 +699,70 @@ static size_t split_workspace(int B, int T, int H, int N, int cus) {
     const size_t recs = (records<PK>(B, T, H, N) + 255) / 256 * 256;
     return recs + BH * ((2 * k - 1) * NN + 2 * (k - 1) * m * GC * N) * sizeof(float);
 }
+// As many segments as one workgroup of all of a head's rows per CU allows, at most 8; the
+// default workspace size holds the buffers of gdn_split_segments of them.
+static int tiles_segments(int B, int T, int H, int cus) {
+    const int n = (T + GC - 1) / GC;
+    return n < 8 ? 1 : max(1, min(min(8, cus / (B * H)), n));
+}
+size_t gdn_forward_workspace_fast(int B, int T, int H, int N, int cus) {
+    return tiles_workspace<false>(B, T, H, N, tiles_segments(B, T, H, cus));
+}
+size_t wkv7_rec_workspace_fast(int B, int T, int H, int N, int cus) {
+    return tiles_workspace<true>(B, T, H, N, tiles_segments(B, T, H, cus));
+}
 size_t gdn_forward_workspace_split(int B, int T, int H, int N, int cus) {
-    return split_workspace<false>(B, T, H, N, cus);
+    return tiles_workspace<false>(B, T, H, N, gdn_split_segments(B, T, H, N, cus));
 }
 size_t wkv7_rec_workspace(int B, int T, int H, int N) { return records<true>(B, T, H, N); }
-size_t wkv7_rec_workspace_split(int B, int T, int H, int N, int cus) { return split_workspace<true>(B, T, H, N, cus); }
 
-// Row groups per head for the scan: groups of four waves (64 value rows).  Measured at
+// Row groups per head for the one-pass scan: groups of four waves (64 value rows).  Measured at
 // B=1, T=2048 (MI355X): N=128 in 2 groups 0.248 ms against 0.279 (1), 0.292 (4) and
 // 0.380 (8); N=64 in 1 group 0.168 ms against 0.192 (2) -- every group moves the whole
 // record into its LDS, and groups of fewer waves wait on that more than they gain.
-static int gdn_row_groups(int N) { return N / 64; }  // (256 lanes each: the kernel's bound)
+static int gdn_row_groups(int N) { return N / 64; }
 
-// The scan over the records at ws: in one pass (with saved states when ckpt), or cut in
-// time when cus allows at least two segments and ws_bytes covers the split's buffers.
+// The scan over the records at ws: in one pass, or cut in time when cus allows and ws_bytes
+// covers the buffers, in as many segments as both allow.
 template <int NK, typename TO, bool PK>
 static void scan_records(int B, int T, int H, int kv, const float* s0, TO* o, float* sT, float* ckpt, void* ws,
                          size_t ws_bytes, int cus, hipStream_t stream) {
     const int nchunk = (T + GC - 1) / GC, BH = B * H;
-    const int rgs = gdn_row_groups(NK), lanes = 64 * (NK / 16) / rgs;
     const uint8_t* const recs = static_cast<const uint8_t*>(ws);
-    const int k = ckpt ? 1 : gdn_split_segments(B, T, H, NK, cus);
-    if (k < 2 || ws_bytes < split_workspace<PK>(B, T, H, NK, cus)) {
-        hipLaunchKernelGGL((gdn_scan<NK, TO, false, PK>), dim3(BH * rgs), dim3(lanes), 0, stream, T, H, BH, kv, s0, o,
-                           sT, recs, GdnSplit{}, ckpt);
+    const size_t rec_bytes = (records<PK>(B, T, H, NK) + 255) / 256 * 256;
+    float* const base = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + rec_bytes);  // buffers after the records
+    if (ckpt) {
+        int k = resume_segments(BH, NK, nchunk, cus);
+        while (k >= 4 && rec_bytes + resume_bytes(BH, NK, k) > ws_bytes) k--;
+        if (k >= 4) {
+            const ScanSplit sp = resume_split(BH, NK, nchunk, k, base);
+            const int rgs = scan_groups(BH, NK, k - 1, cus), lanes = 4 * NK / rgs;
+            hipLaunchKernelGGL((gdn_scan<NK, TO, SCAN_ENDS, PK>), dim3((k - 1) * BH * rgs), dim3(lanes), 0, stream, T, H,
+                               BH, kv, s0, o, sT, recs, sp, ckpt);
+            hipLaunchKernelGGL((scan_chain<NK>), dim3(BH, NK / 16), dim3(4 * NK), 0, stream, BH, k - 2, kv, sp, nullptr);
+            hipLaunchKernelGGL((gdn_scan<NK, TO, SCAN_RESUME, PK>), dim3((k - 1) * BH * rgs), dim3(lanes), 0, stream, T,
+                               H, BH, kv, s0, o, sT, recs, sp, ckpt);
+            return;
+        }
+    }
+    int k = ckpt ? 1 : tiles_segments(B, T, H, cus);
+    while (k >= 2 && tiles_workspace<PK>(B, T, H, NK, k) > ws_bytes) k--;
+    if (k < 2) {
+        const int rgs = gdn_row_groups(NK);
+        hipLaunchKernelGGL((gdn_scan<NK, TO, SCAN_ALL, PK>), dim3(BH * rgs), dim3(4 * NK / rgs), 0, stream, T, H, BH, kv,
+                           s0, o, sT, recs, ScanSplit{}, ckpt);
         return;
     }
-    // the time split: buffers after the records
-    GdnSplit sp;
+    ScanSplit sp;
     sp.k = k;
     gdn_split_lengths(nchunk, k, sp.m0, sp.m);
+    const int rgs = scan_groups(BH, NK, k, cus);
     const size_t NN = (size_t)NK * NK, per = (size_t)(k - 1) * BH;
-    float* const base = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + (records<PK>(B, T, H, NK) + 255) / 256 * 256);
     sp.send0 = base, sp.uend = base + BH * NN, sp.phi = sp.uend + per * NN;
     sp.y0 = sp.phi + per * NN, sp.z = sp.y0 + per * sp.m * GC * NK;
-    hipLaunchKernelGGL((gdn_scan<NK, TO, true, PK>), dim3(k * BH * rgs), dim3(lanes), 0, stream, T, H, BH, kv, s0, o,
-                       sT, recs, sp, nullptr);
-    hipLaunchKernelGGL((gdn_split_chain<NK>), dim3(BH), dim3(64 * (NK / 16)), 0, stream, BH, kv, sp, sT);
+    hipLaunchKernelGGL((gdn_scan<NK, TO, SCAN_TILES, PK>), dim3(k * BH * rgs), dim3(4 * NK / rgs), 0, stream, T, H, BH, kv,
+                       s0, o, sT, recs, sp, nullptr);
+    hipLaunchKernelGGL((scan_chain<NK>), dim3(BH, NK / 16), dim3(4 * NK), 0, stream, BH, k - 1, kv, sp, sT);
     // chunk groups of segments 1 .. k-1; heads along y
     hipLaunchKernelGGL((gdn_split_y<NK, TO>), dim3((k - 1) * ((sp.m + GFY - 1) / GFY), BH), dim3(64 * (NK / 16)), 0,
                        stream, T, H, BH, sp, o);
@@ -836,17 +786,28 @@ void launch_gdn_forward(const Gdn& p) {
     }
 }
 
-// The WKV7 forward on records: bf16, N = 128, flags 0 ([value][key] states), a
-// workspace of at least wkv7_rec_workspace bytes; saved states (ckpt) in the step-serial
-// kernels' [value][key] order.
-void launch_wkv7_rec_forward(const Fwd& p, int cus) {
+// The WKV7 forward on records: bf16, N = 128 or 64, flags 0 ([value][key] states), a
+// workspace of at least wkv7_rec_workspace bytes; saved states (ckpt) at N = 128 in the
+// step-serial kernels' [value][key] order, at N = 64 in the chunked kernels' tiled order.
+template <int NK> static void launch_rec_fwd(const Fwd& p, int cus) {
     const int nchunk = (p.T + GC - 1) / GC, BH = p.B * p.H;
-    hipLaunchKernelGGL((wkv7_rec_prep<128>), dim3(nchunk, BH), dim3(64), 0, p.stream, p.T, p.H,
+    hipLaunchKernelGGL((wkv7_rec_prep<NK>), dim3(nchunk, BH), dim3(64), 0, p.stream, p.T, p.H,
                        static_cast<const bf16_t*>(p.r), static_cast<const bf16_t*>(p.w), static_cast<const bf16_t*>(p.k),
                        static_cast<const bf16_t*>(p.v), static_cast<const bf16_t*>(p.a), static_cast<const bf16_t*>(p.b),
                        static_cast<uint8_t*>(p.ws));
-    scan_records<128, bf16_t, true>(p.B, p.T, p.H, 0, p.s0, static_cast<bf16_t*>(p.y), p.sT, p.ckpt, p.ws, p.ws_bytes,
-                                    cus, p.stream);
+    scan_records<NK, bf16_t, true>(p.B, p.T, p.H, 0, p.s0, static_cast<bf16_t*>(p.y), p.sT, p.ckpt, p.ws, p.ws_bytes,
+                                   cus, p.stream);
 }
+void launch_wkv7_rec_forward(const Fwd& p, int cus) {
+    if (p.N == 64) launch_rec_fwd<64>(p, cus);
+    else launch_rec_fwd<128>(p, cus);
+}
+template <bool PK> static size_t train_workspace(int B, int T, int H, int N, int cus) {
+    const size_t BH = (size_t)B * H;
+    return (records<PK>(B, T, H, N) + 255) / 256 * 256 +
+           resume_bytes(BH, N, resume_segments(BH, N, (T + GC - 1) / GC, cus));
+}
+size_t wkv7_rec_train_workspace(int B, int T, int H, int N, int cus) { return train_workspace<true>(B, T, H, N, cus); }
+size_t gdn_train_workspace(int B, int T, int H, int N, int cus) { return train_workspace<false>(B, T, H, N, cus); }
 
 }  // namespace wkv7

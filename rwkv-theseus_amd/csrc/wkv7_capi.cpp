@@ -6,7 +6,7 @@
 // tensors), picks the kernel family, launches on the caller's stream and
 // reports launch failures like C10_CUDA_KERNEL_LAUNCH_CHECK (cpp:24,36).
 #include "../../include/theseus_wkv7.h"
-#include "../../include/theseus_gdn.h"
+#include "../../include/theseus_gdn_ex.h"
 
 #include <hip/hip_runtime.h>
 
@@ -111,7 +111,7 @@ void launch_forward(const Fwd& p) {
 }
 void launch_backward(const Bwd& p) {
     if (chunk_ok(p.B, p.T, p.H, p.N, p.dtype, p.flags)) launch_chunk_backward(p, cu_count());
-    else if (rec_shape(p.B, p.T, p.H, p.N, p.dtype, p.flags)) launch_wkv7_rec_backward(p);
+    else if (rec_shape(p.B, p.T, p.H, p.N, p.dtype, p.flags)) launch_wkv7_rec_backward(p, cu_count());
     else launch_seq_backward(p);
 }
 // The chunked kernels' handoffs; the step-serial backward replays each
@@ -120,15 +120,21 @@ size_t forward_workspace(int B, int T, int H, int N, int dtype, int flags) {
     return chunk_ok(B, T, H, N, dtype, flags) ? chunk_forward_workspace(B, T, H, cu_count()) : 0;
 }
 size_t forward_workspace_fast(int B, int T, int H, int N, int dtype, int flags) {
-    if (rec_shape(B, T, H, N, dtype, flags)) return wkv7_rec_workspace_split(B, T, H, N, cu_count());
+    if (rec_shape(B, T, H, N, dtype, flags)) return wkv7_rec_workspace_fast(B, T, H, N, cu_count());
     const size_t need = forward_workspace(B, T, H, N, dtype, flags);
     if (!split_shape(B, T, H, N, dtype, flags)) return need;
     const size_t split = chunk_forward_split_workspace(B, T, H, cu_count());
     return split > need ? split : need;
 }
+size_t forward_workspace_best(int B, int T, int H, int N, int dtype, bool saved) {
+    const size_t need = forward_workspace_fast(B, T, H, N, dtype);
+    if (!saved || !rec_shape(B, T, H, N, dtype, 0)) return need;
+    const size_t best = wkv7_rec_train_workspace(B, T, H, N, cu_count());
+    return best > need ? best : need;
+}
 size_t backward_workspace(int B, int T, int H, int N, int dtype, int flags) {
     if (chunk_ok(B, T, H, N, dtype, flags)) return chunk_backward_workspace(B, T, H, cu_count());
-    if (rec_shape(B, T, H, N, dtype, flags)) return wkv7_rec_bwd_workspace(B, T, H);
+    if (rec_shape(B, T, H, N, dtype, flags)) return wkv7_rec_bwd_workspace(B, T, H, N, cu_count());
     return seq_backward_workspace(B, T, H, N);
 }
 
@@ -183,6 +189,11 @@ long long theseus_wkv7_checkpoint_count(int T) {
 size_t theseus_wkv7_forward_workspace_size(int B, int T, int H, int N, int dtype) {
     if (check_dims(B, T, H, N, dtype) != THESEUS_WKV7_OK) return 0;
     return wkv7::forward_workspace_fast(B, T, H, N, dtype);
+}
+
+size_t theseus_wkv7_forward_best_workspace_size(int B, int T, int H, int N, int dtype, int saved_states) {
+    if (check_dims(B, T, H, N, dtype) != THESEUS_WKV7_OK) return 0;
+    return wkv7::forward_workspace_best(B, T, H, N, dtype, saved_states != 0);
 }
 
 size_t theseus_wkv7_backward_workspace_size(int B, int T, int H, int N, int dtype) {
@@ -269,6 +280,15 @@ size_t theseus_gdn_forward_workspace_size(int B, int T, int H, int N) {
     return gdn_dims(B, T, H, N) ? 0 : wkv7::gdn_forward_workspace_split(B, T, H, N, wkv7::cu_count());
 }
 
+size_t theseus_gdn_forward_best_workspace_size(int B, int T, int H, int N, int saved_states) {
+    if (gdn_dims(B, T, H, N)) return 0;
+    const int cus = wkv7::cu_count();
+    const size_t need = wkv7::gdn_forward_workspace_split(B, T, H, N, cus);
+    const size_t best = saved_states ? wkv7::gdn_train_workspace(B, T, H, N, cus)
+                                     : wkv7::gdn_forward_workspace_fast(B, T, H, N, cus);
+    return best > need ? best : need;
+}
+
 int theseus_gdn_forward(int B, int T, int H, int N, int dtype, int qk_l2norm, const void* q, const void* k,
                         const void* v, const float* g, const float* beta, const float* s0, void* o, float* sT,
                         void* workspace, size_t workspace_bytes, hipStream_t stream) {
@@ -292,13 +312,14 @@ int theseus_gdn_forward_train(int B, int T, int H, int N, int dtype, const void*
     if (!workspace || workspace_bytes < wkv7::gdn_forward_workspace(B, T, H, N)) return THESEUS_WKV7_ERR_WORKSPACE;
     wkv7::Gdn p{B, T, H, N, dtype, 0, q, k, v, g, beta, s0, o, sT, workspace, 1, stream};
     p.ws_bytes = workspace_bytes;
+    p.cus = wkv7::cu_count();
     p.ckpt = ckpt;
     wkv7::launch_gdn_forward(p);
     return launch_status();
 }
 
 size_t theseus_gdn_backward_workspace_size(int B, int T, int H, int N) {
-    return gdn_dims(B, T, H, N) || N != 128 ? 0 : wkv7::gdn_backward_workspace(B, T, H);
+    return gdn_dims(B, T, H, N) || N != 128 ? 0 : wkv7::gdn_backward_workspace(B, T, H, wkv7::cu_count());
 }
 
 int theseus_gdn_backward(int B, int T, int H, int N, int dtype, const void* q, const void* k, const void* v,
@@ -310,8 +331,9 @@ int theseus_gdn_backward(int B, int T, int H, int N, int dtype, const void* q, c
     if (dtype != THESEUS_WKV7_BF16 && dtype != THESEUS_WKV7_FP32) return THESEUS_WKV7_ERR_DTYPE;
     if (!q || !k || !v || !g || !beta || !ckpt || !dout || !dq || !dk || !dv || !dg || !dbeta || !ds0)
         return THESEUS_WKV7_ERR_NULL;
-    if (!workspace || workspace_bytes < wkv7::gdn_backward_workspace(B, T, H)) return THESEUS_WKV7_ERR_WORKSPACE;
+    if (!workspace || workspace_bytes < wkv7::gdn_backward_workspace(B, T, H, wkv7::cu_count())) return THESEUS_WKV7_ERR_WORKSPACE;
     wkv7::GdnBwd p{B, T, H, N, dtype, q, k, v, g, beta, ckpt, dout, dsT, dq, dk, dv, dg, dbeta, ds0, workspace, stream};
+    p.cus = wkv7::cu_count();
     wkv7::launch_gdn_backward(p);
     return launch_status();
 }

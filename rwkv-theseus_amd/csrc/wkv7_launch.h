@@ -104,26 +104,32 @@ struct GdnBwd {
     float *dg, *dbeta, *ds0;
     void* ws;
     hipStream_t stream;
+    int cus = 0;  // CUs the reverse scan's time split may fill
 };
-size_t gdn_backward_workspace(int B, int T, int H);
+size_t gdn_backward_workspace(int B, int T, int H, int cus);
 void launch_gdn_backward(const GdnBwd& p);
 // the operand records (the least a call needs); with the time split's buffers when it
 // applies (gdn_split_segments >= 2)
 size_t gdn_forward_workspace(int B, int T, int H, int N);
 size_t gdn_forward_workspace_split(int B, int T, int H, int N, int cus);
+// with the buffers of as many segments as help, without and with saved states
+size_t gdn_forward_workspace_fast(int B, int T, int H, int N, int cus);
+size_t gdn_train_workspace(int B, int T, int H, int N, int cus);
 int gdn_split_segments(int B, int T, int H, int N, int cus);
 void launch_gdn_forward(const Gdn& p);
-// The WKV7 forward for bf16, N = 128 and flags 0 on the same two kernels (per-key
-// decays in the records): wkv7_rec_workspace bytes of records, or
-// wkv7_rec_workspace_split with the time split's buffers (few heads, no saved states).
+// The WKV7 forward for bf16, N = 128 (and 64, few heads in training) and flags 0 on the
+// same two kernels (per-key decays in the records): wkv7_rec_workspace bytes of records,
+// wkv7_rec_workspace_fast with the time split's buffers (few heads, no saved states), or
+// wkv7_rec_train_workspace with those of the split that saves states.
 size_t wkv7_rec_workspace(int B, int T, int H, int N);
-size_t wkv7_rec_workspace_split(int B, int T, int H, int N, int cus);
+size_t wkv7_rec_workspace_fast(int B, int T, int H, int N, int cus);
+size_t wkv7_rec_train_workspace(int B, int T, int H, int N, int cus);
 void launch_wkv7_rec_forward(const Fwd& p, int cus);
-// Its backward (wkv7_rec_bwd.hip), every chunk at once from the [value][key] saved
-// states: a workspace of wkv7_rec_bwd_workspace bytes (the scan's records and dL/dS at
-// every chunk's end).
-size_t wkv7_rec_bwd_workspace(int B, int T, int H);
-void launch_wkv7_rec_backward(const Bwd& p);
+// Its backward (wkv7_rec_bwd.hip), every chunk at once from the saved states: a workspace
+// of wkv7_rec_bwd_workspace bytes (the scan's records, dL/dS at every chunk's end, the
+// reverse scan's time split).
+size_t wkv7_rec_bwd_workspace(int B, int T, int H, int N, int cus);
+void launch_wkv7_rec_backward(const Bwd& p, int cus);
 
 // Family dispatch (wkv7_capi.cpp): the chunked MFMA kernels when they cover
 // the call, else the step-serial ones.
@@ -132,6 +138,8 @@ void launch_backward(const Bwd& p);
 size_t forward_workspace(int B, int T, int H, int N, int dtype, int flags = 0);
 // forward_workspace, or more where the time-split forward could take the call
 size_t forward_workspace_fast(int B, int T, int H, int N, int dtype, int flags = 0);
+// forward_workspace, or more where a forward (with saved states or without) runs faster given more
+size_t forward_workspace_best(int B, int T, int H, int N, int dtype, bool saved);
 size_t backward_workspace(int B, int T, int H, int N, int dtype, int flags = 0);
 
 }  // namespace wkv7

@@ -26,26 +26,27 @@
 // workspace and the first chunk's start as ds0.  wkv7_bwd_chunk then forms every
 // chunk's gradients independently (eight waves; wave w owns value rows 16w..16w+15 for
 // SA, Q, dV and keys 16w..16w+15 for dK, dB, dR, dA, dw).
-#include "wkv7_io.h"
 #include "wkv7_launch.h"
+#include "wkv7_scan.h"
 
 namespace wkv7 {
 namespace {
 
 constexpr int BC = 16;        // chunk length
-constexpr int BNK = 128;      // head size
+constexpr int BNK = 128;      // the gated delta rule's head size here
 constexpr int BKS = BNK / 32, BTJ = BNK / 16;
 constexpr long BNN = (long)BNK * BNK;
 
 // One chunk's record for the scan (byte offsets).
-struct BwdRec {
-    static constexpr size_t BF = 0;                                // B^ [KS][hi, lo][64 lanes] uint4
-    static constexpr size_t PP = BF + (size_t)BKS * 2 * 64 * 16;   // [P | P2] [TJ][hi, lo][64] uint4
-    static constexpr size_t EL = PP + (size_t)BTJ * 2 * 64 * 16;   // e^{gL} [NK]
-    static constexpr size_t BYTES = EL + (size_t)BNK * 4;
+template <int NK> struct BwdRec {
+    static constexpr int KS = NK / 32, TJ = NK / 16;
+    static constexpr size_t BF = 0;                               // B^ [KS][hi, lo][64 lanes] uint4
+    static constexpr size_t PP = BF + (size_t)KS * 2 * 64 * 16;   // [P | P2] [TJ][hi, lo][64] uint4
+    static constexpr size_t EL = PP + (size_t)TJ * 2 * 64 * 16;   // e^{gL} [NK]
+    static constexpr size_t BYTES = EL + (size_t)NK * 4;
     static constexpr int DMA_BLOCKS = (int)((BYTES + 1023) / 1024);
 };
-static_assert(BwdRec::BYTES % 256 == 0, "record alignment");
+static_assert(BwdRec<128>::BYTES % 256 == 0 && BwdRec<64>::BYTES % 256 == 0, "record alignment");
 
 __device__ __forceinline__ f32x4_t mm3(f32x4_t acc, uint4 xh, uint4 xl, uint4 yh, uint4 yl) {
     return mma32(mma32(mma32(acc, xh, yh), xh, yl), xl, yh);
@@ -64,18 +65,19 @@ __device__ __forceinline__ float bf2f(const bf16_t* p, long i) { return io<bf16_
 // Records of chunk blockIdx.x of head blockIdx.y (one wave; lane (q4, r16): token r16's
 // keys 32ks + 4q4 + e and 32ks + 16 + 4q4 + e, as wkv7_rec_prep).
 // ---------------------------------------------------------------------------
+template <int NK>
 __global__ __launch_bounds__(64) void wkv7_bwd_prep(int Tn, int H, const bf16_t* __restrict__ r,
                                                     const bf16_t* __restrict__ w, const bf16_t* __restrict__ k,
                                                     const bf16_t* __restrict__ a, const bf16_t* __restrict__ b,
                                                     uint8_t* __restrict__ ws) {
-    using R = BwdRec;
-    constexpr int LP = BNK + 4;
+    using R = BwdRec<NK>;
+    constexpr int KS = R::KS, TJ = R::TJ, LP = NK + 4;
     const int c = blockIdx.x, bh = blockIdx.y, nchunk = gridDim.x;
     const int bb = bh / H, h = bh - bb * H;
     const int lane = threadIdx.x, q4 = lane >> 4, r16 = lane & 15;
     const int t0 = c * BC, L = min(BC, Tn - t0);
     const bool tv = r16 < L;
-    const long row = (((long)bb * Tn + t0 + (tv ? r16 : 0)) * H + h) * (long)BNK;  // (clamped: read by every lane)
+    const long row = (((long)bb * Tn + t0 + (tv ? r16 : 0)) * H + h) * (long)NK;  // (clamped: read by every lane)
     const uint32_t tm = lane_mask(tv);
     __shared__ __attribute__((aligned(16))) float pa[BC][LP], pr[BC][LP];  // A~, R~ [t][j]
     uint8_t* const rec = ws + ((size_t)bh * nchunk + c) * R::BYTES;
@@ -89,7 +91,7 @@ __global__ __launch_bounds__(64) void wkv7_bwd_prep(int Tn, int H, const bf16_t*
     };
     f32x4_t Aab = zero4(), AabT = zero4(), BrbT = zero4();
 #pragma unroll
-    for (int ks = 0; ks < BKS; ks++) {
+    for (int ks = 0; ks < KS; ks++) {
         const int c0 = 32 * ks + 4 * q4;
         float wv[8], av[8], bv[8], rv[8];
         ld8(w, c0, wv), ld8(a, c0, av), ld8(b, c0, bv), ld8(r, c0, rv);
@@ -112,9 +114,9 @@ __global__ __launch_bounds__(64) void wkv7_bwd_prep(int Tn, int H, const bf16_t*
         }
         uint4 ah, al, bh_, bl, rh, rl, hh, hl;
         pack8(At, ah, al), pack8(Bm, bh_, bl), pack8(Rt, rh, rl), pack8(Bh, hh, hl);
-        uint4* bf = reinterpret_cast<uint4*>(rec + R::BF) + (size_t)(2 * ks) * 64 + lane;
-        bf[0] = hh;
-        bf[64] = hl;
+        uint8_t* bf = rec + R::BF + (size_t)(2 * ks) * 1024;
+        put_frag(bf, lane, hh);
+        put_frag(bf + 1024, lane, hl);
         Aab = mm3(Aab, ah, al, bh_, bl);    // A~_rr . B-_cc
         AabT = mm3(AabT, bh_, bl, ah, al);  // B-_rr . A~_cc
         BrbT = mm3(BrbT, bh_, bl, rh, rl);  // B-_rr . R~_cc
@@ -132,16 +134,16 @@ __global__ __launch_bounds__(64) void wkv7_bwd_prep(int Tn, int H, const bf16_t*
     const Pk pTiT = pk(TiT), pBrbT = pk(BrbT);
     __syncthreads();  // the planes
 #pragma unroll
-    for (int tj = 0; tj < BTJ; tj++) {
+    for (int tj = 0; tj < TJ; tj++) {
         f32x4_t at, rt;  // D layout [t][j], t = 4q4 + e, j = 16tj + r16
 #pragma unroll
         for (int e = 0; e < 4; e++) at[e] = pa[4 * q4 + e][16 * tj + r16], rt[e] = pr[4 * q4 + e][16 * tj + r16];
         const f32x4_t Pt = mm16s(pTiT, pk(at));          // P = Ti A~
         const Pk pP = pk(Pt);
         const Pk pP2 = pk(rt + mm16s(pBrbT, pP));        // P2 = R~ + Brb P
-        uint4* pp = reinterpret_cast<uint4*>(rec + R::PP) + (size_t)(2 * tj) * 64 + lane;
-        pp[0] = cat(pP.h, pP2.h);
-        pp[64] = cat(pP.l, pP2.l);
+        uint8_t* pp = rec + R::PP + (size_t)(2 * tj) * 1024;
+        put_frag(pp, lane, cat(pP.h, pP2.h));
+        put_frag(pp + 1024, lane, cat(pP.l, pP2.l));
     }
 }
 
@@ -153,23 +155,33 @@ __global__ __launch_bounds__(64) void wkv7_bwd_prep(int Tn, int H, const bf16_t*
 // dsT (may be null) and ds0 [key][value] when kv (GDN's layout), else [value][key]; H in
 // the workspace always [value][key].
 // ---------------------------------------------------------------------------
-template <typename TI>
-__global__ __launch_bounds__(256) void wkv7_bwd_scan(int Tn, int H, int BH, int kv, const float* __restrict__ dsT,
+template <int NK, typename TI, ScanMode MODE>
+__global__ __launch_bounds__(4 * NK) void wkv7_bwd_scan(int Tn, int H, int BH, int kv, const float* __restrict__ dsT,
                                                      const TI* __restrict__ dy, float* __restrict__ ds0,
-                                                     float* __restrict__ hbuf, const uint8_t* __restrict__ ws) {
-    using R = BwdRec;
+                                                     float* __restrict__ hbuf, const uint8_t* __restrict__ ws,
+                                                     ScanSplit sp) {
+    using R = BwdRec<NK>;
+    constexpr int KS = R::KS, TJ = R::TJ;
+    constexpr long NN = (long)NK * NK;
     __shared__ __attribute__((aligned(1024))) uint8_t recs[2][R::DMA_BLOCKS * 1024];
-    const int bh = blockIdx.x % BH, rg = blockIdx.x / BH, bb = bh / H, h = bh - bb * H;
+    // workgroup (segment * row groups + rg) * BH + bh, NW waves each
+    const int NW = max(1, __builtin_amdgcn_readfirstlane((int)(blockDim.x >> 6))), RGS = NK / 16 / NW;
+    const int bh = blockIdx.x % BH, rest = blockIdx.x / BH, rg = rest % RGS, bb = bh / H, h = bh - bb * H;
+    const int sgm = MODE == SCAN_ENDS ? rest / RGS : MODE == SCAN_RESUME ? 1 + rest / RGS : 0;
+    const bool dual = MODE == SCAN_ENDS && sgm > 0;  // from zero and from the identity, no H stored
     const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, q4 = lane >> 4, r16 = lane & 15;
-    const int i_own = 16 * (4 * rg + wv) + r16;
+    const int i_own = 16 * (NW * rg + wv) + r16;
     const int nchunk = (Tn + BC - 1) / BC;
+    // this segment's chunks, chi - 1 down to clo (segment 0: the last m0 chunks)
+    const int chi = MODE == SCAN_ALL || sgm == 0 ? nchunk : nchunk - sp.m0 - (sgm - 1) * sp.m;
+    const int clo = MODE == SCAN_ALL ? 0 : max(0, sgm == 0 ? nchunk - sp.m0 : chi - sp.m);
     const i32x4_t rs = dma_rsrc(ws + (size_t)bh * nchunk * R::BYTES, (uint32_t)((size_t)nchunk * R::BYTES));
     auto fetch = [&](int c, int buf) {
         uint32_t so = (uint32_t)((size_t)c * R::BYTES);
         asm volatile("" : "+s"(so));
         const uint32_t base = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)recs[buf];
-        for (int j = wv; j < R::DMA_BLOCKS; j += 4) dma_kb(base + 1024 * j, rs, (uint32_t)(1024 * j + 16 * lane), so);
+        for (int j = wv; j < R::DMA_BLOCKS; j += NW) dma_kb(base + 1024 * j, rs, (uint32_t)(1024 * j + 16 * lane), so);
     };
     // dY[t0 + 4q4 + e][i_own], loaded a chunk ahead as raw element bits: rows past the end
     // read row t0, and the bits are widened and zeroed where they are used (dy_of), so
@@ -179,7 +191,7 @@ __global__ __launch_bounds__(256) void wkv7_bwd_scan(int Tn, int H, int BH, int 
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int t = 4 * q4 + e, tc = t < L ? t : 0;
-            const long i = (((long)bb * Tn + t0 + tc) * H + h) * BNK + i_own;
+            const long i = (((long)bb * Tn + t0 + tc) * H + h) * NK + i_own;
             if constexpr (sizeof(TI) == 2) o[e] = reinterpret_cast<const uint16_t*>(dy)[i];
             else o[e] = reinterpret_cast<const uint32_t*>(dy)[i];
         }
@@ -192,89 +204,119 @@ __global__ __launch_bounds__(256) void wkv7_bwd_scan(int Tn, int H, int BH, int 
             d[e] = keep(lane_mask(4 * q4 + e < L), __uint_as_float(sizeof(TI) == 2 ? o[e] << 16 : o[e]));
         return d;
     };
-    fetch(nchunk - 1, 0);
-    f32x4_t Ht[BTJ];
+    fetch(chi - 1, 0);
+    f32x4_t Ht[TJ], Hp[TJ];  // (Hp: the identity run)
+    const float* const start = MODE == SCAN_RESUME ? seg_state(sp, BH, bh, sgm, NN) : dsT;
 #pragma unroll
-    for (int tj = 0; tj < BTJ; tj++) {
-        if (!dsT) {
+    for (int tj = 0; tj < TJ; tj++) {
+        if (dual || (MODE != SCAN_RESUME && !dsT)) {
             Ht[tj] = zero4();
-        } else if (kv) {
+        } else if (MODE != SCAN_RESUME && kv) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) Ht[tj][e] = dsT[bh * BNN + (long)(16 * tj + 4 * q4 + e) * BNK + i_own];
+            for (int e = 0; e < 4; e++) Ht[tj][e] = dsT[bh * NN + (long)(16 * tj + 4 * q4 + e) * NK + i_own];
         } else {
-            const float4 x = *reinterpret_cast<const float4*>(dsT + bh * BNN + (long)i_own * BNK + 16 * tj + 4 * q4);
+            const float4 x = *reinterpret_cast<const float4*>(start + (MODE == SCAN_RESUME ? 0 : bh * NN) +
+                                                              (long)i_own * NK + 16 * tj + 4 * q4);
             Ht[tj] = f32x4_t{x.x, x.y, x.z, x.w};
         }
+        if (MODE == SCAN_ENDS)
+#pragma unroll
+            for (int e = 0; e < 4; e++) Hp[tj][e] = i_own == 16 * tj + 4 * q4 + e ? 1.f : 0.f;
     }
     uint32_t dyn[4];
-    load_dy(nchunk - 1, dyn);
+    load_dy(chi - 1, dyn);
     vm_wait0();
-    f32x4_t dyc = dy_of(nchunk - 1, dyn);  // this chunk's dY (the next chunk's is formed after each chunk's wait)
+    f32x4_t dyc = dy_of(chi - 1, dyn);  // this chunk's dY (the next chunk's is formed after each chunk's wait)
     __syncthreads();
-    for (int c = nchunk - 1, it = 0; c >= 0; c--, it++) {
-        if (c > 0) fetch(c - 1, (it + 1) & 1);
-        const uint8_t* const rec = recs[it & 1];
-        if (c > 0) load_dy(c - 1, dyn);
-        // H at the chunk's end, stored after the next record's DMA and left in flight by the
-        // closing wait (vmcnt(BTJ): a vmcnt(0) there had waited for these stores every chunk)
-        float* const hout = hbuf + ((long)bh * nchunk + c) * BNN + (long)i_own * BNK + 4 * q4;
-#pragma unroll
-        for (int tj = 0; tj < BTJ; tj++)
-            *reinterpret_cast<float4*>(hout + 16 * tj) = make_float4(Ht[tj][0], Ht[tj][1], Ht[tj][2], Ht[tj][3]);
-        // U^T [t][i_own] = sum_j B^[t][j] H[i_own][j]
+    // U^T [t][i_own] = sum_j B^[t][j] H[i_own][j]
+    auto btimes = [&](const uint8_t* rec, const f32x4_t (&X)[TJ]) {
         f32x4_t u = zero4();
 #pragma unroll
-        for (int ks = 0; ks < BKS; ks++) {
-            const float sv[8] = {Ht[2 * ks][0], Ht[2 * ks][1], Ht[2 * ks][2], Ht[2 * ks][3],
-                                 Ht[2 * ks + 1][0], Ht[2 * ks + 1][1], Ht[2 * ks + 1][2], Ht[2 * ks + 1][3]};
+        for (int ks = 0; ks < KS; ks++) {
+            const float sv[8] = {X[2 * ks][0], X[2 * ks][1], X[2 * ks][2], X[2 * ks][3],
+                                 X[2 * ks + 1][0], X[2 * ks + 1][1], X[2 * ks + 1][2], X[2 * ks + 1][3]};
             uint4 sh, sl;
             pack8(sv, sh, sl);
-            const uint4* bf = reinterpret_cast<const uint4*>(rec + R::BF) + (2 * ks) * 64 + lane;
-            u = mm3(u, bf[0], bf[64], sh, sl);
+            const uint8_t* bf = rec + R::BF + (2 * ks) * 1024;
+            u = mm3(u, get_frag(bf, lane), get_frag(bf + 1024, lane), sh, sl);
         }
-        uint2 uh, ul, dh, dl;
+        return u;
+    };
+    for (int c = chi - 1, it = 0; c >= clo; c--, it++) {
+        if (c > clo) fetch(c - 1, (it + 1) & 1);
+        const uint8_t* const rec = recs[it & 1];
+        if (c > clo) load_dy(c - 1, dyn);
+        // H at the chunk's end, stored after the next record's DMA and left in flight by the
+        // closing wait (vmcnt(TJ): a vmcnt(0) there had waited for these stores every chunk)
+        if (!dual) {
+            float* const hout = hbuf + ((long)bh * nchunk + c) * NN + (long)i_own * NK + 4 * q4;
+#pragma unroll
+            for (int tj = 0; tj < TJ; tj++)
+                *reinterpret_cast<float4*>(hout + 16 * tj) = make_float4(Ht[tj][0], Ht[tj][1], Ht[tj][2], Ht[tj][3]);
+        }
+        const f32x4_t u = btimes(rec, Ht);
+        uint2 uh, ul, dh, dl, ph = {}, pl = {};
         pack4(u, uh, ul);
         pack4(dyc, dh, dl);  // (bf16 dY: dl = 0)
+        if (dual) pack4(btimes(rec, Hp), ph, pl);
         const uint4 bhi = cat(uh, dh), blo = cat(ul, dl);
+        const uint4 phi = cat(ph, make_uint2(0, 0)), plo = cat(pl, make_uint2(0, 0));  // (the identity run has no dY)
 #pragma unroll
-        for (int tj = 0; tj < BTJ; tj++) {
-            const uint4* pp = reinterpret_cast<const uint4*>(rec + R::PP) + (2 * tj) * 64 + lane;
-            const uint4 ah = pp[0], al = pp[64];
+        for (int tj = 0; tj < TJ; tj++) {
+            const uint8_t* pp = rec + R::PP + (2 * tj) * 1024;
+            const uint4 ah = get_frag(pp, lane), al = get_frag(pp + 1024, lane);
             const f32x4_t eg = *reinterpret_cast<const f32x4_t*>(rec + R::EL + 4 * (16 * tj + 4 * q4));
             Ht[tj] = mma32(mma32(mma32(Ht[tj] * eg, ah, bhi), ah, blo), al, bhi);
+            if (dual) Hp[tj] = mma32(mma32(mma32(Hp[tj] * eg, ah, phi), ah, plo), al, phi);
         }
-        vm_wait_n<BTJ>();  // the next record and the dY loads after it have landed (only the stores may not)
+        // the next record and the dY loads after it have landed (only the stores may not)
+        if (dual) vm_wait0();
+        else vm_wait_n<TJ>();
         // the next chunk's dY, formed here where its loads are known complete (formed at the
         // top of the loop, the compiler's own wait there, merged with the path into the loop,
         // would have waited for these stores too)
-        if (c > 0) dyc = dy_of(c - 1, dyn);
+        if (c > clo) dyc = dy_of(c - 1, dyn);
         __syncthreads();
     }
+    if (MODE == SCAN_ENDS) {  // X_1, or U_s and Phi_s
+        const long o4 = ((dual ? (long)(sgm - 1) * BH : 0) + bh) * NN + (long)i_own * NK + 4 * q4;
+        float* const dst = dual ? sp.uend : sp.send0;
 #pragma unroll
-    for (int tj = 0; tj < BTJ; tj++) {
+        for (int tj = 0; tj < TJ; tj++) {
+            *reinterpret_cast<float4*>(dst + o4 + 16 * tj) = make_float4(Ht[tj][0], Ht[tj][1], Ht[tj][2], Ht[tj][3]);
+            if (dual)  // (transposed, as scan_chain reads it)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    sp.phi[((long)(sgm - 1) * BH + bh) * NN + (long)(16 * tj + 4 * q4 + e) * NK + i_own] = Hp[tj][e];
+        }
+        return;
+    }
+    if (clo > 0) return;  // (only the segment of the first chunk ends the head)
+#pragma unroll
+    for (int tj = 0; tj < TJ; tj++) {
         if (kv) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) ds0[bh * BNN + (long)(16 * tj + 4 * q4 + e) * BNK + i_own] = Ht[tj][e];
+            for (int e = 0; e < 4; e++) ds0[bh * NN + (long)(16 * tj + 4 * q4 + e) * NK + i_own] = Ht[tj][e];
         } else {
-            *reinterpret_cast<float4*>(ds0 + bh * BNN + (long)i_own * BNK + 16 * tj + 4 * q4) =
+            *reinterpret_cast<float4*>(ds0 + bh * NN + (long)i_own * NK + 16 * tj + 4 * q4) =
                 make_float4(Ht[tj][0], Ht[tj][1], Ht[tj][2], Ht[tj][3]);
         }
     }
 }
 
 // ---------------------------------------------------------------------------
-// The gradients of one chunk (512 lanes).  Workgroups map to (head, chunk) so that a
+// The gradients of one chunk (4 NK lanes).  Workgroups map to (head, chunk) so that a
 // head's consecutive chunks share an XCD (chunk c's S_end is chunk c + 1's S0 in L2).
 // ---------------------------------------------------------------------------
 // The operands every wave reads as K=32 A/B fragments over the keys or value rows are
 // split into bf16 hi/lo once, by the wave that owns their 16 columns, and kept so in LDS
 // (splitting them in every reader had been most of the kernel's VALU work).
-constexpr int CLB = BNK + 8;  // padded split-plane row (bf16)
-struct SplitPlane {
+template <int NK> struct SplitPlane {
+    static constexpr int CLB = NK + 8;  // padded row (bf16)
     uint16_t h[BC][CLB], l[BC][CLB];
 };
 // a D-layout tile ([t][16 wv + c], rows t = 4q4 + e) into a split plane, 8-byte rows per lane
-__device__ __forceinline__ void put_split(SplitPlane& P, const f32x4_t& d, int lane, int wv) {
+template <int NK> __device__ __forceinline__ void put_split(SplitPlane<NK>& P, const f32x4_t& d, int lane, int wv) {
     uint2 h, l;
     quad_rows_split(d, lane, h, l);  // (cross-lane: every lane takes part)
     const int tr = 4 * (lane >> 4) + (lane & 3), c = 16 * wv + 4 * ((lane >> 2) & 3);
@@ -282,7 +324,8 @@ __device__ __forceinline__ void put_split(SplitPlane& P, const f32x4_t& d, int l
     *reinterpret_cast<uint2*>(&P.l[tr][c]) = l;
 }
 // the K=32 fragment of row r16, columns 32ks + 4q4 .. +3 and 32ks + 16 + 4q4 .. +3
-__device__ __forceinline__ void get_split(const SplitPlane& P, int lane, int ks, uint4& h, uint4& l) {
+template <int NK>
+__device__ __forceinline__ void get_split(const SplitPlane<NK>& P, int lane, int ks, uint4& h, uint4& l) {
     const int r = lane & 15, c = 32 * ks + 4 * (lane >> 4);
     const uint2 a = *reinterpret_cast<const uint2*>(&P.h[r][c]), b = *reinterpret_cast<const uint2*>(&P.h[r][c + 16]);
     const uint2 x = *reinterpret_cast<const uint2*>(&P.l[r][c]), y = *reinterpret_cast<const uint2*>(&P.l[r][c + 16]);
@@ -296,13 +339,17 @@ __device__ __forceinline__ uint4 bf16_frag(const bf16_t* row, int ks, int q4, bo
     const uint2 b = *reinterpret_cast<const uint2*>(row + 32 * ks + 16 + 4 * q4);
     return keepu4(lane_mask(ok), make_uint4(a.x, a.y, b.x, b.y));
 }
-struct ChunkLds {
-    SplitPlane At, Bm, Km, Rt, Bh, Kh;  // [t][j], written by the key owners
-    SplitPlane SA, Q;                   // [t][i], written by the value-row owners
-    float csum[BTJ][BNK];  // per wave: column sums of H_end o S_end over its 16 value rows
+template <int NK> struct ChunkLds {
+    SplitPlane<NK> At, Bm, Km, Rt, Bh, Kh;  // [t][j], written by the key owners
+    SplitPlane<NK> SA, Q;                   // [t][i], written by the value-row owners
+    float csum[NK / 16][NK];  // per wave: column sums of H_end o S_end over its 16 value rows
 };
 
-__global__ __launch_bounds__(512) void wkv7_bwd_chunk(int Tn, int H, int BH, int per_xcd,
+//
+// Saved states: [value][key] at NK = 128; at NK = 64 in the chunked kernels' tiled order
+// (but for the last, final one).
+template <int NK>
+__global__ __launch_bounds__(4 * NK) void wkv7_bwd_chunk(int Tn, int H, int BH, int per_xcd,
                                                       const bf16_t* __restrict__ r, const bf16_t* __restrict__ w,
                                                       const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
                                                       const bf16_t* __restrict__ a, const bf16_t* __restrict__ b,
@@ -311,7 +358,10 @@ __global__ __launch_bounds__(512) void wkv7_bwd_chunk(int Tn, int H, int BH, int
                                                       bf16_t* __restrict__ dw, bf16_t* __restrict__ dk,
                                                       bf16_t* __restrict__ dv, bf16_t* __restrict__ da,
                                                       bf16_t* __restrict__ db) {
-    __shared__ __attribute__((aligned(16))) ChunkLds sm;
+    constexpr int KS = NK / 32, TJ = NK / 16;
+    constexpr long NN = (long)NK * NK;
+    constexpr bool TILED = NK == 64;
+    __shared__ __attribute__((aligned(16))) ChunkLds<NK> sm;
     const int nchunk = (Tn + BC - 1) / BC;
     const int job = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if (job >= nchunk * BH) return;  // (whole workgroup)
@@ -321,26 +371,28 @@ __global__ __launch_bounds__(512) void wkv7_bwd_chunk(int Tn, int H, int BH, int
     const int t0 = c * BC, L = min(BC, Tn - t0);
     const long tok0 = (long)bb * Tn + t0;
     const int col = 16 * wv + r16;  // the lane's key (dK ...) and value column (dV ...)
-    auto at_tok = [&](int t) { return ((tok0 + t) * H + h) * (long)BNK; };
+    auto at_tok = [&](int t) { return ((tok0 + t) * H + h) * (long)NK; };
     const long ncp = nchunk + 1;
-    const float* const S0 = ckpt + ((long)bh * ncp + c) * BNN;
-    const float* const Se = S0 + BNN;
-    const float* const Hm = hbuf + ((long)bh * nchunk + c) * BNN;
+    const float* const S0 = ckpt + ((long)bh * ncp + c) * NN;
+    const float* const Se = S0 + NN;
+    const float* const Hm = hbuf + ((long)bh * nchunk + c) * NN;
     const int irow = 16 * wv + r16;  // value row of the row-strip loads
 
     // ---- the wave's value rows of H_end, S_end and S0 (keys 32ks + 4q4 + e, +16) ----
-    float hr[BKS][8], sr[BKS][8];
-    auto rows = [&](const float* M, float (&o)[BKS][8]) {
+    float hr[KS][8], sr[KS][8];
+    auto rows = [&](const float* M, bool tiled, float (&o)[KS][8]) {
 #pragma unroll
-        for (int ks = 0; ks < BKS; ks++) {
-            const float4 x = *reinterpret_cast<const float4*>(M + (long)irow * BNK + 32 * ks + 4 * q4);
-            const float4 y = *reinterpret_cast<const float4*>(M + (long)irow * BNK + 32 * ks + 16 + 4 * q4);
+        for (int ks = 0; ks < KS; ks++) {
+            // (tiled: tile (wv, 2ks) keeps this lane's four keys at its own float4)
+            const long ox = TILED && tiled ? (wv * TJ + 2 * ks) * 256 + 4 * lane : (long)irow * NK + 32 * ks + 4 * q4;
+            const long oy = ox + (TILED && tiled ? 256 : 16);
+            const float4 x = *reinterpret_cast<const float4*>(M + ox), y = *reinterpret_cast<const float4*>(M + oy);
             o[ks][0] = x.x, o[ks][1] = x.y, o[ks][2] = x.z, o[ks][3] = x.w;
             o[ks][4] = y.x, o[ks][5] = y.y, o[ks][6] = y.z, o[ks][7] = y.w;
         }
     };
-    rows(Hm, hr);
-    rows(Se, sr);
+    rows(Hm, false, hr);
+    rows(Se, c + 1 < nchunk, sr);
 
     // ---- the chunk operands of the wave's keys in D layout ([t][col], t = 4q4 + e) ----
     float xr[4], xw[4], xk[4], xa[4], xb[4];
@@ -373,25 +425,25 @@ __global__ __launch_bounds__(512) void wkv7_bwd_chunk(int Tn, int H, int BH, int
     put_split(sm.Rt, Rt, lane, wv), put_split(sm.Bh, Bm * eLj, lane, wv), put_split(sm.Kh, Km * eLj, lane, wv);
     // the carry's partial column sums over this wave's value rows
 #pragma unroll
-    for (int ks = 0; ks < BKS; ks++)
+    for (int ks = 0; ks < KS; ks++)
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             const float s = row_sum16(hr[ks][e] * sr[ks][e]);
             if (r16 == 0) sm.csum[wv][32 * ks + (e < 4 ? 4 * q4 + e : 16 + 4 * q4 + e - 4)] = s;
         }
-    uint4 Hh[BKS], Hl[BKS], Sh[BKS], Sl[BKS];
+    uint4 Hh[KS], Hl[KS], Sh[KS], Sl[KS];
 #pragma unroll
-    for (int ks = 0; ks < BKS; ks++) pack8(hr[ks], Hh[ks], Hl[ks]);
-    rows(S0, sr);
+    for (int ks = 0; ks < KS; ks++) pack8(hr[ks], Hh[ks], Hl[ks]);
+    rows(S0, true, sr);
 #pragma unroll
-    for (int ks = 0; ks < BKS; ks++) pack8(sr[ks], Sh[ks], Sl[ks]);
+    for (int ks = 0; ks < KS; ks++) pack8(sr[ks], Sh[ks], Sl[ks]);
     __syncthreads();
 
     // ---- chunk matrices (every wave) and the wave's [t][i] products over the keys ----
     f32x4_t Aab = zero4(), AabT = zero4(), Aak = zero4(), Brb = zero4(), Brk = zero4();
     f32x4_t P1 = zero4(), P2 = zero4(), P3 = zero4();
 #pragma unroll
-    for (int ks = 0; ks < BKS; ks++) {
+    for (int ks = 0; ks < KS; ks++) {
         uint4 ah, al, bh_, bl, kh, kl, rh, rl, hh, hl, xh, xl;
         get_split(sm.At, lane, ks, ah, al), get_split(sm.Bm, lane, ks, bh_, bl);
         get_split(sm.Km, lane, ks, kh, kl), get_split(sm.Rt, lane, ks, rh, rl);
@@ -443,15 +495,15 @@ __global__ __launch_bounds__(512) void wkv7_bwd_chunk(int Tn, int H, int BH, int
     // the key columns of H_end and S0 (value rows 32ks + 4q4 + e, +16) for the products over
     // the value rows
 #pragma unroll
-    for (int ks = 0; ks < BKS; ks++)
+    for (int ks = 0; ks < KS; ks++)
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             const int i = 32 * ks + (e < 4 ? 4 * q4 + e : 16 + 4 * q4 + e - 4);
-            hr[ks][e] = Hm[(long)i * BNK + col];
-            sr[ks][e] = S0[(long)i * BNK + col];
+            hr[ks][e] = Hm[(long)i * NK + col];
+            sr[ks][e] = S0[TILED ? ((i / 16 * TJ + wv) * 64 + 16 * (r16 / 4) + i % 16) * 4 + r16 % 4 : (long)i * NK + col];
         }
 #pragma unroll
-    for (int ks = 0; ks < BKS; ks++) pack8(hr[ks], Hh[ks], Hl[ks]), pack8(sr[ks], Sh[ks], Sl[ks]);
+    for (int ks = 0; ks < KS; ks++) pack8(hr[ks], Hh[ks], Hl[ks]), pack8(sr[ks], Sh[ks], Sl[ks]);
     __syncthreads();  // SA, Q, csum
 
     // ---- dK, dB, dR, dA, dw for the wave's keys ----
@@ -459,7 +511,7 @@ __global__ __launch_bounds__(512) void wkv7_bwd_chunk(int Tn, int H, int BH, int
     f32x4_t Gqv = zero4(), Gyv = zero4(), Gqs = zero4(), Gys = zero4();  // Gram matrices over the value rows
     const bool tv = r16 < L;
 #pragma unroll
-    for (int ks = 0; ks < BKS; ks++) {
+    for (int ks = 0; ks < KS; ks++) {
         uint4 sh, sl, qh, ql;
         get_split(sm.SA, lane, ks, sh, sl), get_split(sm.Q, lane, ks, qh, ql);
         const long o = at_tok(tv ? r16 : 0);
@@ -510,7 +562,7 @@ __global__ __launch_bounds__(512) void wkv7_bwd_chunk(int Tn, int H, int BH, int
         const float ya_ = (q4 < 1 ? Y1 : 0.f) + (q4 < 2 ? Y2 : 0.f) + (q4 < 3 ? Y3 : 0.f);
         float carry = 0.f;
 #pragma unroll
-        for (int u = 0; u < BTJ; u++) carry += sm.csum[u][col];
+        for (int u = 0; u < TJ; u++) carry += sm.csum[u][col];
 #pragma unroll
         for (int e = 0; e < 4; e++) sx[e] += xa_ + carry, sy[e] += ya_;
     }
@@ -558,7 +610,7 @@ template <typename TI>
 __global__ __launch_bounds__(64) void gdn_bwd_prep(int Tn, int H, const TI* __restrict__ q, const TI* __restrict__ k,
                                                    const float* __restrict__ g, const float* __restrict__ beta,
                                                    uint8_t* __restrict__ ws) {
-    using R = BwdRec;
+    using R = BwdRec<BNK>;
     const int c = blockIdx.x, bh = blockIdx.y, nchunk = gridDim.x;
     const int bb = bh / H, h = bh - bb * H;
     const int lane = threadIdx.x, q4 = lane >> 4, r16 = lane & 15;
@@ -589,9 +641,9 @@ __global__ __launch_bounds__(64) void gdn_bwd_prep(int Tn, int H, const TI* __re
         for (int e = 0; e < 8; e++) br8[e] = kr[e] * sb;
         uint4 kh, kl, qh, ql, bh_, bl;
         pack8(kr, kh, kl), pack8(qr, qh, ql), pack8(br8, bh_, bl);
-        uint4* bf = reinterpret_cast<uint4*>(rec + R::BF) + (size_t)(2 * ks) * 64 + lane;
-        bf[0] = bh_;
-        bf[64] = bl;
+        uint8_t* bf = rec + R::BF + (size_t)(2 * ks) * 1024;
+        put_frag(bf, lane, bh_);
+        put_frag(bf + 1024, lane, bl);
         KK = mm3(KK, kh, kl, kh, kl);  // k_rr . k_cc
         KR = mm3(KR, kh, kl, qh, ql);  // k_rr . q_cc
     }
@@ -628,9 +680,9 @@ __global__ __launch_bounds__(64) void gdn_bwd_prep(int Tn, int H, const TI* __re
         const f32x4_t Pt = mm16s(pTiT, pk(at));
         const Pk pP = pk(Pt);
         const Pk pP2 = pk(rt + mm16s(pBrbT, pP));
-        uint4* pp = reinterpret_cast<uint4*>(rec + R::PP) + (size_t)(2 * tj) * 64 + lane;
-        pp[0] = cat(pP.h, pP2.h);
-        pp[64] = cat(pP.l, pP2.l);
+        uint8_t* pp = rec + R::PP + (size_t)(2 * tj) * 1024;
+        put_frag(pp, lane, cat(pP.h, pP2.h));
+        put_frag(pp + 1024, lane, cat(pP.l, pP2.l));
     }
     if (lane < BNK / 4) {
         const float egL = __expf(gL);
@@ -639,8 +691,8 @@ __global__ __launch_bounds__(64) void gdn_bwd_prep(int Tn, int H, const TI* __re
 }
 
 struct GdnChunkLds {
-    SplitPlane K, R;   // k, r = q / sqrt(N) [t][j], written by the key owners
-    SplitPlane SA, Q;  // [t][i], written by the value-row owners
+    SplitPlane<BNK> K, R;   // k, r = q / sqrt(N) [t][j], written by the key owners
+    SplitPlane<BNK> SA, Q;  // [t][i], written by the value-row owners
     float gam[BC], gm1[BC], beta[BC];
     float csum[BTJ][BNK];
     float pv[BTJ][BC], pd[BTJ][BC], pk[BTJ][BC];  // per wave and token: sum v dV', sum dlogd, sum k dB
@@ -896,41 +948,70 @@ __global__ __launch_bounds__(512) void gdn_bwd_chunk(int Tn, int H, int BH, int 
 
 }  // namespace
 
-size_t wkv7_rec_bwd_workspace(int B, int T, int H) {
-    const size_t n = (size_t)B * H * ((T + BC - 1) / BC);
-    return (n * BwdRec::BYTES + 255) / 256 * 256 + n * BNN * sizeof(float);
+// Workspace: the scan's records, H = dL/dS at every chunk's end, the time split's buffers.
+template <int NK> static size_t bwd_records(size_t chunks) { return (chunks * BwdRec<NK>::BYTES + 255) / 256 * 256; }
+template <int NK> static size_t bwd_workspace(int B, int T, int H, int cus) {
+    const int n = (T + BC - 1) / BC;
+    const size_t BH = (size_t)B * H;
+    return bwd_records<NK>(BH * n) + BH * n * NK * NK * sizeof(float) +
+           resume_bytes(BH, NK, resume_segments(BH, NK, n, cus));
+}
+size_t wkv7_rec_bwd_workspace(int B, int T, int H, int N, int cus) {
+    return N == 64 ? bwd_workspace<64>(B, T, H, cus) : bwd_workspace<128>(B, T, H, cus);
+}
+// The reverse scan over the records at ws, in one pass or in time segments.
+template <int NK, typename TI>
+static const float* scan_back(int T, int H, int BH, int kv, const float* dsT, const void* dy, float* ds0, void* ws,
+                              int cus, hipStream_t stream) {
+    const int n = (T + BC - 1) / BC, k = resume_segments(BH, NK, n, cus);
+    const int rgs = k < 2 ? NK / 64 : scan_groups(BH, NK, k - 1, cus), lanes = 4 * NK / rgs;
+    const uint8_t* const recs = static_cast<const uint8_t*>(ws);
+    float* const hbuf = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + bwd_records<NK>((size_t)BH * n));
+    const TI* const y = static_cast<const TI*>(dy);
+    if (k < 2) {
+        hipLaunchKernelGGL((wkv7_bwd_scan<NK, TI, SCAN_ALL>), dim3(BH * rgs), dim3(lanes), 0, stream, T, H, BH, kv, dsT, y,
+                           ds0, hbuf, recs, ScanSplit{});
+        return hbuf;
+    }
+    const ScanSplit sp = resume_split(BH, NK, n, k, hbuf + (size_t)BH * n * NK * NK);
+    hipLaunchKernelGGL((wkv7_bwd_scan<NK, TI, SCAN_ENDS>), dim3((k - 1) * BH * rgs), dim3(lanes), 0, stream, T, H, BH, kv,
+                       dsT, y, ds0, hbuf, recs, sp);
+    hipLaunchKernelGGL((scan_chain<NK>), dim3(BH, NK / 16), dim3(4 * NK), 0, stream, BH, k - 2, kv, sp, nullptr);
+    hipLaunchKernelGGL((wkv7_bwd_scan<NK, TI, SCAN_RESUME>), dim3((k - 1) * BH * rgs), dim3(lanes), 0, stream, T, H, BH, kv,
+                       dsT, y, ds0, hbuf, recs, sp);
+    return hbuf;
 }
 
-void launch_wkv7_rec_backward(const Bwd& p) {
+template <int NK> static void launch_rec_bwd(const Bwd& p, int cus) {
     const int nchunk = (p.T + BC - 1) / BC, BH = p.B * p.H;
-    uint8_t* const recs = static_cast<uint8_t*>(p.ws);
-    float* const hbuf = reinterpret_cast<float*>(recs + ((size_t)BH * nchunk * BwdRec::BYTES + 255) / 256 * 256);
     const bf16_t *r = static_cast<const bf16_t*>(p.r), *w = static_cast<const bf16_t*>(p.w),
                  *k = static_cast<const bf16_t*>(p.k), *v = static_cast<const bf16_t*>(p.v),
                  *a = static_cast<const bf16_t*>(p.a), *b = static_cast<const bf16_t*>(p.b),
                  *dy = static_cast<const bf16_t*>(p.dy);
-    hipLaunchKernelGGL(wkv7_bwd_prep, dim3(nchunk, BH), dim3(64), 0, p.stream, p.T, p.H, r, w, k, a, b, recs);
-    hipLaunchKernelGGL(wkv7_bwd_scan<bf16_t>, dim3(BH * (BNK / 64)), dim3(256), 0, p.stream, p.T, p.H, BH, 0, p.dsT,
-                       dy, p.ds0, hbuf, recs);
+    hipLaunchKernelGGL(wkv7_bwd_prep<NK>, dim3(nchunk, BH), dim3(64), 0, p.stream, p.T, p.H, r, w, k, a, b,
+                       static_cast<uint8_t*>(p.ws));
+    const float* const hbuf = scan_back<NK, bf16_t>(p.T, p.H, BH, 0, p.dsT, dy, p.ds0, p.ws, cus, p.stream);
     const int jobs = nchunk * BH, per_xcd = (jobs + 7) / 8;
-    hipLaunchKernelGGL(wkv7_bwd_chunk, dim3(8 * per_xcd), dim3(512), 0, p.stream, p.T, p.H, BH, per_xcd, r, w, k, v,
-                       a, b, dy, p.ckpt, hbuf, static_cast<bf16_t*>(p.dr), static_cast<bf16_t*>(p.dw),
+    hipLaunchKernelGGL(wkv7_bwd_chunk<NK>, dim3(8 * per_xcd), dim3(4 * NK), 0, p.stream, p.T, p.H, BH, per_xcd, r, w, k,
+                       v, a, b, dy, p.ckpt, hbuf, static_cast<bf16_t*>(p.dr), static_cast<bf16_t*>(p.dw),
                        static_cast<bf16_t*>(p.dk), static_cast<bf16_t*>(p.dv), static_cast<bf16_t*>(p.da),
                        static_cast<bf16_t*>(p.db));
 }
+void launch_wkv7_rec_backward(const Bwd& p, int cus) {
+    if (p.N == 64) launch_rec_bwd<64>(p, cus);
+    else launch_rec_bwd<128>(p, cus);
+}
 
-size_t gdn_backward_workspace(int B, int T, int H) { return wkv7_rec_bwd_workspace(B, T, H); }
+size_t gdn_backward_workspace(int B, int T, int H, int cus) { return bwd_workspace<BNK>(B, T, H, cus); }
 
 template <typename TI>
 static void launch_gdn_bwd(const GdnBwd& p) {
     const int nchunk = (p.T + BC - 1) / BC, BH = p.B * p.H;
-    uint8_t* const recs = static_cast<uint8_t*>(p.ws);
-    float* const hbuf = reinterpret_cast<float*>(recs + ((size_t)BH * nchunk * BwdRec::BYTES + 255) / 256 * 256);
     const TI *q = static_cast<const TI*>(p.q), *k = static_cast<const TI*>(p.k), *v = static_cast<const TI*>(p.v),
              *dout = static_cast<const TI*>(p.dout);
-    hipLaunchKernelGGL(gdn_bwd_prep<TI>, dim3(nchunk, BH), dim3(64), 0, p.stream, p.T, p.H, q, k, p.g, p.beta, recs);
-    hipLaunchKernelGGL(wkv7_bwd_scan<TI>, dim3(BH * (BNK / 64)), dim3(256), 0, p.stream, p.T, p.H, BH, 1, p.dsT, dout,
-                       p.ds0, hbuf, recs);
+    hipLaunchKernelGGL(gdn_bwd_prep<TI>, dim3(nchunk, BH), dim3(64), 0, p.stream, p.T, p.H, q, k, p.g, p.beta,
+                       static_cast<uint8_t*>(p.ws));
+    const float* const hbuf = scan_back<BNK, TI>(p.T, p.H, BH, 1, p.dsT, dout, p.ds0, p.ws, p.cus, p.stream);
     const int jobs = nchunk * BH, per_xcd = (jobs + 7) / 8;
     hipLaunchKernelGGL(gdn_bwd_chunk<TI>, dim3(8 * per_xcd), dim3(512), 0, p.stream, p.T, p.H, BH, per_xcd, q, k, v,
                        p.g, p.beta, dout, p.ckpt, hbuf, static_cast<TI*>(p.dq), static_cast<TI*>(p.dk),

@@ -109,6 +109,8 @@ class Extension:
         for fn in (lib.theseus_wkv7_forward_workspace_size, lib.theseus_wkv7_backward_workspace_size):
             fn.argtypes = [i32] * 5
             fn.restype = sz
+        lib.theseus_wkv7_forward_best_workspace_size.argtypes = [i32] * 6
+        lib.theseus_wkv7_forward_best_workspace_size.restype = sz
         lib.theseus_wkv7_forward.argtypes = [i32] * 5 + [vp] * 10 + [vp, sz, vp]
         lib.theseus_wkv7_forward.restype = i32
         lib.theseus_wkv7_backward.argtypes = [i32] * 5 + [vp] * 16 + [vp, sz, vp]
@@ -135,6 +137,8 @@ class Extension:
         lib.theseus_gdn_forward.restype = i32
         lib.theseus_gdn_forward_workspace_size.argtypes = [i32] * 4
         lib.theseus_gdn_forward_workspace_size.restype = sz
+        lib.theseus_gdn_forward_best_workspace_size.argtypes = [i32] * 5
+        lib.theseus_gdn_forward_best_workspace_size.restype = sz
         lib.theseus_gdn_forward_train.argtypes = [i32] * 5 + [vp] * 9 + [vp, sz, vp]
         lib.theseus_gdn_forward_train.restype = i32
         lib.theseus_gdn_backward.argtypes = [i32] * 5 + [vp] * 14 + [vp, sz, vp]
@@ -243,8 +247,8 @@ class Extension:
             else:
                 if T > 1 or save_history:  # (a T=1 step without saved states runs the single-step kernel)
                     self._warn_fallback(B, T, H, N, dt)
-                ws, ws_bytes = _workspace(int(self.lib.theseus_wkv7_forward_workspace_size(B, T, H, N, dt)),
-                                          r.device)
+                ws, ws_bytes = _workspace(
+                    int(self.lib.theseus_wkv7_forward_best_workspace_size(B, T, H, N, dt, int(save_history))), r.device)
                 status = self.lib.theseus_wkv7_forward(
                     B, T, H, N, dt, *map(_ptr, (r, w, k, v, a, b, s0, y, end)), ck, _ptr(ws),
                     ctypes.c_size_t(ws_bytes), _stream(r.device))
@@ -276,7 +280,7 @@ class Extension:
         with _on(q.device):
             o = torch.empty_like(q)
             sT = torch.empty_like(s0)
-            ws, nbytes = _workspace(self.lib.theseus_gdn_forward_workspace_size(B, T, H, N), q.device)
+            ws, nbytes = _workspace(self.lib.theseus_gdn_forward_best_workspace_size(B, T, H, N, 0), q.device)
             p = lambda t: t.data_ptr()  # noqa: E731
             self._raise(self.lib.theseus_gdn_forward(
                 B, T, H, N, _BF16 if q.dtype == torch.bfloat16 else _FP32, 1 if qk_l2norm else 0, p(q), p(k), p(v), p(g), p(beta), p(s0),
@@ -309,7 +313,7 @@ class Extension:
             o = torch.empty_like(q)
             sT = torch.empty_like(s0)
             saved = torch.empty((B, H, self.checkpoint_count(T), N, N), dtype=torch.float32, device=q.device)
-            ws, nbytes = _workspace(self.lib.theseus_gdn_forward_workspace_size(B, T, H, N), q.device)
+            ws, nbytes = _workspace(self.lib.theseus_gdn_forward_best_workspace_size(B, T, H, N, 1), q.device)
             p = lambda t: t.data_ptr()  # noqa: E731
             self._raise(self.lib.theseus_gdn_forward_train(
                 B, T, H, N, _BF16 if q.dtype == torch.bfloat16 else _FP32, p(q), p(k), p(v), p(g), p(beta), p(s0),
