@@ -33,7 +33,7 @@ import functools
 
 import torch
 
-from .wkv7 import DECAY_EXP, STATE_KEY_VALUE, extension, wkv7_ex
+from .wkv7 import DECAY_EXP, STATE_KEY_VALUE, _native, extension, wkv7_ex
 
 # head sizes of the chunked forward (theseus_gdn_forward); others use the step-serial kernels
 CHUNKED_HEAD_SIZES = (64, 128)
@@ -98,7 +98,8 @@ def gated_delta_rule(query, key, value, g, beta, initial_state=None, output_fina
         # gradients wanted: the chunked forward with saved states and the chunked backward,
         # in float32 as transformers' functions compute
         q, k, v, gf, bf = (x.float().contiguous() for x in (query, key, value, g, beta))
-        o, sT = _GDN.apply(q, k, v, gf, bf, s0)
+        native = _native(q, k, v, gf, bf, s0)
+        o, sT = (_GDN.apply if native is None else native.gdn)(q, k, v, gf, bf, s0)
         return o.to(out_dtype), (sT if output_final_state else None)
     q, k, v, gf, bf = (x.float() for x in (query, key, value, g, beta))
     eg = torch.exp(gf)

@@ -419,6 +419,33 @@ def extension():
     return Extension(ctypes.CDLL(str(LIB_PATH)))
 
 
+@lru_cache(maxsize=1)
+def _native_module():
+    """theseus._native (csrc/torch_bind.cpp): the autograd functions of this module and of
+    theseus.gdn as native torch nodes, the same checks and the same C-ABI calls without the
+    interpreter in the backward.  None where it was not built (the library alone was copied
+    next to this file) or does not load in this torch: the Python functions below then run."""
+    extension()  # (raises where the library itself is missing)
+    if not (LIB_PATH.parent / "_native.so").exists():
+        return None
+    try:
+        from . import _native
+    except ImportError as e:
+        warnings.warn(f"theseus._native does not load ({e}); the Python autograd functions run instead "
+                      "(rebuild with `make -C rwkv-theseus_amd/csrc`)", RuntimeWarning, stacklevel=2)
+        return None
+    return _native
+
+
+def _native(*xs):
+    """The native functions when they cover a call: plain tensors, no functorch transform (the
+    Python functions say there what they do not support)."""
+    m = _native_module()
+    if m is None or torch._C._are_functorch_transforms_active():
+        return None
+    return m if all(type(x) in (torch.Tensor, torch.nn.Parameter) for x in xs) else None
+
+
 class _WKV(torch.autograd.Function):
     """Autograd Function over the HIP kernels (theseus/wkv7.py:39-56)."""
 
@@ -449,6 +476,9 @@ def wkv7(r, w, k, v, a, b, state, backend="cuda"):
         raise ValueError(f"Unknown WKV backend: {backend}")
     if not r.is_cuda:
         raise ValueError("CUDA backend requested on CPU; use backend='reference' for tests")
+    native = _native(r, w, k, v, a, b, state)
+    if native is not None:
+        return native.wkv7(r, w, k, v, a, b, state)
     if not torch.is_grad_enabled() or not any(x.requires_grad for x in (r, w, k, v, a, b, state)):
         xs = [x.contiguous() for x in (r, w, k, v, a, b)]
         y, end, _ = extension().forward(*xs, state.float().contiguous(), False)
