@@ -143,6 +143,9 @@ size_t theseus_wkv7_forward_workspace_size(int B, int T, int H, int N, int dtype
 size_t theseus_wkv7_backward_workspace_size(int B, int T, int H, int N, int dtype);
 /* The workspace with which a forward runs fastest, at least theseus_wkv7_forward_workspace_size:
  * more for calls whose few heads leave CUs idle.  saved_states: whether ckpt is given.
+ *  - bf16, N = 64 with saved states and few heads (n = ceil(T/16) > 16 chunks,
+ *    (CUs/4 - B*H) n > 600): the chunk records of the two-launch form and its time split
+ *    (the saved states' order does not depend on it);
  *  - bf16, N = 128: the buffers of up to 9 time segments. */
 size_t theseus_wkv7_forward_best_workspace_size(int B, int T, int H, int N, int dtype, int saved_states);
 

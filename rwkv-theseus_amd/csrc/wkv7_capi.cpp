@@ -97,6 +97,28 @@ static bool split_ok(const Fwd& p) {
            p.ws_bytes >= chunk_forward_split_workspace(p.B, p.T, p.H, cu_count());
 }
 
+// bf16, N = 64 with few heads and many chunks, in training: a chain of chunks per head sets
+// the chunked kernels' time (1.55 us a chunk forward, 2.8 backward, one workgroup per head
+// and the other CUs idle: 4.35 n + 12 us for both, n chunks a head, whatever the heads), so the
+// chunk-record kernels take it, whose scans carry less per chunk, are cut in time and leave
+// the rest to every chunk at once (about 50 + 0.053 B H n us on 256 CUs).  The two meet at
+// B H = 82 - 717 / n; the line is drawn a fifth below.  Forward + backward in us, chunked
+// against records: T=272 8 heads 83 / 64, 40 heads 86 / 89; T=512 20 heads 144 / 96; T=1021
+// 40 heads 276 / 177, 80 heads 280 / 321; T=4096 40 heads 1034 / 647.  The saved states are
+// the chunked kernels' (tiled), so each direction decides by itself: the forward when the
+// workspace holds the records (forward_workspace_best), the backward by its own size.
+static bool rec64_shape(int B, int T, int H, int N, int dtype, int flags) {
+    if (!chunk_ok(B, T, H, N, dtype, flags) || (long long)B * H > 65535 ||
+        wkv7_rec_workspace(1, T, 1, N) >= (1ull << 32))
+        return false;
+    const long long n = (T + kCkptInterval - 1) / kCkptInterval, room = cu_count() / 4 - (long long)B * H;
+    return n > 16 && room > 0 && room * n > 600;
+}
+static bool rec64_ok(const Fwd& p) {
+    return p.ckpt && rec64_shape(p.B, p.T, p.H, p.N, p.dtype, p.flags) && p.ws &&
+           p.ws_bytes >= wkv7_rec_workspace(p.B, p.T, p.H, p.N);
+}
+
 void launch_forward(const Fwd& p) {
     if (p.T == 1 && !p.ckpt && !force_seq() && !(p.flags & FLAG_STATE_KV)) {
         // one step without saved states (the serving step through the operator):
@@ -105,12 +127,14 @@ void launch_forward(const Fwd& p) {
         d.flags = p.flags;
         launch_decode(d);
     } else if (split_ok(p)) launch_chunk_forward_split(p, cu_count());
+    else if (rec64_ok(p)) launch_wkv7_rec_forward(p, cu_count());
     else if (chunk_ok(p.B, p.T, p.H, p.N, p.dtype, p.flags)) launch_chunk_forward(p, cu_count());
     else if (rec_ok(p)) launch_wkv7_rec_forward(p, cu_count());
     else launch_seq_forward(p);
 }
 void launch_backward(const Bwd& p) {
-    if (chunk_ok(p.B, p.T, p.H, p.N, p.dtype, p.flags)) launch_chunk_backward(p, cu_count());
+    if (rec64_shape(p.B, p.T, p.H, p.N, p.dtype, p.flags)) launch_wkv7_rec_backward(p, cu_count());
+    else if (chunk_ok(p.B, p.T, p.H, p.N, p.dtype, p.flags)) launch_chunk_backward(p, cu_count());
     else if (rec_shape(p.B, p.T, p.H, p.N, p.dtype, p.flags)) launch_wkv7_rec_backward(p, cu_count());
     else launch_seq_backward(p);
 }
@@ -128,11 +152,12 @@ size_t forward_workspace_fast(int B, int T, int H, int N, int dtype, int flags) 
 }
 size_t forward_workspace_best(int B, int T, int H, int N, int dtype, bool saved) {
     const size_t need = forward_workspace_fast(B, T, H, N, dtype);
-    if (!saved || !rec_shape(B, T, H, N, dtype, 0)) return need;
+    if (!saved || !(rec_shape(B, T, H, N, dtype, 0) || rec64_shape(B, T, H, N, dtype, 0))) return need;
     const size_t best = wkv7_rec_train_workspace(B, T, H, N, cu_count());
     return best > need ? best : need;
 }
 size_t backward_workspace(int B, int T, int H, int N, int dtype, int flags) {
+    if (rec64_shape(B, T, H, N, dtype, flags)) return wkv7_rec_bwd_workspace(B, T, H, N, cu_count());
     if (chunk_ok(B, T, H, N, dtype, flags)) return chunk_backward_workspace(B, T, H, cu_count());
     if (rec_shape(B, T, H, N, dtype, flags)) return wkv7_rec_bwd_workspace(B, T, H, N, cu_count());
     return seq_backward_workspace(B, T, H, N);
