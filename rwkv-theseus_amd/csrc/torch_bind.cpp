@@ -179,7 +179,7 @@ void gdn_check(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& 
 
 struct Gdn : torch::autograd::Function<Gdn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g,
-                                 const Tensor& beta, const Tensor& s0) {
+                                 const Tensor& beta, const Tensor& s0, bool qk_l2norm) {
         ctx->set_materialize_grads(false);
         gdn_check(q, k, v, g, beta, s0);
         const Dims d(q);
@@ -187,10 +187,12 @@ struct Gdn : torch::autograd::Function<Gdn> {
         const Tensor o = at::empty_like(q), sT = at::empty_like(s0), saved = at::empty(d.saved(), s0.options());
         const size_t need = theseus_gdn_forward_best_workspace_size(d.B, d.T, d.H, d.N, 1);
         const Tensor ws = scratch(need, q);
-        raise_status(theseus_gdn_forward_train(d.B, d.T, d.H, d.N, d.dt, ptr(q), ptr(k), ptr(v), fptr(g), fptr(beta),
-                                               fptr(s0), ptr(o), fptr(sT), fptr(saved), ptr(ws), need, stream_of(q)),
+        raise_status(theseus_gdn_forward_train_ex(d.B, d.T, d.H, d.N, d.dt, qk_l2norm, ptr(q), ptr(k), ptr(v), fptr(g),
+                                                  fptr(beta), fptr(s0), ptr(o), fptr(sT), fptr(saved), ptr(ws), need,
+                                                  stream_of(q)),
                      "theseus_wkv7");
         ctx->save_for_backward({q, k, v, g, beta, saved});
+        ctx->saved_data["qk_l2norm"] = qk_l2norm;
         return {o, sT};
     }
     static variable_list backward(AutogradContext* ctx, variable_list gr) {
@@ -210,18 +212,20 @@ struct Gdn : torch::autograd::Function<Gdn> {
                         at::empty({d.B, d.H, d.N, d.N}, saved.options())};
         const size_t need = theseus_gdn_backward_workspace_size(d.B, d.T, d.H, d.N);
         const Tensor ws = scratch(need, q);
-        raise_status(theseus_gdn_backward(d.B, d.T, d.H, d.N, d.dt, ptr(q), ptr(k), ptr(v), fptr(g), fptr(beta),
-                                          fptr(saved), ptr(dout), fptr(dsT), ptr(o[0]), ptr(o[1]), ptr(o[2]), fptr(o[3]),
-                                          fptr(o[4]), fptr(o[5]), ptr(ws), need, stream_of(q)),
+        raise_status(theseus_gdn_backward_ex(d.B, d.T, d.H, d.N, d.dt, ctx->saved_data["qk_l2norm"].toBool(), ptr(q),
+                                             ptr(k), ptr(v), fptr(g), fptr(beta), fptr(saved), ptr(dout), fptr(dsT),
+                                             ptr(o[0]), ptr(o[1]), ptr(o[2]), fptr(o[3]), fptr(o[4]), fptr(o[5]), ptr(ws),
+                                             need, stream_of(q)),
                      "theseus_wkv7");
+        o.emplace_back();  // (qk_l2norm)
         return o;
     }
 };
 
 std::pair<Tensor, Tensor> gdn(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& beta,
-                              const Tensor& s0) {
+                              const Tensor& s0, bool qk_l2norm) {
     py::gil_scoped_release free;
-    const variable_list o = Gdn::apply(q, k, v, g, beta, s0);
+    const variable_list o = Gdn::apply(q, k, v, g, beta, s0, qk_l2norm);
     return {o[0], o[1]};
 }
 
@@ -229,5 +233,6 @@ std::pair<Tensor, Tensor> gdn(const Tensor& q, const Tensor& k, const Tensor& v,
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("wkv7", &wkv7, "(y, end state) of the recurrence, differentiable");
-    m.def("gdn", &gdn, "(o, end state) of the gated delta rule with gradients, differentiable");
+    m.def("gdn", &gdn, "(o, end state) of the gated delta rule with gradients, differentiable", py::arg("q"),
+          py::arg("k"), py::arg("v"), py::arg("g"), py::arg("beta"), py::arg("s0"), py::arg("qk_l2norm") = false);
 }

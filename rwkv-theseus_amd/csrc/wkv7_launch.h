@@ -89,8 +89,7 @@ struct Gdn {
     int cus = 0;          // CUs the time split may spread the segments over (0: no split)
     float* ckpt = nullptr;  // saved states for gdn backward ([value][key], every 16 steps + final); no split
 };
-// Its backward for N = 128 (wkv7_rec_bwd.hip): q, k as the forward used them (normalised
-// by the caller), dout [B,T,H,N] and the gradients of q, k, v in dtype; g, beta and their
+// Its backward for N = 128 (wkv7_rec_bwd.hip): q, k and qk_norm as the forward had them, dout [B,T,H,N] and the gradients of q, k, v in dtype; g, beta and their
 // gradients [B,T,H] float32; dsT (may be null) and ds0 [B,H,key,value]; the forward's
 // saved states; a workspace of gdn_backward_workspace bytes.
 struct GdnBwd {
@@ -105,6 +104,7 @@ struct GdnBwd {
     void* ws;
     hipStream_t stream;
     int cus = 0;  // CUs the reverse scan's time split may fill
+    int qk_norm = 0;
 };
 size_t gdn_backward_workspace(int B, int T, int H, int cus);
 void launch_gdn_backward(const GdnBwd& p);

@@ -588,7 +588,8 @@ __global__ __launch_bounds__(4 * NK) void wkv7_bwd_chunk(int Tn, int H, int BH, 
 
 // ---------------------------------------------------------------------------
 // The gated delta rule's backward (GDN layers: one decay e^{g_t} per token and head,
-// r = q/sqrt(N), a = k, b = -e^{g} beta k, v' = beta v; q and k as the forward used them).
+// r = q/sqrt(N), a = k, b = -e^{g} beta k, v' = beta v; q and k as the forward used them: with
+// qk_norm L2-normalised here again, and their gradients carried through the normalisation).
 // With gamma the chunk's inclusive cumulative g, the per-key factors above become 16x16
 // decay-ratio masks, every one of them e^{(a later gamma) - (an earlier one)} <= 1, so
 // nothing overflows for any decay (as gdn_prep in the forward):
@@ -607,7 +608,7 @@ __global__ __launch_bounds__(4 * NK) void wkv7_bwd_chunk(int Tn, int H, int BH, 
 // per key), so wkv7_bwd_scan runs them unchanged.
 // ---------------------------------------------------------------------------
 template <typename TI>
-__global__ __launch_bounds__(64) void gdn_bwd_prep(int Tn, int H, const TI* __restrict__ q, const TI* __restrict__ k,
+__global__ __launch_bounds__(64) void gdn_bwd_prep(int Tn, int H, int qk_norm, const TI* __restrict__ q, const TI* __restrict__ k,
                                                    const float* __restrict__ g, const float* __restrict__ beta,
                                                    uint8_t* __restrict__ ws) {
     using R = BwdRec<BNK>;
@@ -618,29 +619,44 @@ __global__ __launch_bounds__(64) void gdn_bwd_prep(int Tn, int H, const TI* __re
     const long tok0 = (long)bb * Tn + t0;
     auto row = [&](int t) { return ((tok0 + t) * H + h) * (long)BNK; };
     const float rs = 1.f / __builtin_sqrtf((float)BNK);
-    __shared__ float gsh[3][BC];  // gamma_t, gamma_{t-1}, beta_t (past the end: 0)
+    __shared__ float gsh[5][BC];  // gamma_t, gamma_{t-1}, beta_t, k_t's and q_t's norm factors (past the end: 0)
     const bool tv = r16 < L;
     const int tl = tv ? r16 : 0;  // (clamped: every lane loads)
     const float g_ = g[(tok0 + tl) * H + h], b_ = beta[(tok0 + tl) * H + h];
     const uint32_t tm = lane_mask(tv);
     const float gt = keep(tm, g_), bt = keep(tm, b_);
     const float gam = row_prefix_sum(gt), gm1 = row_prev(gam, 0.f), gL = row_last(gam);
-    if (q4 == 0) gsh[0][r16] = gam, gsh[1][r16] = gm1, gsh[2][r16] = bt;
     uint8_t* const rec = ws + ((size_t)bh * nchunk + c) * R::BYTES;
-    const float sb = -bt * __expf(gL - gm1);  // B^ = sb k for the lane's token
-    f32x4_t KK = zero4(), KR = zero4();
+    float kr[BKS][8], qr[BKS][8], ssk = 0.f, ssq = 0.f;
 #pragma unroll
     for (int ks = 0; ks < BKS; ks++) {
         const int c0 = 32 * ks + 4 * q4;
         const float4 ka = keep4(tm, ld4f(k + row(tl) + c0)), kb = keep4(tm, ld4f(k + row(tl) + c0 + 16));
         const float4 qa = keep4(tm, ld4f(q + row(tl) + c0)), qb = keep4(tm, ld4f(q + row(tl) + c0 + 16));
-        const float kr[8] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
-        const float qr[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+        const float kx[8] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
+        const float qx[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            kr[ks][e] = kx[e], qr[ks][e] = qx[e];
+            ssk += kx[e] * kx[e], ssq += qx[e] * qx[e];
+        }
+    }
+    float nk = 1.f, nq = 1.f;  // the rows' L2-norm factors (gdn_prep's)
+    if (qk_norm) {
+        ssk += __shfl_xor(ssk, 16), ssq += __shfl_xor(ssq, 16);
+        ssk += __shfl_xor(ssk, 32), ssq += __shfl_xor(ssq, 32);
+        nk = __frsqrt_rn(ssk + 1e-6f), nq = __frsqrt_rn(ssq + 1e-6f);
+    }
+    if (q4 == 0) gsh[0][r16] = gam, gsh[1][r16] = gm1, gsh[2][r16] = bt, gsh[3][r16] = nk, gsh[4][r16] = nq;
+    const float sb = -bt * __expf(gL - gm1);  // B^ = sb k for the lane's token
+    f32x4_t KK = zero4(), KR = zero4();
+#pragma unroll
+    for (int ks = 0; ks < BKS; ks++) {
         float br8[8];
 #pragma unroll
-        for (int e = 0; e < 8; e++) br8[e] = kr[e] * sb;
+        for (int e = 0; e < 8; e++) kr[ks][e] *= nk, qr[ks][e] *= nq, br8[e] = kr[ks][e] * sb;
         uint4 kh, kl, qh, ql, bh_, bl;
-        pack8(kr, kh, kl), pack8(qr, qh, ql), pack8(br8, bh_, bl);
+        pack8(kr[ks], kh, kl), pack8(qr[ks], qh, ql), pack8(br8, bh_, bl);
         uint8_t* bf = rec + R::BF + (size_t)(2 * ks) * 1024;
         put_frag(bf, lane, bh_);
         put_frag(bf + 1024, lane, bl);
@@ -669,8 +685,8 @@ __global__ __launch_bounds__(64) void gdn_bwd_prep(int Tn, int H, const TI* __re
         const int t = 4 * q4 + e;
         krow[e] = k + row(t < L ? t : 0) + r16;
         qrow[e] = q + row(t < L ? t : 0) + r16;
-        ea[e] = t < L ? __expf(gsh[1][t]) : 0.f;
-        er[e] = t < L ? rs * __expf(gsh[0][t]) : 0.f;
+        ea[e] = t < L ? gsh[3][t] * __expf(gsh[1][t]) : 0.f;
+        er[e] = t < L ? gsh[4][t] * rs * __expf(gsh[0][t]) : 0.f;
     }
 #pragma unroll
     for (int tj = 0; tj < BTJ; tj++) {
@@ -696,10 +712,12 @@ struct GdnChunkLds {
     float gam[BC], gm1[BC], beta[BC];
     float csum[BTJ][BNK];
     float pv[BTJ][BC], pd[BTJ][BC], pk[BTJ][BC];  // per wave and token: sum v dV', sum dlogd, sum k dB
+    float nk[BTJ][BC], nq[BTJ][BC];  // with qk_norm: sum k^2, sum q^2; then sum k dk, sum q dq of the normalised
 };
 
 template <typename TI>
-__global__ __launch_bounds__(512) void gdn_bwd_chunk(int Tn, int H, int BH, int per_xcd, const TI* __restrict__ q,
+__global__ __launch_bounds__(512) void gdn_bwd_chunk(int Tn, int H, int BH, int per_xcd, int qk_norm,
+                                                     const TI* __restrict__ q,
                                                      const TI* __restrict__ k, const TI* __restrict__ v,
                                                      const float* __restrict__ g, const float* __restrict__ beta,
                                                      const TI* __restrict__ dy, const float* __restrict__ ckpt,
@@ -755,7 +773,15 @@ __global__ __launch_bounds__(512) void gdn_bwd_chunk(int Tn, int H, int BH, int 
         kD[e] = keep(lane_mask(ok), k_);
         rD[e] = keep(lane_mask(ok), q_) * rs;
     }
+    // (with qk_norm the planes hold k and r as given: their products are scaled below)
     put_split(sm.K, kD, lane, wv), put_split(sm.R, rD, lane, wv);
+    if (qk_norm) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float sk = row_sum16(kD[e] * kD[e]), sq = row_sum16(rD[e] * rD[e]);
+            if (r16 == 0) sm.nk[wv][4 * q4 + e] = sk, sm.nq[wv][4 * q4 + e] = sq;
+        }
+    }
 #pragma unroll
     for (int ks = 0; ks < BKS; ks++)
 #pragma unroll
@@ -777,6 +803,22 @@ __global__ __launch_bounds__(512) void gdn_bwd_chunk(int Tn, int H, int BH, int 
 #pragma unroll
     for (int e = 0; e < 4; e++) gr[e] = sm.gam[4 * q4 + e], gm1r[e] = sm.gm1[4 * q4 + e], br[e] = sm.beta[4 * q4 + e];
     const float gc = sm.gam[cc], gm1c = sm.gm1[cc], bc = sm.beta[cc], gL = sm.gam[BC - 1];
+    // the norm factors x * rsqrt(sum x^2 + 1e-6) of rows rr and column token cc (r = q / sqrt(N))
+    float nkr[4] = {1.f, 1.f, 1.f, 1.f}, nqr[4] = {1.f, 1.f, 1.f, 1.f}, nkc = 1.f;
+    if (qk_norm) {
+        float sk = 0.f;
+#pragma unroll
+        for (int u = 0; u < BTJ; u++) sk += sm.nk[u][cc];
+        nkc = __frsqrt_rn(sk + 1e-6f);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            float a = 0.f, b = 0.f;
+#pragma unroll
+            for (int u = 0; u < BTJ; u++) a += sm.nk[u][4 * q4 + e], b += sm.nq[u][4 * q4 + e];
+            nkr[e] = __frsqrt_rn(a + 1e-6f), nqr[e] = __frsqrt_rn(b * (float)BNK + 1e-6f);
+            kD[e] *= nkr[e], rD[e] *= nqr[e];
+        }
+    }
     // Gram matrices over the keys and the wave's products k S0^T, k H^T
     f32x4_t KK = zero4(), RK = zero4(), kS = zero4(), kH = zero4();
 #pragma unroll
@@ -792,6 +834,7 @@ __global__ __launch_bounds__(512) void gdn_bwd_chunk(int Tn, int H, int BH, int 
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         const int rr = 4 * q4 + e;
+        KK[e] *= nkr[e] * nkc, RK[e] *= nqr[e] * nkc, kS[e] *= nkr[e], kH[e] *= nkr[e];
         Aab[e] = cc < rr ? -bc * KK[e] * __expf(gm1r[e] - gm1c) : 0.f;
         AabT[e] = rr < cc ? -br[e] * KK[e] * __expf(gm1c - gm1r[e]) : 0.f;
         Aak[e] = cc < rr ? KK[e] * __expf(gm1r[e] - gc) : 0.f;
@@ -932,9 +975,30 @@ __global__ __launch_bounds__(512) void gdn_bwd_chunk(int Tn, int H, int BH, int 
         const float sd = row_sum16(sx[e] + sy[e]), skb = row_sum16(kD[e] * gB[e]);
         if (r16 == 0) sm.pd[wv][4 * q4 + e] = sd, sm.pk[wv][4 * q4 + e] = skb;
     }
-    put(dq, gR * rs);
-    put(dk, gK + gA - egb * gB);
-    __syncthreads();  // pd, pk
+    // gradients of q and k as the recurrence takes them; with qk_norm dx = n (dy - y (y . dy)) of
+    // y = n x, the dot over the token's keys summed over the waves
+    f32x4_t gq = gR * rs, gk = gK + gA - egb * gB;
+    if (qk_norm) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float sk = row_sum16(kD[e] * gk[e]), sq = row_sum16(rD[e] * gR[e]);  // (q . dq = r . dr)
+            if (r16 == 0) sm.nk[wv][4 * q4 + e] = sk, sm.nq[wv][4 * q4 + e] = sq;
+        }
+    }
+    __syncthreads();  // pd, pk, nk, nq
+    if (qk_norm) {
+        const float sn = __builtin_sqrtf((float)BNK);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            float a = 0.f, b = 0.f;
+#pragma unroll
+            for (int u = 0; u < BTJ; u++) a += sm.nk[u][4 * q4 + e], b += sm.nq[u][4 * q4 + e];
+            gk[e] = nkr[e] * (gk[e] - kD[e] * a);
+            gq[e] = nqr[e] * (gq[e] - rD[e] * sn * b);
+        }
+    }
+    put(dq, gq);
+    put(dk, gk);
     if (wv == 0 && lane < L) {
         float spv = 0.f, spd = 0.f, spk = 0.f;
 #pragma unroll
@@ -1009,12 +1073,12 @@ static void launch_gdn_bwd(const GdnBwd& p) {
     const int nchunk = (p.T + BC - 1) / BC, BH = p.B * p.H;
     const TI *q = static_cast<const TI*>(p.q), *k = static_cast<const TI*>(p.k), *v = static_cast<const TI*>(p.v),
              *dout = static_cast<const TI*>(p.dout);
-    hipLaunchKernelGGL(gdn_bwd_prep<TI>, dim3(nchunk, BH), dim3(64), 0, p.stream, p.T, p.H, q, k, p.g, p.beta,
-                       static_cast<uint8_t*>(p.ws));
+    hipLaunchKernelGGL(gdn_bwd_prep<TI>, dim3(nchunk, BH), dim3(64), 0, p.stream, p.T, p.H, p.qk_norm, q, k,
+                       p.g, p.beta, static_cast<uint8_t*>(p.ws));
     const float* const hbuf = scan_back<BNK, TI>(p.T, p.H, BH, 1, p.dsT, dout, p.ds0, p.ws, p.cus, p.stream);
     const int jobs = nchunk * BH, per_xcd = (jobs + 7) / 8;
-    hipLaunchKernelGGL(gdn_bwd_chunk<TI>, dim3(8 * per_xcd), dim3(512), 0, p.stream, p.T, p.H, BH, per_xcd, q, k, v,
-                       p.g, p.beta, dout, p.ckpt, hbuf, static_cast<TI*>(p.dq), static_cast<TI*>(p.dk),
+    hipLaunchKernelGGL(gdn_bwd_chunk<TI>, dim3(8 * per_xcd), dim3(512), 0, p.stream, p.T, p.H, BH, per_xcd,
+                       p.qk_norm, q, k, v, p.g, p.beta, dout, p.ckpt, hbuf, static_cast<TI*>(p.dq), static_cast<TI*>(p.dk),
                        static_cast<TI*>(p.dv), p.dg, p.dbeta);
 }
 void launch_gdn_backward(const GdnBwd& p) {

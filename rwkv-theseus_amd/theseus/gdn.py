@@ -18,8 +18,7 @@ carries the kernels' gradients back to q, k, v, g and beta.  When no gradient is
 of the gated delta rule instead (``theseus_gdn_forward``, include/theseus_gdn.h); with
 gradients at head size 128, the chunked forward with saved states and the chunked backward
 (``theseus_gdn_forward_train`` / ``theseus_gdn_backward``).  Like transformers'
-functions it computes in float32 (the operands are passed to the kernels as float32)
-and returns the output in the query's dtype.  The state must be square (K == V, the
+functions it computes in float32 and returns the output in the query's dtype.  The state must be square (K == V, the
 kernels' N, 2..128).
 
 ``chunk_gated_delta_rule`` and ``recurrent_gated_delta_rule`` have transformers'
@@ -42,15 +41,16 @@ CHUNKED_GRAD_HEAD_SIZES = (128,)
 
 
 class _GDN(torch.autograd.Function):
-    """The gated delta rule on the chunked kernels with gradients: q, k (as the layer
-    normalised them), v, g, beta, s0 float32 or q/k/v bfloat16; saved states between
+    """The gated delta rule on the chunked kernels with gradients: q, k (L2-normalised in the
+    kernels when qk_l2norm), v, g, beta, s0 float32 or q/k/v bfloat16; saved states between
     the two calls."""
 
     @staticmethod
-    def forward(ctx, q, k, v, g, beta, s0):
+    def forward(ctx, q, k, v, g, beta, s0, qk_l2norm=False):
         ctx.set_materialize_grads(False)
-        o, sT, saved = extension().gdn_forward_train(q, k, v, g, beta, s0)
+        o, sT, saved = extension().gdn_forward_train(q, k, v, g, beta, s0, qk_l2norm)
         ctx.save_for_backward(q, k, v, g, beta, saved)
+        ctx.qk_l2norm = qk_l2norm
         return o, sT
 
     @staticmethod
@@ -58,7 +58,7 @@ class _GDN(torch.autograd.Function):
         q, k, v, g, beta, saved = ctx.saved_tensors
         do = torch.zeros_like(q) if do is None else do.to(q.dtype).contiguous()
         dsT = None if dsT is None else dsT.float().contiguous()
-        return extension().gdn_backward(q, k, v, g, beta, saved, do, dsT)
+        return (*extension().gdn_backward(q, k, v, g, beta, saved, do, dsT, ctx.qk_l2norm), None)
 
 
 def l2norm(x, dim=-1, eps=1e-6):
@@ -91,16 +91,19 @@ def gated_delta_rule(query, key, value, g, beta, initial_state=None, output_fina
         o, sT = extension().gdn_forward(q, k, v, g.float().contiguous(), beta.float().contiguous(), s0,
                                         qk_l2norm=use_qk_l2norm_in_kernel)
         return o.to(out_dtype), (sT if output_final_state else None)
-    if use_qk_l2norm_in_kernel:
-        query, key = l2norm(query), l2norm(key)
     if (K in CHUNKED_GRAD_HEAD_SIZES and query.is_cuda
             and extension().lib.theseus_gdn_backward_workspace_size(B, T, H, K) > 0):
-        # gradients wanted: the chunked forward with saved states and the chunked backward,
-        # in float32 as transformers' functions compute
-        q, k, v, gf, bf = (x.float().contiguous() for x in (query, key, value, g, beta))
+        # gradients wanted: the chunked forward with saved states and the chunked backward, which
+        # take bf16 or fp32 q/k/v as they are and normalise q and k themselves (float32 inside)
+        io = query.dtype if query.dtype == key.dtype == value.dtype and query.dtype in (torch.bfloat16, torch.float32) \
+            else torch.float32
+        q, k, v = (x.to(io).contiguous() for x in (query, key, value))
+        gf, bf = g.float().contiguous(), beta.float().contiguous()
         native = _native(q, k, v, gf, bf, s0)
-        o, sT = (_GDN.apply if native is None else native.gdn)(q, k, v, gf, bf, s0)
+        o, sT = (_GDN.apply if native is None else native.gdn)(q, k, v, gf, bf, s0, use_qk_l2norm_in_kernel)
         return o.to(out_dtype), (sT if output_final_state else None)
+    if use_qk_l2norm_in_kernel:
+        query, key = l2norm(query), l2norm(key)
     q, k, v, gf, bf = (x.float() for x in (query, key, value, g, beta))
     eg = torch.exp(gf)
     r = q * (K ** -0.5)

@@ -141,8 +141,12 @@ class Extension:
         lib.theseus_gdn_forward_best_workspace_size.restype = sz
         lib.theseus_gdn_forward_train.argtypes = [i32] * 5 + [vp] * 9 + [vp, sz, vp]
         lib.theseus_gdn_forward_train.restype = i32
+        lib.theseus_gdn_forward_train_ex.argtypes = [i32] * 6 + [vp] * 9 + [vp, sz, vp]
+        lib.theseus_gdn_forward_train_ex.restype = i32
         lib.theseus_gdn_backward.argtypes = [i32] * 5 + [vp] * 14 + [vp, sz, vp]
         lib.theseus_gdn_backward.restype = i32
+        lib.theseus_gdn_backward_ex.argtypes = [i32] * 6 + [vp] * 14 + [vp, sz, vp]
+        lib.theseus_gdn_backward_ex.restype = i32
         lib.theseus_gdn_backward_workspace_size.argtypes = [i32] * 4
         lib.theseus_gdn_backward_workspace_size.restype = sz
         self.abi_version = lib.theseus_wkv7_abi_version()
@@ -303,10 +307,10 @@ class Extension:
                                    and tuple(s0.shape) == (B, H, N, N)):
             raise RuntimeError("theseus_gdn: expected contiguous float32 state [B,H,N,N]")
 
-    def gdn_forward_train(self, q, k, v, g, beta, s0):
+    def gdn_forward_train(self, q, k, v, g, beta, s0, qk_l2norm=False):
         """The gated delta rule forward of a call that needs gradients
-        (theseus_gdn_forward_train): q and k used as given, and the saved states for
-        ``gdn_backward``.  Returns (o in q's dtype, sT, saved [B,H,ceil(T/16)+1,N,N])."""
+        (theseus_gdn_forward_train_ex): q and k used as given, or L2-normalised in the kernel,
+        and the saved states for ``gdn_backward``.  Returns (o in q's dtype, sT, saved [B,H,ceil(T/16)+1,N,N])."""
         self._gdn_check(q, k, v, g, beta, s0)
         B, T, H, N = q.shape
         with _on(q.device):
@@ -315,13 +319,14 @@ class Extension:
             saved = torch.empty((B, H, self.checkpoint_count(T), N, N), dtype=torch.float32, device=q.device)
             ws, nbytes = _workspace(self.lib.theseus_gdn_forward_best_workspace_size(B, T, H, N, 1), q.device)
             p = lambda t: t.data_ptr()  # noqa: E731
-            self._raise(self.lib.theseus_gdn_forward_train(
-                B, T, H, N, _BF16 if q.dtype == torch.bfloat16 else _FP32, p(q), p(k), p(v), p(g), p(beta), p(s0),
+            self._raise(self.lib.theseus_gdn_forward_train_ex(
+                B, T, H, N, _BF16 if q.dtype == torch.bfloat16 else _FP32, 1 if qk_l2norm else 0, p(q), p(k), p(v), p(g), p(beta), p(s0),
                 p(o), p(sT), p(saved), None if ws is None else p(ws), nbytes, _stream(q.device)))
         return o, sT, saved
 
-    def gdn_backward(self, q, k, v, g, beta, saved, dout, dsT):
-        """Backward of ``gdn_forward_train`` (theseus_gdn_backward, N = 128): dout in q's
+    def gdn_backward(self, q, k, v, g, beta, saved, dout, dsT, qk_l2norm=False):
+        """Backward of ``gdn_forward_train`` (theseus_gdn_backward_ex, N = 128; the same
+        ``qk_l2norm``): dout in q's
         dtype, dsT [B,H,key,value] float32 or None.  Returns (dq, dk, dv in q's dtype, dg,
         dbeta [B,T,H] and ds0 [B,H,key,value] float32)."""
         self._gdn_check(q, k, v, g, beta, dsT)
@@ -338,8 +343,8 @@ class Extension:
             ds0 = torch.empty((B, H, N, N), dtype=torch.float32, device=q.device)
             ws, nbytes = _workspace(self.lib.theseus_gdn_backward_workspace_size(B, T, H, N), q.device)
             p = lambda t: None if t is None else t.data_ptr()  # noqa: E731
-            self._raise(self.lib.theseus_gdn_backward(
-                B, T, H, N, _BF16 if q.dtype == torch.bfloat16 else _FP32, p(q), p(k), p(v), p(g), p(beta),
+            self._raise(self.lib.theseus_gdn_backward_ex(
+                B, T, H, N, _BF16 if q.dtype == torch.bfloat16 else _FP32, 1 if qk_l2norm else 0, p(q), p(k), p(v), p(g), p(beta),
                 p(saved), p(dout), p(dsT), p(dq), p(dk), p(dv), p(dg), p(dbeta), p(ds0), p(ws), nbytes,
                 _stream(q.device)))
         return dq, dk, dv, dg, dbeta, ds0
