@@ -12,7 +12,7 @@
 // vectors); row sums are 8-lane butterflies.  Parameter gradients are
 // accumulated per (head, token block) and reduced over token blocks by
 // reduce_blocks in a fixed order, so results are deterministic.
-#include "../../include/theseus_timemix.h"
+#include "../../include/theseus_timemix_ex.h"
 #include "../../include/theseus_wkv7.h"
 #include "wkv7_common.h"
 
@@ -92,7 +92,7 @@ __device__ __forceinline__ float sum8(float x) {  // over the 8 lanes of a head 
 // ---------------------------------------------------------------- shift-lerp
 // Thread: 8 channels of SLT consecutive tokens (the six coefficient vectors loaded once,
 // all x rows issued before use, x[t-1] taken from the previous token's registers).
-constexpr int SLT = 8;
+template <int SLT>
 __global__ __launch_bounds__(256) void shift_lerp_fwd(long M, int T, int C, const uint16_t* __restrict__ x,
                                                       const uint16_t* __restrict__ st,
                                                       const float* __restrict__ coef, uint16_t* o0,
@@ -317,6 +317,22 @@ __global__ __launch_bounds__(256) void add_param_bf16(long n8, int C, const uint
     st_bf8(out + 8 * i, o);
 }
 
+// ---------------------------------------------------------------- parameters
+// n parameter vectors of C elements, bf16 or float32, as float32 rows: one launch where a
+// conversion each (13 of a layer with bf16 weights, and the coefficients' stack) had been 16
+// of the 35 launches of a prompt.
+constexpr int MAX_PACK = 16;
+struct Pack {
+    const void* src[MAX_PACK];
+    uint32_t bf16;  // bit n: src[n] is bf16
+};
+__global__ __launch_bounds__(256) void pack_params(Pack p, int C, float* __restrict__ out) {
+    const int n = blockIdx.y, c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= C) return;
+    out[(long)n * C + c] = (p.bf16 >> n & 1) ? bf16_to_f32(static_cast<const uint16_t*>(p.src[n])[c])
+                                             : static_cast<const float*>(p.src[n])[c];
+}
+
 // ---------------------------------------------------------------- kk / k-mod
 // The forward kernels: ceil(H / 8) x ceil(M / (4 U)) workgroups of 256 lanes, head groups
 // first (workgroups next in line read neighbouring 1 KB runs of the same tokens; token-first
@@ -327,23 +343,39 @@ __global__ __launch_bounds__(256) void add_param_bf16(long n8, int C, const uint
 // KU / FU tokens per wave: 4 for long inputs, 1 for short ones (a serving step's 64 tokens
 // would fill only 40 workgroups with 4: 7.3 against 4.5 µs per gn_fwd call)
 constexpr int U_LONG = 4;
+// zw (may be null): also w = (w0 + zw).to(bf16) into wd, so that a call without gradients needs
+// no launch of its own for it (4.7 us of a 64-lane serving step at C = 5120).
 template <int KU>
 __global__ __launch_bounds__(256) void kk_fwd(long M, int H, int C, const uint16_t* __restrict__ k,
                                               const uint16_t* __restrict__ za, const float* __restrict__ a0p,
                                               const float* __restrict__ kkp, const float* __restrict__ kap,
-                                              uint16_t* kw, uint16_t* aw, uint16_t* bw) {
+                                              uint16_t* kw, uint16_t* aw, uint16_t* bw,
+                                              const uint16_t* __restrict__ zw, const float* __restrict__ w0p,
+                                              uint16_t* wd) {
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, sub = l & 7;
     const int ng = (H + 7) / 8, h = (int)(blockIdx.x % ng) * 8 + (l >> 3);
     const bool hok = h < H;
     const int c = (hok ? h : 0) * HN + 8 * sub;
     const long mb = ((long)(blockIdx.x / ng) * 4 + w) * KU;
-    uint4 kr[KU], zr[KU];
+    uint4 kr[KU], zr[KU], wr[KU];
 #pragma unroll
     for (int u = 0; u < KU; u++) {
         const bool ok = hok && mb + u < M;
         const long o = ok ? (mb + u) * C + c : c;
         kr[u] = ld_str8(k + o);
         zr[u] = ld_str8(za + o);
+        if (zw) wr[u] = ld_str8(zw + o);
+    }
+    if (zw) {  // the decay input, add_param_bf16's sum
+        const V8 w0 = ld_f8(w0p + c);
+#pragma unroll
+        for (int u = 0; u < KU; u++) {
+            const V8 z = cvt_bf8(wr[u]);
+            V8 o;
+#pragma unroll
+            for (int e = 0; e < 8; e++) o.x[e] = w0.x[e] + z.x[e];
+            if (hok && mb + u < M) st_bf8(wd + (mb + u) * C + c, o);
+        }
     }
     const V8 kk_ = ld_f8(kkp + c), ka = ld_f8(kap + c), a0 = ld_f8(a0p + c);
 #pragma unroll
@@ -668,10 +700,19 @@ int theseus_tm_shift_lerp_fwd(int B, int T, int C, const void* x, const void* st
     if (!x || !st || !coef || !out) return THESEUS_WKV7_ERR_NULL;
     for (int n = 0; n < 6; n++)
         if (!out[n]) return THESEUS_WKV7_ERR_NULL;
-    const long M = (long)B * T, total = (M + tmix::SLT - 1) / tmix::SLT * (C / 8);
-    hipLaunchKernelGGL(tmix::shift_lerp_fwd, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, M, T, C,
-                       (const uint16_t*)x, (const uint16_t*)st, coef, (uint16_t*)out[0], (uint16_t*)out[1],
-                       (uint16_t*)out[2], (uint16_t*)out[3], (uint16_t*)out[4], (uint16_t*)out[5]);
+    // tokens per thread: the most that still gives two workgroups per CU (512); few tokens get
+    // one each, since a thread's tokens wait on their rows one after another (64 tokens of
+    // C = 5120 at 8: 20 workgroups, 10.9 us; at 1: 4.8; 777 of C = 2048: 9.3 against 8.3)
+    const long M = (long)B * T, cv = C / 8;
+    auto launch = [&](auto kernel, int S) {
+        const long total = (M + S - 1) / S * cv;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, M, T, C,
+                           (const uint16_t*)x, (const uint16_t*)st, coef, (uint16_t*)out[0], (uint16_t*)out[1],
+                           (uint16_t*)out[2], (uint16_t*)out[3], (uint16_t*)out[4], (uint16_t*)out[5]);
+    };
+    if (M / 8 * cv >= 512 * 256) launch(tmix::shift_lerp_fwd<8>, 8);
+    else if (M / 2 * cv >= 512 * 256) launch(tmix::shift_lerp_fwd<2>, 2);
+    else launch(tmix::shift_lerp_fwd<1>, 1);
     return tm_status();
 }
 
@@ -708,16 +749,46 @@ int theseus_tm_add_param_fwd(int B, int T, int C, const void* z, const float* p,
     return tm_status();
 }
 
-int theseus_tm_kk_fwd(int B, int T, int C, const void* k, const void* za, const float* a0, const float* k_k,
-                      const float* k_a, void* kw, void* aw, void* bw, hipStream_t stream) {
-    if (int e = tm_check(B, T, C)) return e;
-    if (!k || !za || !a0 || !k_k || !k_a || !kw || !aw || !bw) return THESEUS_WKV7_ERR_NULL;
+static void launch_kk(int B, int T, int C, const void* k, const void* za, const float* a0, const float* k_k,
+                      const float* k_a, void* kw, void* aw, void* bw, const void* zw, const float* w0, void* w,
+                      hipStream_t stream) {
     const int H = C / tmix::HN;
     const long M = (long)B * T;
     const int U = M >= 4096 ? tmix::U_LONG : 1;
     hipLaunchKernelGGL(U == 1 ? tmix::kk_fwd<1> : tmix::kk_fwd<tmix::U_LONG>,
                        dim3((unsigned)((M + 4 * U - 1) / (4 * U) * ((H + 7) / 8))), dim3(256), 0, stream, M, H, C,
-                       (const uint16_t*)k, (const uint16_t*)za, a0, k_k, k_a, (uint16_t*)kw, (uint16_t*)aw, (uint16_t*)bw);
+                       (const uint16_t*)k, (const uint16_t*)za, a0, k_k, k_a, (uint16_t*)kw, (uint16_t*)aw,
+                       (uint16_t*)bw, (const uint16_t*)zw, w0, (uint16_t*)w);
+}
+
+int theseus_tm_kk_fwd(int B, int T, int C, const void* k, const void* za, const float* a0, const float* k_k,
+                      const float* k_a, void* kw, void* aw, void* bw, hipStream_t stream) {
+    if (int e = tm_check(B, T, C)) return e;
+    if (!k || !za || !a0 || !k_k || !k_a || !kw || !aw || !bw) return THESEUS_WKV7_ERR_NULL;
+    launch_kk(B, T, C, k, za, a0, k_k, k_a, kw, aw, bw, nullptr, nullptr, nullptr, stream);
+    return tm_status();
+}
+
+int theseus_tm_kk_w_fwd(int B, int T, int C, const void* k, const void* za, const float* a0, const float* k_k,
+                        const float* k_a, void* kw, void* aw, void* bw, const void* zw, const float* w0, void* w,
+                        hipStream_t stream) {
+    if (int e = tm_check(B, T, C)) return e;
+    if (!k || !za || !a0 || !k_k || !k_a || !kw || !aw || !bw || !zw || !w0 || !w) return THESEUS_WKV7_ERR_NULL;
+    launch_kk(B, T, C, k, za, a0, k_k, k_a, kw, aw, bw, zw, w0, w, stream);
+    return tm_status();
+}
+
+int theseus_tm_pack_params(int n, int C, const void* const* src, const int* dtypes, float* out, hipStream_t stream) {
+    if (n < 1 || n > tmix::MAX_PACK || C < 1) return THESEUS_WKV7_ERR_SHAPE;
+    if (!src || !dtypes || !out) return THESEUS_WKV7_ERR_NULL;
+    tmix::Pack p{};
+    for (int i = 0; i < n; i++) {
+        if (!src[i]) return THESEUS_WKV7_ERR_NULL;
+        if (dtypes[i] != THESEUS_WKV7_BF16 && dtypes[i] != THESEUS_WKV7_FP32) return THESEUS_WKV7_ERR_DTYPE;
+        p.src[i] = src[i];
+        if (dtypes[i] == THESEUS_WKV7_BF16) p.bf16 |= 1u << i;
+    }
+    hipLaunchKernelGGL(tmix::pack_params, dim3((C + 255) / 256, n), dim3(256), 0, stream, p, C, out);
     return tm_status();
 }
 

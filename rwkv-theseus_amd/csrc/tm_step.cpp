@@ -10,7 +10,7 @@
 // token issuing these launches and allocating their outputs (C = 5120, B = 64), twice the
 // kernels' own 0.13 ms; here every intermediate lives in the caller's workspace.
 #include "../../include/theseus_gemm.h"
-#include "../../include/theseus_timemix.h"
+#include "../../include/theseus_timemix_ex.h"
 #include "../../include/theseus_wkv7.h"
 
 #include <hip/hip_runtime.h>
@@ -107,9 +107,8 @@ int theseus_tm_serving_step(const theseus_tm_layer* L, int B, const void* x, con
     problems(L, ws, o, a, b);
     if ((st = theseus_gemm_rows_group(B, 6, a, at(o.gws_a), o.ga, stream))) return st;
     if ((st = theseus_gemm_rows_group(B, 3, b, at(o.gws_b), o.gb, stream))) return st;
-    if ((st = theseus_tm_add_param_fwd(B, 1, C, at(o.up[0]), L->w0, at(o.w), stream))) return st;
-    if ((st = theseus_tm_kk_fwd(B, 1, C, at(o.k), at(o.up[1]), L->a0, L->k_k, L->k_a, at(o.kw), at(o.aw), at(o.bw),
-                                stream)))
+    if ((st = theseus_tm_kk_w_fwd(B, 1, C, at(o.k), at(o.up[1]), L->a0, L->k_k, L->k_a, at(o.kw), at(o.aw), at(o.bw),
+                                  at(o.up[0]), L->w0, at(o.w), stream)))
         return st;
     if (wkv_out == wkv_in)
         st = theseus_wkv7_decode_step(B, H, N, THESEUS_WKV7_BF16, at(o.r), at(o.w), at(o.kw), at(o.v), at(o.aw),

@@ -47,6 +47,8 @@ def _lib():
             lib.theseus_tm_shift_lerp_bwd.argtypes = [i32] * 3 + [vp] * 8 + [sz, vp]
             lib.theseus_tm_add_param_fwd.argtypes = [i32] * 3 + [vp] * 3 + [vp]
             lib.theseus_tm_kk_fwd.argtypes = [i32] * 3 + [vp] * 8 + [vp]
+            lib.theseus_tm_kk_w_fwd.argtypes = [i32] * 3 + [vp] * 11 + [vp]
+            lib.theseus_tm_pack_params.argtypes = [i32] * 2 + [vp] * 3 + [vp]
             lib.theseus_tm_kk_workspace.argtypes = [i32] * 3
             lib.theseus_tm_kk_workspace.restype = sz
             lib.theseus_tm_kk_bwd.argtypes = [i32] * 3 + [vp] * 15 + [sz, vp]
@@ -57,8 +59,8 @@ def _lib():
             lib.theseus_tm_serving_step_workspace.argtypes = [ctypes.POINTER(TmLayer), i32]
             lib.theseus_tm_serving_step_workspace.restype = sz
             lib.theseus_tm_serving_step.argtypes = [ctypes.POINTER(TmLayer), i32] + [vp] * 7 + [sz, vp]
-            for n in ("shift_lerp_fwd", "shift_lerp_bwd", "add_param_fwd", "kk_fwd", "kk_bwd", "gn_fwd", "gn_bwd",
-                      "serving_step"):
+            for n in ("shift_lerp_fwd", "shift_lerp_bwd", "add_param_fwd", "kk_fwd", "kk_w_fwd", "kk_bwd", "gn_fwd",
+                      "gn_bwd", "pack_params", "serving_step"):
                 getattr(lib, "theseus_tm_" + n).restype = i32
             _ready = True
         except AttributeError:
@@ -183,27 +185,50 @@ def native_layer(m):
     return _cached("tm_layer", params, make)
 
 
+def pack_params(params, C):
+    """The C-element parameters as float32 rows [n, C] in one launch (bf16 or float32 ones; others
+    are converted first): a call's own copies, the kernels' inputs without gradients."""
+    src = [p.detach() if p.dtype in (torch.float32, torch.bfloat16) else p.detach().float() for p in params]
+    src = [p if p.is_contiguous() else p.contiguous() for p in src]
+    n, dev = len(src), src[0].device
+    out = torch.empty(n, C, dtype=torch.float32, device=dev)
+    ptrs = (ctypes.c_void_p * n)(*[p.data_ptr() for p in src])
+    dts = (ctypes.c_int * n)(*[0 if p.dtype == torch.bfloat16 else 1 for p in src])
+    with torch.cuda.device(dev):
+        _check(_lib().theseus_tm_pack_params(n, C, ptrs, dts, _p(out), _s(dev)))
+    return out
+
+
 def _vec(p, C):
+    if p.dtype == torch.float32 and p.dim() == 1 and not p.requires_grad and p.is_contiguous():
+        return p  # (a row of pack_params)
     if p.dtype == torch.float32:
         return p.detach().reshape(C).contiguous()
     return _cached("vec", (p,), lambda: p.detach().reshape(C).float().contiguous())
 
 
 def _coef_matrix(coefs, C):
+    if isinstance(coefs, torch.Tensor):  # (rows of pack_params)
+        return coefs
     return _cached("coefs", tuple(coefs), lambda: torch.stack([_vec(c, C) for c in coefs]).contiguous())
+
+
+def _shift_lerp_fwd(x, shift, coefs):
+    B, T, C = x.shape
+    x = x.contiguous()
+    shift = shift.to(x.dtype).contiguous()
+    cf = _coef_matrix(coefs, C)
+    outs = [torch.empty_like(x) for _ in range(6)]
+    arr = (ctypes.c_void_p * 6)(*[o.data_ptr() for o in outs])
+    with torch.cuda.device(x.device):
+        _check(_lib().theseus_tm_shift_lerp_fwd(B, T, C, _p(x), _p(shift), _p(cf), arr, _s(x.device)))
+    return (x, shift, cf), outs
 
 
 class _ShiftLerp(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, shift, *coefs):
-        B, T, C = x.shape
-        x = x.contiguous()
-        shift = shift.to(x.dtype).contiguous()
-        cf = _coef_matrix(coefs, C)
-        outs = [torch.empty_like(x) for _ in range(6)]
-        arr = (ctypes.c_void_p * 6)(*[o.data_ptr() for o in outs])
-        with torch.cuda.device(x.device):
-            _check(_lib().theseus_tm_shift_lerp_fwd(B, T, C, _p(x), _p(shift), _p(cf), arr, _s(x.device)))
+        (x, shift, cf), outs = _shift_lerp_fwd(x, shift, coefs)
         ctx.save_for_backward(x, shift, cf)
         ctx.coef_meta = [(c.shape, c.dtype) for c in coefs]
         ctx.shift_dtype = shift.dtype
@@ -229,6 +254,9 @@ class _ShiftLerp(torch.autograd.Function):
 
 
 def shift_lerp(x, shift, coefs):
+    """coefs: the six parameters, or (without gradients) their rows of ``pack_params``."""
+    if isinstance(coefs, torch.Tensor) or not _needs_grad(x, shift, *coefs):  # (no autograd node)
+        return tuple(_shift_lerp_fwd(x, shift, coefs)[1])
     return _ShiftLerp.apply(x, shift, *coefs)
 
 
@@ -266,18 +294,22 @@ def _needs_grad(*ts):
     return torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in ts)
 
 
-def _kk_fwd(k, za, a0, k_k, k_a, N, dtype):
+def _kk_fwd(k, za, a0, k_k, k_a, N, dtype, zw=None, w0=None):
     B, T, C = k.shape
     k = k.to(torch.bfloat16).contiguous()
     zs = za.to(torch.bfloat16).contiguous()
     a0v, kk_, ka = _vec(a0, C), _vec(k_k, C), _vec(k_a, C)
     kw, aw, bw = (torch.empty((B, T, C // N, N), dtype=torch.bfloat16, device=k.device) for _ in range(3))
+    args = (B, T, C, _p(k), _p(zs), _p(a0v), _p(kk_), _p(ka), _p(kw), _p(aw), _p(bw))
+    outs = (kw, aw, bw)
     with torch.cuda.device(k.device):
-        _check(_lib().theseus_tm_kk_fwd(B, T, C, _p(k), _p(zs), _p(a0v), _p(kk_), _p(ka), _p(kw), _p(aw),
-                                        _p(bw), _s(k.device)))
-    if dtype != torch.bfloat16:
-        kw, aw, bw = kw.to(dtype), aw.to(dtype), bw.to(dtype)
-    return (k, zs, a0v, kk_, ka), (kw, aw, bw)
+        if zw is None:
+            _check(_lib().theseus_tm_kk_fwd(*args, _s(k.device)))
+        else:
+            zws, w0v, w = zw.to(torch.bfloat16).contiguous(), _vec(w0, C), torch.empty_like(kw)
+            _check(_lib().theseus_tm_kk_w_fwd(*args, _p(zws), _p(w0v), _p(w), _s(k.device)))
+            outs = (w, *outs)
+    return (k, zs, a0v, kk_, ka), tuple(o if dtype == torch.bfloat16 else o.to(dtype) for o in outs)
 
 
 class _KkKmod(torch.autograd.Function):
@@ -323,6 +355,12 @@ def kk_kmod(k, za, a0, k_k, k_a, N, dtype):
         return (*_kk_fwd(k, za, a0, k_k, k_a, N, dtype)[1], _KMod(k, za, a0, k_a, None))
     kw, aw, bw, carrier = _KkKmod.apply(k, za, a0, k_k, k_a, N, dtype)
     return kw, aw, bw, _KMod(k, za, a0, k_a, carrier)
+
+
+def kk_kmod_w(k, za, a0, k_k, k_a, zw, w0, N, dtype):
+    """kk_kmod and add_param(zw, w0) in one launch, without gradients: (w, kw, aw, bw [B,T,H,N],
+    what gn_bonus_gate needs)."""
+    return (*_kk_fwd(k, za, a0, k_k, k_a, N, dtype, zw, w0)[1], _KMod(k, za, a0, k_a, None))
 
 
 class _KMod:

@@ -204,10 +204,20 @@ class TimeMix(nn.Module):
             return self._native_step(x, state, inplace)
         shape = (B, T, self.heads, self.head_size)
         fused_ok = self._fused(x)
+        nograd = False
         if fused_ok:
             from . import fused
-            mixed = dict(zip("rwkvag", fused.shift_lerp(
-                x, state["shift"], [getattr(self, "x_" + n) for n in "rwkvag"])))
+            coefs = [getattr(self, "x_" + n) for n in "rwkvag"]
+            vecs = (self.w0, self.a0, self.k_k, self.k_a, self.r_k, self.ln_x.weight, self.ln_x.bias)
+            nograd = not (torch.is_grad_enabled() and (x.requires_grad or state["shift"].requires_grad
+                                                       or any(p.requires_grad for p in self.parameters())))
+            if nograd and fused._store is None and any(p.dtype != torch.float32 for p in (*coefs, *vecs)):
+                # the kernels' float32 parameters, made for this call in one launch (a serving
+                # loop's store keeps its own copies)
+                packed = fused.pack_params((*coefs, *vecs), self.width)
+                coefs, vecs = packed[:6], packed[6:].unbind(0)
+            w0, a0, k_k, k_a, r_k, ln_w, ln_b = vecs
+            mixed = dict(zip("rwkvag", fused.shift_lerp(x, state["shift"], coefs)))
         else:
             mixed = dict(zip("rwkvag", _shift_lerp_ops(
                 x, state["shift"], [getattr(self, "x_" + n) for n in "rwkvag"])))
@@ -243,16 +253,17 @@ class TimeMix(nn.Module):
             g = torch.sigmoid(mixed["g"] @ self.g1) @ self.g2
         if fused_ok:
             from . import fused
-            w = fused.add_param(zw, self.w0)  # (w0 + zw) in the recurrence's bf16, in one pass
-        else:
-            w = self.w0 + zw
-        if fused_ok:
-            from . import fused
-            # a = sigmoid(a0 + za) (the reference's theseus/timemix.py:75) is formed inside the kernels
-            kw, aw, bw, kmod = fused.kk_kmod(k, za, self.a0, self.k_k, self.k_a, self.head_size, r.dtype)
+            # w = (w0 + zw) in the recurrence's bf16; a = sigmoid(a0 + za) (the reference's
+            # theseus/timemix.py:75) is formed inside the kernels
+            if nograd and not fused._needs_grad(k, za, zw):
+                w, kw, aw, bw, kmod = fused.kk_kmod_w(k, za, a0, k_k, k_a, zw, w0, self.head_size, r.dtype)
+            else:
+                w = fused.add_param(zw, w0)
+                kw, aw, bw, kmod = fused.kk_kmod(k, za, a0, k_k, k_a, self.head_size, r.dtype)
             args = [r.reshape(shape).to(r.dtype).contiguous(), w.reshape(shape).to(r.dtype).contiguous(),
                     kw, v.reshape(shape).to(r.dtype).contiguous(), aw, bw]
         else:
+            w = self.w0 + zw
             a = torch.sigmoid(self.a0 + za)
             kk = F.normalize((k.float() * self.k_k).reshape(shape), dim=-1, eps=1e-12)
             k = k * (1 + (a - 1) * self.k_a)
@@ -265,8 +276,7 @@ class TimeMix(nn.Module):
             y, end = wkv7(*args, state["wkv"], backend=self.backend)
         if fused_ok:
             from . import fused
-            out = fused.gn_bonus_gate(y, r, kmod, v, g, self.r_k, self.ln_x.weight, self.ln_x.bias,
-                                      self.ln_x.eps, x.dtype)
+            out = fused.gn_bonus_gate(y, r, kmod, v, g, r_k, ln_w, ln_b, self.ln_x.eps, x.dtype)
         else:
             # norms in fp32 with autocast off, cast back for the output projection
             with torch.autocast(x.device.type, enabled=False):

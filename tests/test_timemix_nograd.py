@@ -1,0 +1,76 @@
+"""The fused TimeMix pieces of calls without gradients: the parameters in one launch, the decay
+input in the kk kernel's launch, and the token shift at every number of tokens per thread,
+against the separate launches (the same arithmetic, so the same bits) and the torch chain."""
+import pytest
+import torch
+
+from theseus import fused
+from theseus.timemix import TimeMix, _shift_lerp_ops
+
+pytestmark = pytest.mark.gpu
+bf = torch.bfloat16
+
+
+@pytest.mark.parametrize("C", [64, 320, 5120])
+def test_pack_params_is_the_conversions(C):
+    g = torch.Generator(device="cuda").manual_seed(C)
+    ps = [torch.randn(1, 1, C, generator=g, device="cuda").to(d) for d in (bf, torch.float32, torch.float16)]
+    ps += [torch.randn(C // 64, 64, generator=g, device="cuda").to(bf), torch.randn(2 * C, generator=g, device="cuda")[::2]]
+    out = fused.pack_params(ps, C)
+    assert out.shape == (5, C) and out.dtype == torch.float32
+    for row, p in zip(out, ps):
+        assert torch.equal(row, p.float().reshape(C))
+
+
+# below, at and above each line of the dispatch (512 workgroups of 256 threads at 2 and 8
+# tokens per thread), odd token counts, a sequence start inside a thread's tokens
+@pytest.mark.parametrize("B,T,C", [(1, 1, 64), (64, 1, 5120), (3, 5, 128), (2, 255, 5120), (1, 511, 5120),
+                                   (1, 410, 5120), (2, 411, 2560), (3, 683, 5120), (1, 1639, 5120), (7, 235, 5120)])
+def test_shift_lerp_forward_at_every_width(B, T, C):
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(B, T, C, generator=g, device="cuda").to(bf)
+    shift = torch.randn(B, C, generator=g, device="cuda").to(bf)
+    coefs = [torch.rand(1, 1, C, generator=g, device="cuda") for _ in range(6)]
+    with torch.no_grad():
+        got = fused.shift_lerp(x, shift, coefs)
+        rows = fused.shift_lerp(x, shift, fused.pack_params(coefs, C))
+        want = _shift_lerp_ops(x, shift, coefs)
+    for a, b, c in zip(got, rows, want):
+        # (torch rounds product and sum apart, 2^-23 of the mix's terms; the bf16 roundings of the
+        # two are then equal or neighbours, 2^-7 apart)
+        assert torch.equal(a, b)
+        torch.testing.assert_close(a, c, rtol=2 ** -7, atol=1e-5)
+        assert (a != c).float().mean() < 1e-3
+
+
+@pytest.mark.parametrize("B,T,C", [(1, 1, 64), (3, 7, 320), (1, 4096, 128), (5, 821, 192)])
+def test_decay_input_in_the_kk_launch(B, T, C):
+    g = torch.Generator(device="cuda").manual_seed(T)
+    k, za, zw = (torch.randn(B, T, C, generator=g, device="cuda").to(bf) for _ in range(3))
+    a0, kk, ka, w0 = (torch.randn(1, 1, C, generator=g, device="cuda") for _ in range(4))
+    with torch.no_grad():
+        w, *got, _ = fused.kk_kmod_w(k, za, a0, kk, ka, zw, w0, 64, bf)
+        *want, _ = fused.kk_kmod(k, za, a0, kk, ka, 64, bf)
+        assert torch.equal(w.reshape(B, T, C), fused.add_param(zw, w0))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("dtype", [bf, torch.float32])
+def test_layer_without_gradients_equals_the_layer_with(dtype):
+    """The no-grad layer (packed parameters, one kk launch) against the same call with autograd
+    on, which converts each parameter: the same bits."""
+    torch.manual_seed(0)
+    m = TimeMix(256, 2, 6, backend="cuda")
+    with torch.no_grad():
+        for n, p in m.named_parameters():
+            if n in ("w1", "a1", "g1", "output.weight"):
+                p.normal_(0, .05)
+    m = m.cuda().to(dtype)
+    x = torch.randn(2, 100, 256, device="cuda", dtype=bf)
+    with torch.autocast("cuda", dtype=bf):
+        ref, st = m(x)
+        with torch.no_grad():
+            out, st2 = m(x)
+    # (7 chunks: below the time split, which only calls without saved states take)
+    assert torch.equal(out, ref) and not out.requires_grad
+    assert torch.equal(st["wkv"], st2["wkv"])
