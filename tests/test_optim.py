@@ -199,3 +199,28 @@ def test_fused_step_is_deterministic():
         runs.append([p.detach().clone() for p in a.parameters()] + [norm.clone()])
     for x, y in zip(*runs):
         assert torch.equal(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count, size", [(1, 16384 * 3200 + 5), (70, 16384 * 47 + 3), (33, 16385)],
+                         ids=["one-past-the-kept", "three-launches-past-the-kept", "all-kept"])
+def test_update_in_reverse_order_reads_every_chunk_once(count, size):
+    """The norm keeps the last 192 MB of gradients (3072 chunks) cached and the update walks
+    from the last chunk: past that line, with more than one launch, and within it, every
+    element gets exactly one step (the first step moves each parameter by lr * g / (|g| + eps *
+    sqrt(bias)), i.e. by lr to 1e-3 for |g| >= 1e-2 at eps 1e-8) and the norm is the sum over
+    all (sizes not multiples of 4, so the second tensor on is not 16-byte aligned in `flat`)."""
+    from theseus.optim import FusedAdamW
+    g = torch.Generator(device="cuda").manual_seed(count)
+    flat = torch.empty(count * size, device="cuda")
+    flat.uniform_(.5, 1.0, generator=g).mul_(torch.randint(0, 2, flat.shape, device="cuda", generator=g) * 2.0 - 1)
+    ps = [torch.nn.Parameter(torch.zeros(size, device="cuda")) for _ in range(count)]
+    for i, p in enumerate(ps):
+        p.grad = flat[i * size:(i + 1) * size]
+    opt = FusedAdamW(ps, lr=1e-2, weight_decay=0.0)
+    norm = opt.step_after_backward(grad_scale=1.0, max_norm=1e9)
+    torch.testing.assert_close(float(norm), float(flat.double().square().sum().sqrt()), rtol=1e-6, atol=0)
+    for i, p in enumerate(ps):
+        want = -1e-2 * p.grad.sign()
+        assert float((p.detach() - want).abs().max()) < 1e-6, i  # eps/|g| 2e-8 + fp32 rounding of 1e-2
+        torch.testing.assert_close(opt.state[p]["exp_avg"], p.grad * .1, rtol=1e-5, atol=0)
