@@ -254,15 +254,21 @@ __global__ __launch_bounds__(64) void gdn_prep(int Tn, int H, int qk_norm, const
 // (contractions over the keys on the matrix cores), V = v, and e^{gL} per key.  One wave
 // per chunk as gdn_prep, writing the same record layout (GdnRec<NK, true>).  Lane (q4,
 // r16) holds token r16's keys 32ks + 4q4 + e and 32ks + 16 + 4q4 + e; the D-layout tiles
-// of A~, B^ and K^ ([t][j], rows t = 4q4 + e) are read back from LDS planes.
+// of A~, B^, K^ and V ([t][j], rows t = 4q4 + e) are transpose reads of their split bf16
+// rows: A~'s (needed after the inverse) from a plane of all keys, the others' from one
+// buffer of 32 keys, block after block.  With fp32 planes of all four the LDS held 4 waves
+// per CU at 128 keys and 9 at 64 (now 12 and 16): 4 lanes of 2048 tokens and 32 heads of 128, 291 -> 227 us
+// (1.1 GB, 217 us at the rate of a copy); one lane of 1021 tokens and 40 heads of 64,
+// 29.1 -> 24.8 us.
 // ---------------------------------------------------------------------------
 template <int NK>
-__global__ __launch_bounds__(64) void wkv7_rec_prep(int Tn, int H, const bf16_t* __restrict__ r,
+__global__ __launch_bounds__(64, NK == 64 ? 4 : 3) void wkv7_rec_prep(int Tn, int H, const bf16_t* __restrict__ r,
                                                     const bf16_t* __restrict__ w, const bf16_t* __restrict__ k,
                                                     const bf16_t* __restrict__ v, const bf16_t* __restrict__ a,
                                                     const bf16_t* __restrict__ b, uint8_t* __restrict__ ws) {
     using R = GdnRec<NK, true>;
-    constexpr int KS = R::KS, LP = NK + 4;
+    constexpr int KS = R::KS;
+    constexpr int LA = NK + 20, LB = 36;  // rows (bf16) that spread over the banks
     const int c = blockIdx.x, bh = blockIdx.y, nchunk = gridDim.x;
     const int bb = bh / H, h = bh - bb * H;
     const int lane = threadIdx.x, q4 = lane >> 4, r16 = lane & 15;
@@ -271,18 +277,32 @@ __global__ __launch_bounds__(64) void wkv7_rec_prep(int Tn, int H, const bf16_t*
     const bool tv = r16 < L;
     const long row = ((tok0 + (tv ? r16 : 0)) * H + h) * (long)NK;  // token r16's row (clamped: every lane loads)
     const uint32_t tm = lane_mask(tv);
-    // A~, B^, K^ as rows [t][j] for the D-layout reads; v as rows [t][i]
-    __shared__ __attribute__((aligned(16))) float pa[GC][LP], pb[GC][LP], pkh[GC][LP], vsh[GC][LP];
+    __shared__ __attribute__((aligned(16))) uint16_t pa[2][GC][LA], pb[2][GC][LB];  // hi, lo
     uint8_t* const rec = ws + ((size_t)bh * nchunk + c) * R::BYTES;
     f32x4_t Aab = zero4(), AabT = zero4(), Aak = zero4(), BrbT = zero4(), BrkT = zero4();
     float rt[KS][8];  // R~ of the lane's keys, kept for P2
-    auto ld8 = [&](const bf16_t* x, int c0, float (&o)[8]) {
-        const float4 p = keep4(tm, ld4f(x + row + c0)), q = keep4(tm, ld4f(x + row + c0 + 16));
-        o[0] = p.x, o[1] = p.y, o[2] = p.z, o[3] = p.w, o[4] = q.x, o[5] = q.y, o[6] = q.z, o[7] = q.w;
+    // the lane's eight keys of a tensor, packed until they are used
+    auto ld8 = [&](const bf16_t* x, int c0) {
+        const uint2 p = *reinterpret_cast<const uint2*>(x + row + c0), q = *reinterpret_cast<const uint2*>(x + row + c0 + 16);
+        return keepu4(tm, cat(p, q));
     };
-    auto st8 = [&](float (*pl)[LP], int c0, const float (&x)[8]) {
-        *reinterpret_cast<float4*>(&pl[r16][c0]) = make_float4(x[0], x[1], x[2], x[3]);
-        *reinterpret_cast<float4*>(&pl[r16][c0 + 16]) = make_float4(x[4], x[5], x[6], x[7]);
+    auto f8 = [](uint4 x, float (&o)[8]) {
+        const uint32_t u[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[2 * i] = __uint_as_float(u[i] << 16), o[2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
+    };
+    // 32 keys of the token rows into a plane at key k0 (one half of the split pair)
+    auto st8 = [&](uint16_t* pl, int ld, int k0, uint4 x) {
+        uint16_t* const d = pl + r16 * ld + k0 + 4 * q4;
+        *reinterpret_cast<uint2*>(d) = make_uint2(x.x, x.y);
+        *reinterpret_cast<uint2*>(d + 16) = make_uint2(x.z, x.w);
+    };
+    // both 16-key tiles of a 32-key block, transposed, through the small buffer
+    auto turn = [&](uint4 hi, uint4 lo, Pk (&o)[2]) {
+        st8(&pb[0][0][0], LB, 0, hi), st8(&pb[1][0][0], LB, 0, lo);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            o[u].h = ldtr(&pb[0][0][16 * u], LB, lane), o[u].l = ldtr(&pb[1][0][16 * u], LB, lane);
     };
     // split products over one K=32 step: acc += X Y^T (X, Y: the lanes' token rows)
     auto mm3 = [](f32x4_t acc, uint4 xh, uint4 xl, uint4 yh, uint4 yl) {
@@ -291,34 +311,63 @@ __global__ __launch_bounds__(64) void wkv7_rec_prep(int Tn, int H, const bf16_t*
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
         const int c0 = 32 * ks + 4 * q4;
-        float wv[8], av[8], bv[8], kv[8], vv[8];
-        ld8(w, c0, wv), ld8(a, c0, av), ld8(b, c0, bv), ld8(k, c0, kv), ld8(r, c0, rt[ks]), ld8(v, c0, vv);
-        st8(vsh, c0, vv);
-        float At[8], Bm[8], Km[8], Bh[8], Kh[8], eL[8];
+        const uint4 xw = ld8(w, c0), xa = ld8(a, c0), xb = ld8(b, c0), xk = ld8(k, c0), xr = ld8(r, c0), xv = ld8(v, c0);
+        // (one operand after another, each split before the next: all eight at once, as the
+        // compiler would have them, are 183 registers at 128 keys)
+        float x[8], y[8], eA[8], eR[8], em[8], eh[8], eL[8];
+        f8(xw, x);
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-            const float g = row_prefix_sum(tv ? log_decay(wv[e]) : 0.f);  // (0 past the end)
+            const float g = row_prefix_sum(tv ? log_decay(x[e]) : 0.f);  // (0 past the end)
             const float gp = row_prev(g, 0.f), gL = row_last(g);
-            const float em = __expf(-g), eh = __expf(gL - g);
-            At[e] = av[e] * __expf(gp);
-            rt[ks][e] *= __expf(g);
-            Bm[e] = bv[e] * em, Km[e] = kv[e] * em;
-            Bh[e] = bv[e] * eh, Kh[e] = kv[e] * eh;
-            eL[e] = __expf(gL);
+            em[e] = __expf(-g), eh[e] = __expf(gL - g), eA[e] = __expf(gp), eR[e] = __expf(g), eL[e] = __expf(gL);
         }
-        st8(pa, c0, At), st8(pb, c0, Bh), st8(pkh, c0, Kh);
         if (r16 == 0) {
             float* el = reinterpret_cast<float*>(rec + R::EL);
             *reinterpret_cast<float4*>(el + c0) = make_float4(eL[0], eL[1], eL[2], eL[3]);
             *reinterpret_cast<float4*>(el + c0 + 16) = make_float4(eL[4], eL[5], eL[6], eL[7]);
         }
-        uint4 ah, al, bh_, bl, kh, kl, rh, rl;
-        pack8(At, ah, al), pack8(Bm, bh_, bl), pack8(Km, kh, kl), pack8(rt[ks], rh, rl);
+        __builtin_amdgcn_sched_barrier(0);
+        auto scaled = [&](const float (&f)[8], uint4& hi, uint4& lo) {  // the split pair of x o f
+#pragma unroll
+            for (int e = 0; e < 8; e++) y[e] = x[e] * f[e];
+            pack8(y, hi, lo);
+        };
+        uint4 ah, al, bh_, bl, kh, kl, rh, rl, hh, hl;
+        Pk tb[2], tk[2];
+        f8(xa, x), scaled(eA, ah, al);
+        st8(&pa[0][0][0], LA, 32 * ks, ah), st8(&pa[1][0][0], LA, 32 * ks, al);
+        __builtin_amdgcn_sched_barrier(0);
+        f8(xb, x), scaled(em, bh_, bl);
         Aab = mm3(Aab, ah, al, bh_, bl);     // [rr][cc] = A~_rr . B-_cc
         AabT = mm3(AabT, bh_, bl, ah, al);   // B-_rr . A~_cc
+        scaled(eh, hh, hl), turn(hh, hl, tb);
+        __builtin_amdgcn_sched_barrier(0);
+        f8(xk, x), scaled(em, kh, kl);
         Aak = mm3(Aak, ah, al, kh, kl);      // A~_rr . K-_cc
+        scaled(eh, hh, hl), turn(hh, hl, tk);
+        __builtin_amdgcn_sched_barrier(0);
+        f8(xr, x), scaled(eR, rh, rl);
+#pragma unroll
+        for (int e = 0; e < 8; e++) rt[ks][e] = y[e];
         BrbT = mm3(BrbT, bh_, bl, rh, rl);   // B-_rr . R~_cc
         BrkT = mm3(BrkT, kh, kl, rh, rl);    // K-_rr . R~_cc
+        // the update operands B^, K^, and V as the K=16 B operand of each block of 16 value rows
+        // (lane: value 16rb + r16, steps 4q4 + e; zero past the end; exact in bf16)
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            uint8_t* uf = rec + R::UF + (size_t)(2 * (2 * ks + u)) * 1024;
+            put_frag(uf, lane, cat(tb[u].h, tk[u].h));
+            put_frag(uf + 1024, lane, cat(tb[u].l, tk[u].l));
+        }
+        st8(&pb[0][0][0], LB, 0, xv);
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            uint2* vf = reinterpret_cast<uint2*>(rec + R::VF) + (size_t)(2 * (2 * ks + u)) * 64 + lane;
+            vf[0] = ldtr(&pb[0][0][16 * u], LB, lane);
+            vf[64] = make_uint2(0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
     }
     // the chunk matrices in D layout (element [rr][cc], rr = 4q4 + e, cc = r16), masked
     const int cc = r16;
@@ -341,44 +390,22 @@ __global__ __launch_bounds__(64) void wkv7_rec_prep(int Tn, int H, const bf16_t*
         uint2* qf = reinterpret_cast<uint2*>(rec + R::QF) + lane;
         qf[0] = pQ1T.h, qf[64] = pQ1T.l, qf[128] = pQ2T.h, qf[192] = pQ2T.l;
     }
-    __syncthreads();  // the planes
-    // V as the K=16 B operand of each block of 16 value rows (lane: value 16rb + r16,
-    // steps 4q4 + e; zero past the end), split
-#pragma unroll
-    for (int rb = 0; rb < R::TJ; rb++) {
-        f32x4_t vq;
-#pragma unroll
-        for (int e = 0; e < 4; e++) vq[e] = vsh[4 * q4 + e][16 * rb + r16];
-        const Pk pv = pk(vq);
-        uint2* vf = reinterpret_cast<uint2*>(rec + R::VF) + (size_t)(2 * rb) * 64 + lane;
-        vf[0] = pv.h;
-        vf[64] = pv.l;
-    }
-    // per pair of 16-key tiles (one K-step): P, P2 and the update operands
+    __syncthreads();  // A~
+    // per pair of 16-key tiles (one K-step): P and P2
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
         Pk pPT[2], pP2T[2];
 #pragma unroll
         for (int u = 0; u < 2; u++) {
             const int tj = 2 * ks + u;
-            f32x4_t at, bhat, khat;  // D layout [t][j], t = 4q4 + e, j = 16tj + r16
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                at[e] = pa[4 * q4 + e][16 * tj + r16];
-                bhat[e] = pb[4 * q4 + e][16 * tj + r16];
-                khat[e] = pkh[4 * q4 + e][16 * tj + r16];
-            }
-            const Pk pA = pk(at);
+            // D layout [t][j], t = 4q4 + e, j = 16tj + r16
+            const Pk pA{ldtr(&pa[0][0][16 * tj], LA, lane), ldtr(&pa[1][0][16 * tj], LA, lane)};
             const f32x4_t Pt = mm16s(pTiT, pA);   // P tile [t][j]
             pPT[u] = pk(mm16s(pA, pTiT));          // P^T tile [j][t]
             f32x4_t rr4;                            // R~[t = r16][16tj + 4q4 + e]
 #pragma unroll
             for (int e = 0; e < 4; e++) rr4[e] = rt[ks][4 * u + e];
             pP2T[u] = pk(rr4 + mm16s(pk(Pt), pBrbT));  // P2^T = R~^T + P^T Brb^T
-            const Pk pb4 = pk(bhat), pk4 = pk(khat);
-            uint8_t* uf = rec + R::UF + (size_t)(2 * tj) * 1024;
-            put_frag(uf, lane, cat(pb4.h, pk4.h));
-            put_frag(uf + 1024, lane, cat(pb4.l, pk4.l));
         }
         uint8_t* pf = rec + R::PF + (size_t)(2 * ks) * 1024;
         put_frag(pf, lane, cat(pPT[0].h, pPT[1].h));
