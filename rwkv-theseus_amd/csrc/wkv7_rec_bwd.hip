@@ -25,7 +25,8 @@
 // double-buffered in LDS by DMA as gdn_scan's), storing H at every chunk's end in the
 // workspace and the first chunk's start as ds0.  wkv7_bwd_chunk then forms every
 // chunk's gradients independently (eight waves; wave w owns value rows 16w..16w+15 for
-// SA, Q, dV and keys 16w..16w+15 for dK, dB, dR, dA, dw).
+// SA, Q, dV and keys 16w..16w+15 for dK, dB, dR, dA, dw), with the chunk's matrices from
+// wkv7_bwd_prep.
 #include "wkv7_launch.h"
 #include "wkv7_scan.h"
 
@@ -61,17 +62,23 @@ __device__ __forceinline__ f32x4_t transpose16(const f32x4_t& m, int lane) {
 }
 __device__ __forceinline__ float bf2f(const bf16_t* p, long i) { return io<bf16_t>::ld(p, i); }
 
+// The chunk's 16x16 matrices for wkv7_bwd_chunk, packed split pairs (uint4 per lane).
+enum { MAT_AAKT, MAT_AAK, MAT_BRB, MAT_BRK, MAT_TI, MAT_TIT, MATS };
+
 // ---------------------------------------------------------------------------
 // Records of chunk blockIdx.x of head blockIdx.y (one wave; lane (q4, r16): token r16's
-// keys 32ks + 4q4 + e and 32ks + 16 + 4q4 + e, as wkv7_rec_prep).
+// keys 32ks + 4q4 + e and 32ks + 16 + 4q4 + e, planes and order as wkv7_rec_prep).  Bound by
+// its bytes (4 lanes of 2048 tokens, 32 heads of 128: 850 MB, 167 us at the rate of a copy;
+// measured 185).
 // ---------------------------------------------------------------------------
 template <int NK>
-__global__ __launch_bounds__(64) void wkv7_bwd_prep(int Tn, int H, const bf16_t* __restrict__ r,
+__global__ __launch_bounds__(64, NK == 64 ? 4 : 3) void wkv7_bwd_prep(int Tn, int H, const bf16_t* __restrict__ r,
                                                     const bf16_t* __restrict__ w, const bf16_t* __restrict__ k,
                                                     const bf16_t* __restrict__ a, const bf16_t* __restrict__ b,
-                                                    uint8_t* __restrict__ ws) {
+                                                    uint8_t* __restrict__ ws, uint4* __restrict__ mats) {
     using R = BwdRec<NK>;
-    constexpr int KS = R::KS, TJ = R::TJ, LP = NK + 4;
+    constexpr int KS = R::KS;
+    constexpr int LA = NK + 20, LB = 36;  // rows (bf16) that spread over the banks
     const int c = blockIdx.x, bh = blockIdx.y, nchunk = gridDim.x;
     const int bb = bh / H, h = bh - bb * H;
     const int lane = threadIdx.x, q4 = lane >> 4, r16 = lane & 15;
@@ -79,47 +86,70 @@ __global__ __launch_bounds__(64) void wkv7_bwd_prep(int Tn, int H, const bf16_t*
     const bool tv = r16 < L;
     const long row = (((long)bb * Tn + t0 + (tv ? r16 : 0)) * H + h) * (long)NK;  // (clamped: read by every lane)
     const uint32_t tm = lane_mask(tv);
-    __shared__ __attribute__((aligned(16))) float pa[BC][LP], pr[BC][LP];  // A~, R~ [t][j]
+    __shared__ __attribute__((aligned(16))) uint16_t pa[2][BC][LA], pb[2][BC][LB];  // hi, lo
     uint8_t* const rec = ws + ((size_t)bh * nchunk + c) * R::BYTES;
-    auto ld8 = [&](const bf16_t* x, int c0, float (&o)[8]) {
-        const float4 p = keep4(tm, ld4f(x + row + c0)), q = keep4(tm, ld4f(x + row + c0 + 16));
-        o[0] = p.x, o[1] = p.y, o[2] = p.z, o[3] = p.w, o[4] = q.x, o[5] = q.y, o[6] = q.z, o[7] = q.w;
+    auto ld8 = [&](const bf16_t* x, int c0) {
+        const uint2 p = *reinterpret_cast<const uint2*>(x + row + c0), q = *reinterpret_cast<const uint2*>(x + row + c0 + 16);
+        return keepu4(tm, cat(p, q));
     };
-    auto st8 = [&](float (*pl)[LP], int c0, const float (&x)[8]) {
-        *reinterpret_cast<float4*>(&pl[r16][c0]) = make_float4(x[0], x[1], x[2], x[3]);
-        *reinterpret_cast<float4*>(&pl[r16][c0 + 16]) = make_float4(x[4], x[5], x[6], x[7]);
+    auto f8 = [](uint4 x, float (&o)[8]) {
+        const uint32_t u[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[2 * i] = __uint_as_float(u[i] << 16), o[2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
     };
-    f32x4_t Aab = zero4(), AabT = zero4(), BrbT = zero4();
+    auto st8 = [&](uint16_t* pl, int ld, int k0, uint4 x) {
+        uint16_t* const d = pl + r16 * ld + k0 + 4 * q4;
+        *reinterpret_cast<uint2*>(d) = make_uint2(x.x, x.y);
+        *reinterpret_cast<uint2*>(d + 16) = make_uint2(x.z, x.w);
+    };
+    f32x4_t Aab = zero4(), AabT = zero4(), BrbT = zero4(), Aak = zero4(), Brb = zero4(), Brk = zero4();
+    float rt[KS][8];  // R~ of the lane's keys, kept for P2
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
         const int c0 = 32 * ks + 4 * q4;
-        float wv[8], av[8], bv[8], rv[8];
-        ld8(w, c0, wv), ld8(a, c0, av), ld8(b, c0, bv), ld8(r, c0, rv);
-        float At[8], Bm[8], Rt[8], Bh[8], eL[8];
+        const uint4 xw = ld8(w, c0), xa = ld8(a, c0), xb = ld8(b, c0), xk = ld8(k, c0), xr = ld8(r, c0);
+        // (one operand after another, as wkv7_rec_prep)
+        float x[8], y[8], eA[8], eR[8], em[8], eh[8], eL[8];
+        f8(xw, x);
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-            const float g = row_prefix_sum(tv ? log_decay(wv[e]) : 0.f);
+            const float g = row_prefix_sum(tv ? log_decay(x[e]) : 0.f);
             const float gp = row_prev(g, 0.f), gL = row_last(g);
-            At[e] = av[e] * __expf(gp);
-            Rt[e] = rv[e] * __expf(g);
-            Bm[e] = bv[e] * __expf(-g);
-            Bh[e] = bv[e] * __expf(gL - g);
-            eL[e] = __expf(gL);
+            em[e] = __expf(-g), eh[e] = __expf(gL - g), eA[e] = __expf(gp), eR[e] = __expf(g), eL[e] = __expf(gL);
         }
-        st8(pa, c0, At), st8(pr, c0, Rt);
         if (r16 == 0) {
             float* el = reinterpret_cast<float*>(rec + R::EL);
             *reinterpret_cast<float4*>(el + c0) = make_float4(eL[0], eL[1], eL[2], eL[3]);
             *reinterpret_cast<float4*>(el + c0 + 16) = make_float4(eL[4], eL[5], eL[6], eL[7]);
         }
-        uint4 ah, al, bh_, bl, rh, rl, hh, hl;
-        pack8(At, ah, al), pack8(Bm, bh_, bl), pack8(Rt, rh, rl), pack8(Bh, hh, hl);
+        __builtin_amdgcn_sched_barrier(0);
+        auto scaled = [&](const float (&f)[8], uint4& hi, uint4& lo) {  // the split pair of x o f
+#pragma unroll
+            for (int e = 0; e < 8; e++) y[e] = x[e] * f[e];
+            pack8(y, hi, lo);
+        };
+        uint4 ah, al, bh_, bl, rh, rl, hh, hl, kh, kl;
+        f8(xa, x), scaled(eA, ah, al);
+        st8(&pa[0][0][0], LA, 32 * ks, ah), st8(&pa[1][0][0], LA, 32 * ks, al);
+        __builtin_amdgcn_sched_barrier(0);
+        f8(xb, x), scaled(eh, hh, hl);
         uint8_t* bf = rec + R::BF + (size_t)(2 * ks) * 1024;
         put_frag(bf, lane, hh);
         put_frag(bf + 1024, lane, hl);
+        scaled(em, bh_, bl);
         Aab = mm3(Aab, ah, al, bh_, bl);    // A~_rr . B-_cc
         AabT = mm3(AabT, bh_, bl, ah, al);  // B-_rr . A~_cc
+        __builtin_amdgcn_sched_barrier(0);
+        f8(xk, x), scaled(em, kh, kl);
+        Aak = mm3(Aak, ah, al, kh, kl);
+        __builtin_amdgcn_sched_barrier(0);
+        f8(xr, x), scaled(eR, rh, rl);
+#pragma unroll
+        for (int e = 0; e < 8; e++) rt[ks][e] = y[e];
         BrbT = mm3(BrbT, bh_, bl, rh, rl);  // B-_rr . R~_cc
+        Brb = mm3(Brb, rh, rl, bh_, bl);
+        Brk = mm3(Brk, rh, rl, kh, kl);
+        __builtin_amdgcn_sched_barrier(0);
     }
     const int cc = r16;
 #pragma unroll
@@ -128,22 +158,41 @@ __global__ __launch_bounds__(64) void wkv7_bwd_prep(int Tn, int H, const bf16_t*
         Aab[e] = cc < rr ? Aab[e] : 0.f;
         AabT[e] = rr < cc ? AabT[e] : 0.f;
         BrbT[e] = rr <= cc ? BrbT[e] : 0.f;  // Brb[cc][rr]
+        Aak[e] = cc < rr ? Aak[e] : 0.f;
+        Brb[e] = cc <= rr ? Brb[e] : 0.f;
+        Brk[e] = cc <= rr ? Brk[e] : 0.f;
     }
+    uint4* const mt = mats + ((size_t)bh * nchunk + c) * (MATS * 64) + lane;
+    auto put_mat = [&](int i, const Pk& m) { mt[64 * i] = cat(m.h, m.l); };
+    put_mat(MAT_AAKT, pk(transpose16(Aak, lane))), put_mat(MAT_AAK, pk(Aak));
+    put_mat(MAT_BRB, pk(Brb)), put_mat(MAT_BRK, pk(Brk));
     f32x4_t Ti, TiT;
     tri_inverse(Aab, AabT, lane, Ti, TiT);
     const Pk pTiT = pk(TiT), pBrbT = pk(BrbT);
-    __syncthreads();  // the planes
+    put_mat(MAT_TI, pk(Ti)), put_mat(MAT_TIT, pTiT);
+    __syncthreads();  // A~
 #pragma unroll
-    for (int tj = 0; tj < TJ; tj++) {
-        f32x4_t at, rt;  // D layout [t][j], t = 4q4 + e, j = 16tj + r16
+    for (int ks = 0; ks < KS; ks++) {
+        Pk pP[2], p2[2];
 #pragma unroll
-        for (int e = 0; e < 4; e++) at[e] = pa[4 * q4 + e][16 * tj + r16], rt[e] = pr[4 * q4 + e][16 * tj + r16];
-        const f32x4_t Pt = mm16s(pTiT, pk(at));          // P = Ti A~
-        const Pk pP = pk(Pt);
-        const Pk pP2 = pk(rt + mm16s(pBrbT, pP));        // P2 = R~ + Brb P
-        uint8_t* pp = rec + R::PP + (size_t)(2 * tj) * 1024;
-        put_frag(pp, lane, cat(pP.h, pP2.h));
-        put_frag(pp + 1024, lane, cat(pP.l, pP2.l));
+        for (int u = 0; u < 2; u++) {
+            const int tj = 2 * ks + u;
+            // D layout [t][j], t = 4q4 + e, j = 16tj + r16
+            const Pk pA{ldtr(&pa[0][0][16 * tj], LA, lane), ldtr(&pa[1][0][16 * tj], LA, lane)};
+            pP[u] = pk(mm16s(pTiT, pA));           // P = Ti A~
+            f32x4_t rr4;                            // R~[t = r16][16tj + 4q4 + e]
+#pragma unroll
+            for (int e = 0; e < 4; e++) rr4[e] = rt[ks][4 * u + e];
+            p2[u] = pk(rr4 + mm16s(pP[u], pBrbT));  // P2^T = R~^T + P^T Brb^T
+        }
+        // P2's tiles as P's lie, by transpose reads
+        st8(&pb[0][0][0], LB, 0, cat(p2[0].h, p2[1].h)), st8(&pb[1][0][0], LB, 0, cat(p2[0].l, p2[1].l));
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            uint8_t* pp = rec + R::PP + (size_t)(2 * (2 * ks + u)) * 1024;
+            put_frag(pp, lane, cat(pP[u].h, ldtr(&pb[0][0][16 * u], LB, lane)));
+            put_frag(pp + 1024, lane, cat(pP[u].l, ldtr(&pb[1][0][16 * u], LB, lane)));
+        }
     }
 }
 
@@ -339,26 +388,64 @@ __device__ __forceinline__ uint4 bf16_frag(const bf16_t* row, int ks, int q4, bo
     const uint2 b = *reinterpret_cast<const uint2*>(row + 32 * ks + 16 + 4 * q4);
     return keepu4(lane_mask(ok), make_uint4(a.x, a.y, b.x, b.y));
 }
+// One half (hi or lo) of H_end or S0, [value row][key] without padding: each wave puts the 16
+// value rows that it loaded and split and takes its 16 keys over all value rows with transpose
+// reads.  8-byte piece c of row p lies at c ^ swz_state(p): the writes down 16 rows (16 lanes
+// per cycle over 32 banks) and the transpose reads (32 lanes over 64 banks) meet no conflict at
+// 128 keys.
+template <int NK> __device__ __forceinline__ int state_at(int row, int col) {  // col a multiple of 4
+    const int sw = NK == 64 ? swz<SwLane>(row) : 4 * (row & 7) + 2 * ((row >> 3) & 1) + ((row >> 2) & 1);
+    return row * NK + (((col >> 2) ^ sw) << 2);
+}
+// row `row`'s keys as the K=32 operand holds them (slots 32ks + 4q4 + e, +16)
+template <int NK> __device__ __forceinline__ void put_state(uint16_t* x, uint4 v, int row, int ks, int q4) {
+    *reinterpret_cast<uint2*>(x + state_at<NK>(row, 32 * ks + 4 * q4)) = make_uint2(v.x, v.y);
+    *reinterpret_cast<uint2*>(x + state_at<NK>(row, 32 * ks + 16 + 4 * q4)) = make_uint2(v.z, v.w);
+}
+// the K=32 operand of key 16 wv + r16 over the value rows (the same slots)
+template <int NK> __device__ __forceinline__ uint4 get_state(const uint16_t* x, int ks, int wv, int lane) {
+    const int row = 32 * ks + 4 * (lane >> 4) + ((lane & 15) >> 2), c = 16 * wv + 4 * (lane & 3);
+    return cat(tr_at(x + state_at<NK>(row, c)), tr_at(x + state_at<NK>(row + 16, c)));
+}
 template <int NK> struct ChunkLds {
-    SplitPlane<NK> At, Bm, Km, Rt, Bh, Kh;  // [t][j], written by the key owners
-    SplitPlane<NK> SA, Q;                   // [t][i], written by the value-row owners
-    float csum[NK / 16][NK];  // per wave: column sums of H_end o S_end over its 16 value rows
+    union {
+        struct {
+            SplitPlane<NK> At, Bh, Kh;  // [t][j], written by the key owners
+        };
+        uint16_t st[NK * NK];  // (then) the states, one half after another
+    };
+    SplitPlane<NK> SA, Q;              // [t][i], written by the value-row owners
+    uint16_t V[BC][NK + 8], dY[BC][NK + 8];  // as given (exact in bf16)
+    float csum[NK / 16][NK];           // per wave: column sums of H_end o S_end over its 16 value rows
+    uint4 M[8][64];                    // the masked Gram matrices, packed
 };
 
+// What bounds it: H_end, S_end and S0 (64 KB each at 128 keys, S_end mostly from L2) and the
+// registers that hide their latency.  Measured at 4 lanes of 2048 tokens and 32 heads of 128
+// (rocprofv3; 3.4 GB through HBM, 670 us at the rate of a copy), in this order: 1206 us when each
+// wave formed all the chunk's matrices and Gram matrices itself and loaded its key columns
+// from memory (232 registers, one workgroup per CU); 1080 with the matrices from
+// wkv7_bwd_prep, the Gram matrices shared out and the key operands formed twice instead of
+// held (116 registers, two workgroups per CU; the prep kernel 151 -> 183 us); 908 with the
+// states turned through LDS, one half of the split pair after another (all four halves at
+// once, 128 KB and one workgroup per CU, had been 1320 us).  The column sums from key columns
+// of S_end instead of its rows spill (1466 us).  At 64 keys, one lane of 1021 tokens and 40
+// heads: 58 -> 49 us.
 //
 // Saved states: [value][key] at NK = 128; at NK = 64 in the chunked kernels' tiled order
 // (but for the last, final one).
 template <int NK>
-__global__ __launch_bounds__(4 * NK) void wkv7_bwd_chunk(int Tn, int H, int BH, int per_xcd,
+__global__ __launch_bounds__(4 * NK, 4) void wkv7_bwd_chunk(int Tn, int H, int BH, int per_xcd,
                                                       const bf16_t* __restrict__ r, const bf16_t* __restrict__ w,
                                                       const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
                                                       const bf16_t* __restrict__ a, const bf16_t* __restrict__ b,
                                                       const bf16_t* __restrict__ dy, const float* __restrict__ ckpt,
-                                                      const float* __restrict__ hbuf, bf16_t* __restrict__ dr,
+                                                      const float* __restrict__ hbuf, const uint4* __restrict__ mats,
+                                                      bf16_t* __restrict__ dr,
                                                       bf16_t* __restrict__ dw, bf16_t* __restrict__ dk,
                                                       bf16_t* __restrict__ dv, bf16_t* __restrict__ da,
                                                       bf16_t* __restrict__ db) {
-    constexpr int KS = NK / 32, TJ = NK / 16;
+    constexpr int KS = NK / 32, TJ = NK / 16, CLB = NK + 8;
     constexpr long NN = (long)NK * NK;
     constexpr bool TILED = NK == 64;
     __shared__ __attribute__((aligned(16))) ChunkLds<NK> sm;
@@ -376,6 +463,7 @@ __global__ __launch_bounds__(4 * NK) void wkv7_bwd_chunk(int Tn, int H, int BH, 
     const float* const S0 = ckpt + ((long)bh * ncp + c) * NN;
     const float* const Se = S0 + NN;
     const float* const Hm = hbuf + ((long)bh * nchunk + c) * NN;
+    const uint4* const mt = mats + (size_t)job * (MATS * 64) + lane;
     const int irow = 16 * wv + r16;  // value row of the row-strip loads
 
     // ---- the wave's value rows of H_end, S_end and S0 (keys 32ks + 4q4 + e, +16) ----
@@ -393,36 +481,55 @@ __global__ __launch_bounds__(4 * NK) void wkv7_bwd_chunk(int Tn, int H, int BH, 
     };
     rows(Hm, false, hr);
     rows(Se, c + 1 < nchunk, sr);
+    {  // V and dY: eight bytes per thread, rows past the chunk's end zero
+        const int t = tid / (NK / 4), cv = 4 * (tid % (NK / 4));
+        const uint32_t m = lane_mask(t < L);
+        const long o = at_tok(t < L ? t : 0) + cv;
+        const uint2 x = *reinterpret_cast<const uint2*>(v + o), y = *reinterpret_cast<const uint2*>(dy + o);
+        *reinterpret_cast<uint2*>(&sm.V[t][cv]) = make_uint2(x.x & m, x.y & m);
+        *reinterpret_cast<uint2*>(&sm.dY[t][cv]) = make_uint2(y.x & m, y.y & m);
+    }
 
     // ---- the chunk operands of the wave's keys in D layout ([t][col], t = 4q4 + e) ----
-    float xr[4], xw[4], xk[4], xa[4], xb[4];
+    // (formed here for the planes and again for the gradients: kept, they and the decays would
+    // be 48 registers through the products between)
+    float xr[4], xw[4], xk[4], xa[4], xb[4], eLj;
+    f32x4_t eA, eR, eM;
+    auto keys = [&]() {
+        int q = q4;
+        asm volatile("" : "+v"(q));  // (opaque: the second call is not merged with the first)
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const int t = 4 * q4 + e;
-        const bool ok = t < L;
-        const long o = at_tok(ok ? t : 0) + col;  // (clamped: every lane loads)
-        const float r_ = bf2f(r, o), w_ = bf2f(w, o), k_ = bf2f(k, o), a_ = bf2f(a, o), b_ = bf2f(b, o);
-        const uint32_t m = lane_mask(ok);
-        xr[e] = keep(m, r_), xw[e] = keep(m, w_), xk[e] = keep(m, k_), xa[e] = keep(m, a_), xb[e] = keep(m, b_);
+        for (int e = 0; e < 4; e++) {
+            const int t = 4 * q + e;
+            const bool ok = t < L;
+            const long o = at_tok(ok ? t : 0) + col;  // (clamped: every lane loads)
+            const float r_ = bf2f(r, o), w_ = bf2f(w, o), k_ = bf2f(k, o), a_ = bf2f(a, o), b_ = bf2f(b, o);
+            const uint32_t m = lane_mask(ok);
+            xr[e] = keep(m, r_), xw[e] = keep(m, w_), xk[e] = keep(m, k_), xa[e] = keep(m, a_), xb[e] = keep(m, b_);
+        }
+        float ld[4], p[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) ld[e] = (4 * q + e) < L ? log_decay(xw[e]) : 0.f;
+        p[0] = ld[0], p[1] = p[0] + ld[1], p[2] = p[1] + ld[2], p[3] = p[2] + ld[3];
+        // cumulative over the four lane groups (tokens 4q'..4q'+3 of the same key)
+        const float T0 = __shfl(p[3], r16), T1 = __shfl(p[3], 16 + r16), T2 = __shfl(p[3], 32 + r16),
+                    T3 = __shfl(p[3], 48 + r16);
+        const float excl = (q > 0 ? T0 : 0.f) + (q > 1 ? T1 : 0.f) + (q > 2 ? T2 : 0.f);
+        eLj = __expf(T0 + T1 + T2 + T3);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float g = excl + p[e], gp = e ? excl + p[e - 1] : excl;
+            eA[e] = __expf(gp), eR[e] = __expf(g), eM[e] = __expf(-g);
+        }
+    };
+    keys();
+    {
+        f32x4_t At, Bh, Kh;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            At[e] = xa[e] * eA[e], Bh[e] = xb[e] * eM[e] * eLj, Kh[e] = xk[e] * eM[e] * eLj;
+        put_split(sm.At, At, lane, wv), put_split(sm.Bh, Bh, lane, wv), put_split(sm.Kh, Kh, lane, wv);
     }
-    float ld[4], p[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) ld[e] = (4 * q4 + e) < L ? log_decay(xw[e]) : 0.f;
-    p[0] = ld[0], p[1] = p[0] + ld[1], p[2] = p[1] + ld[2], p[3] = p[2] + ld[3];
-    // cumulative over the four lane groups (tokens 4q'..4q'+3 of the same key)
-    const float T0 = __shfl(p[3], r16), T1 = __shfl(p[3], 16 + r16), T2 = __shfl(p[3], 32 + r16),
-                T3 = __shfl(p[3], 48 + r16);
-    const float excl = (q4 > 0 ? T0 : 0.f) + (q4 > 1 ? T1 : 0.f) + (q4 > 2 ? T2 : 0.f);
-    const float eLj = __expf(T0 + T1 + T2 + T3);
-    f32x4_t At, Rt, Bm, Km, eA, eR, eM;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const float g = excl + p[e], gp = e ? excl + p[e - 1] : excl;
-        eA[e] = __expf(gp), eR[e] = __expf(g), eM[e] = __expf(-g);
-        At[e] = xa[e] * eA[e], Rt[e] = xr[e] * eR[e], Bm[e] = xb[e] * eM[e], Km[e] = xk[e] * eM[e];
-    }
-    put_split(sm.At, At, lane, wv), put_split(sm.Bm, Bm, lane, wv), put_split(sm.Km, Km, lane, wv);
-    put_split(sm.Rt, Rt, lane, wv), put_split(sm.Bh, Bm * eLj, lane, wv), put_split(sm.Kh, Km * eLj, lane, wv);
     // the carry's partial column sums over this wave's value rows
 #pragma unroll
     for (int ks = 0; ks < KS; ks++)
@@ -439,113 +546,108 @@ __global__ __launch_bounds__(4 * NK) void wkv7_bwd_chunk(int Tn, int H, int BH, 
     for (int ks = 0; ks < KS; ks++) pack8(sr[ks], Sh[ks], Sl[ks]);
     __syncthreads();
 
-    // ---- chunk matrices (every wave) and the wave's [t][i] products over the keys ----
-    f32x4_t Aab = zero4(), AabT = zero4(), Aak = zero4(), Brb = zero4(), Brk = zero4();
+    // ---- the wave's [t][i] products over the keys ----
     f32x4_t P1 = zero4(), P2 = zero4(), P3 = zero4();
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-        uint4 ah, al, bh_, bl, kh, kl, rh, rl, hh, hl, xh, xl;
-        get_split(sm.At, lane, ks, ah, al), get_split(sm.Bm, lane, ks, bh_, bl);
-        get_split(sm.Km, lane, ks, kh, kl), get_split(sm.Rt, lane, ks, rh, rl);
-        get_split(sm.Bh, lane, ks, hh, hl), get_split(sm.Kh, lane, ks, xh, xl);
-        Aab = mm3(Aab, ah, al, bh_, bl);
-        AabT = mm3(AabT, bh_, bl, ah, al);
-        Aak = mm3(Aak, ah, al, kh, kl);
-        Brb = mm3(Brb, rh, rl, bh_, bl);   // R~_rr . B-_cc
-        Brk = mm3(Brk, rh, rl, kh, kl);    // R~_rr . K-_cc
+        uint4 ah, al, hh, hl, xh, xl;
+        get_split(sm.At, lane, ks, ah, al), get_split(sm.Bh, lane, ks, hh, hl), get_split(sm.Kh, lane, ks, xh, xl);
         P1 = mm3(P1, ah, al, Sh[ks], Sl[ks]);  // A~ S0^T
         P2 = mm3(P2, hh, hl, Hh[ks], Hl[ks]);  // B^ H^T
         P3 = mm3(P3, xh, xl, Hh[ks], Hl[ks]);  // K^ H^T
     }
-    const int cc = r16;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const int rr = 4 * q4 + e;
-        Aab[e] = cc < rr ? Aab[e] : 0.f;
-        AabT[e] = rr < cc ? AabT[e] : 0.f;
-        Aak[e] = cc < rr ? Aak[e] : 0.f;
-        Brb[e] = cc <= rr ? Brb[e] : 0.f;
-        Brk[e] = cc <= rr ? Brk[e] : 0.f;
-    }
-    f32x4_t Ti, TiT;
-    tri_inverse(Aab, AabT, lane, Ti, TiT);
-    const Pk pAak = pk(Aak), pBrb = pk(Brb), pBrk = pk(Brk), pTi = pk(Ti), pTiT = pk(TiT);
-    const Pk pAakT = pk(transpose16(Aak, lane));
-
     // ---- SA, Q, dV for the wave's value columns ----
-    f32x4_t vD, dyD;  // [t][col]
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const int t = 4 * q4 + e;
-        const long o = at_tok(t < L ? t : 0) + col;
-        const float v_ = bf2f(v, o), y_ = bf2f(dy, o);
-        vD[e] = keep(lane_mask(t < L), v_);
-        dyD[e] = keep(lane_mask(t < L), y_);
-    }
-    const Pk pV = pk(vD), pdY = pk(dyD);
-    const f32x4_t SA = mm16s(pTiT, pk(P1 + mm16s(pAakT, pV)));  // Ti (A~ S0^T + Aak V)
-    const f32x4_t Q = mm16s(pTi, pk(P2 + mm16s(pBrb, pdY)));    // Ti^T (B^ H^T + Brb^T dY)
-    const f32x4_t dV = P3 + mm16s(pAak, pk(Q)) + mm16s(pBrk, pdY);
+    auto mat = [&](int i) {
+        const uint4 m = mt[64 * i];
+        return Pk{make_uint2(m.x, m.y), make_uint2(m.z, m.w)};
+    };
+    auto mx = [&](const Pk& A, uint2 B) { return mma16(mma16(zero4(), A.h, B), A.l, B); };  // (B exact)
+    const uint2 hV = ldtr(&sm.V[0][16 * wv], CLB, lane), hY = ldtr(&sm.dY[0][16 * wv], CLB, lane);
+    const f32x4_t SA = mm16s(mat(MAT_TIT), pk(P1 + mx(mat(MAT_AAKT), hV)));  // Ti (A~ S0^T + Aak V)
+    const f32x4_t Q = mm16s(mat(MAT_TI), pk(P2 + mx(mat(MAT_BRB), hY)));     // Ti^T (B^ H^T + Brb^T dY)
+    const f32x4_t dV = P3 + mm16s(mat(MAT_AAK), pk(Q)) + mx(mat(MAT_BRK), hY);
     put_split(sm.SA, SA, lane, wv), put_split(sm.Q, Q, lane, wv);
     {
         const int tr = 4 * q4 + (lane & 3);  // the row quad_rows_bf16 gives this lane
         const uint2 q = quad_rows_bf16(dV, lane);  // (cross-lane: every lane takes part)
         if (tr < L) *reinterpret_cast<uint2*>(dv + at_tok(tr) + 16 * wv + 4 * ((lane >> 2) & 3)) = q;
     }
-    // the key columns of H_end and S0 (value rows 32ks + 4q4 + e, +16) for the products over
-    // the value rows
+    // ---- the products over the value rows ----
+    f32x4_t VH = zero4(), SAH = zero4(), dYS = zero4(), QS = zero4();
+    auto turn = [&](const uint4 (&x)[KS]) {
+        __syncthreads();  // (the key planes or the half before are read)
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++)
+        for (int ks = 0; ks < KS; ks++) put_state<NK>(sm.st, x[ks], irow, ks, q4);
+        __syncthreads();  // (the first also: SA, Q, csum)
+    };
+    // acc += X m, acc2 += Y m with X exact in bf16 and Y = (h, l) (`low`: m is a lo half)
+    auto over_rows = [&](const uint16_t* X, const SplitPlane<NK>& Y, bool low, f32x4_t& acc, f32x4_t& acc2) {
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int i = 32 * ks + (e < 4 ? 4 * q4 + e : 16 + 4 * q4 + e - 4);
-            hr[ks][e] = Hm[(long)i * NK + col];
-            sr[ks][e] = S0[TILED ? ((i / 16 * TJ + wv) * 64 + 16 * (r16 / 4) + i % 16) * 4 + r16 % 4 : (long)i * NK + col];
+        for (int ks = 0; ks < KS; ks++) {
+            const uint4 m = get_state<NK>(sm.st, ks, wv, lane);
+            acc = mma32(acc, fragp(X, CLB, r16, 32 * ks, lane), m);
+            acc2 = mma32(acc2, fragp(&Y.h[0][0], CLB, r16, 32 * ks, lane), m);
+            if (!low) acc2 = mma32(acc2, fragp(&Y.l[0][0], CLB, r16, 32 * ks, lane), m);
         }
+    };
+    turn(Hh), over_rows(&sm.V[0][0], sm.SA, false, VH, SAH);
+    turn(Hl), over_rows(&sm.V[0][0], sm.SA, true, VH, SAH);
+    turn(Sh), over_rows(&sm.dY[0][0], sm.Q, false, dYS, QS);
+    turn(Sl), over_rows(&sm.dY[0][0], sm.Q, true, dYS, QS);
+
+    // ---- the intra-chunk matrices' masked transposes M1..M8, shared out over the waves:
+    // element [rr][cc] = X_rr . Y_cc over the value rows ----
+    //   0 triu_s(V Q^T)^T   1 triu(V dY^T)^T   2 triu_s(SA Q^T)^T   3 triu(SA dY^T)^T
+    //   4 tril(dY SA^T)^T   5 tril(dY V^T)^T   6 tril_s(Q SA^T)^T   7 tril_s(Q V^T)^T
+    for (int j = wv; j < 8; j += TJ) {
+        // (X, Y): (Q, V) (dY, V) (Q, SA) (dY, SA) (SA, dY) (V, dY) (SA, Q) (V, Q)
+        const bool up = j < 4, tok = up ? (j & 1) == 0 : j >= 6;    // tok: Q, else dY
+        const bool sa = up ? j >= 2 : (j & 1) == 0;                 // sa: SA, else V
+        const uint16_t *gh = tok ? &sm.Q.h[0][0] : &sm.dY[0][0], *gl = tok ? &sm.Q.l[0][0] : nullptr;
+        const uint16_t *fh = sa ? &sm.SA.h[0][0] : &sm.V[0][0], *fl = sa ? &sm.SA.l[0][0] : nullptr;
+        const uint16_t *xh = up ? gh : fh, *xl = up ? gl : fl, *yh = up ? fh : gh, *yl = up ? fl : gl;
+        f32x4_t G = zero4();
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) pack8(hr[ks], Hh[ks], Hl[ks]), pack8(sr[ks], Sh[ks], Sl[ks]);
-    __syncthreads();  // SA, Q, csum
+        for (int ks = 0; ks < KS; ks++) {
+            const uint4 X = fragp(xh, CLB, r16, 32 * ks, lane), Y = fragp(yh, CLB, r16, 32 * ks, lane);
+            G = mma32(G, X, Y);
+            if (yl) G = mma32(G, X, fragp(yl, CLB, r16, 32 * ks, lane));
+            if (xl) G = mma32(G, fragp(xl, CLB, r16, 32 * ks, lane), Y);
+        }
+        const int strict = up ? (j & 1) == 0 : j >= 6;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int d = up ? 4 * q4 + e - r16 : r16 - (4 * q4 + e);
+            G[e] = d >= strict ? G[e] : 0.f;
+        }
+        const Pk g = pk(G);
+        sm.M[j][lane] = cat(g.h, g.l);
+    }
+    keys();
+    __syncthreads();  // M
 
     // ---- dK, dB, dR, dA, dw for the wave's keys ----
-    f32x4_t VH = zero4(), SAH = zero4(), dYS = zero4(), QS = zero4();
-    f32x4_t Gqv = zero4(), Gyv = zero4(), Gqs = zero4(), Gys = zero4();  // Gram matrices over the value rows
-    const bool tv = r16 < L;
+    auto M = [&](int i) {
+        const uint4 m = sm.M[i][lane];
+        return Pk{make_uint2(m.x, m.y), make_uint2(m.z, m.w)};
+    };
+    f32x4_t gK, gB, gR, gA;
+    {
+        f32x4_t At, Rt;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-        uint4 sh, sl, qh, ql;
-        get_split(sm.SA, lane, ks, sh, sl), get_split(sm.Q, lane, ks, qh, ql);
-        const long o = at_tok(tv ? r16 : 0);
-        const uint4 vh = bf16_frag(v + o, ks, q4, tv), yh = bf16_frag(dy + o, ks, q4, tv);  // (exact in bf16)
-        VH = mma32(mma32(VH, vh, Hh[ks]), vh, Hl[ks]);
-        SAH = mm3(SAH, sh, sl, Hh[ks], Hl[ks]);
-        dYS = mma32(mma32(dYS, yh, Sh[ks]), yh, Sl[ks]);
-        QS = mm3(QS, qh, ql, Sh[ks], Sl[ks]);
-        Gqv = mma32(mma32(Gqv, qh, vh), ql, vh);   // Q_rr . V_cc
-        Gyv = mma32(Gyv, yh, vh);                  // dY_rr . V_cc
-        Gqs = mm3(Gqs, qh, ql, sh, sl);            // Q_rr . SA_cc
-        Gys = mma32(mma32(Gys, yh, sh), yh, sl);   // dY_rr . SA_cc
+        for (int e = 0; e < 4; e++) At[e] = xa[e] * eA[e], Rt[e] = xr[e] * eR[e];
+        const Pk pAt = pk(At), pRt = pk(Rt);
+        gK = eM * (VH * eLj + mm16s(M(0), pAt) + mm16s(M(1), pRt));
+        gB = eM * (SAH * eLj + mm16s(M(2), pAt) + mm16s(M(3), pRt));
     }
-    const f32x4_t Gvq = transpose16(Gqv, lane), Gvy = transpose16(Gyv, lane);
-    const f32x4_t Gsq = transpose16(Gqs, lane), Gsy = transpose16(Gys, lane);
-    // masked transposes of the intra-chunk matrices, element [rr][cc] (rr = 4q4 + e, cc = r16)
-    f32x4_t M1, M2, M3, M4, M5, M6, M7, M8;
+    {
+        f32x4_t Bm, Km;
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const int rr = 4 * q4 + e;
-        M1[e] = rr > cc ? Gqv[e] : 0.f;   // triu_s(V Q^T)^T
-        M2[e] = rr >= cc ? Gyv[e] : 0.f;  // triu(V dY^T)^T
-        M3[e] = rr > cc ? Gqs[e] : 0.f;   // triu_s(SA Q^T)^T
-        M4[e] = rr >= cc ? Gys[e] : 0.f;  // triu(SA dY^T)^T
-        M5[e] = rr <= cc ? Gsy[e] : 0.f;  // tril(dY SA^T)^T
-        M6[e] = rr <= cc ? Gvy[e] : 0.f;  // tril(dY V^T)^T
-        M7[e] = rr < cc ? Gsq[e] : 0.f;   // tril_s(Q SA^T)^T
-        M8[e] = rr < cc ? Gvq[e] : 0.f;   // tril_s(Q V^T)^T
+        for (int e = 0; e < 4; e++) Bm[e] = xb[e] * eM[e], Km[e] = xk[e] * eM[e];
+        const Pk pBm = pk(Bm), pKm = pk(Km);
+        gR = eR * (dYS + mm16s(M(4), pBm) + mm16s(M(5), pKm));
+        gA = eA * (QS + mm16s(M(6), pBm) + mm16s(M(7), pKm));
     }
-    const Pk pAt = pk(At), pRt = pk(Rt), pBm = pk(Bm), pKm = pk(Km);
-    const f32x4_t gK = eM * (VH * eLj + mm16s(pk(M1), pAt) + mm16s(pk(M2), pRt));
-    const f32x4_t gB = eM * (SAH * eLj + mm16s(pk(M3), pAt) + mm16s(pk(M4), pRt));
-    const f32x4_t gR = eR * (dYS + mm16s(pk(M5), pBm) + mm16s(pk(M6), pKm));
-    const f32x4_t gA = eA * (QS + mm16s(pk(M7), pBm) + mm16s(pk(M8), pKm));
     // dlogd_t = sum_{s>=t} (r dR - b dB - k dK)_s + sum_{s>t} (a dA)_s + carry
     float sx[4], sy[4];
     {
@@ -1020,8 +1122,10 @@ template <int NK> static size_t bwd_workspace(int B, int T, int H, int cus) {
     return bwd_records<NK>(BH * n) + BH * n * NK * NK * sizeof(float) +
            resume_bytes(BH, NK, resume_segments(BH, NK, n, cus));
 }
+// (WKV7: and the chunks' matrices behind them)
 size_t wkv7_rec_bwd_workspace(int B, int T, int H, int N, int cus) {
-    return N == 64 ? bwd_workspace<64>(B, T, H, cus) : bwd_workspace<128>(B, T, H, cus);
+    const size_t mats = (size_t)B * H * ((T + BC - 1) / BC) * MATS * 64 * sizeof(uint4);
+    return mats + (N == 64 ? bwd_workspace<64>(B, T, H, cus) : bwd_workspace<128>(B, T, H, cus));
 }
 // The reverse scan over the records at ws, in one pass or in time segments.
 template <int NK, typename TI>
@@ -1052,12 +1156,14 @@ template <int NK> static void launch_rec_bwd(const Bwd& p, int cus) {
                  *k = static_cast<const bf16_t*>(p.k), *v = static_cast<const bf16_t*>(p.v),
                  *a = static_cast<const bf16_t*>(p.a), *b = static_cast<const bf16_t*>(p.b),
                  *dy = static_cast<const bf16_t*>(p.dy);
+    uint4* const mats =
+        reinterpret_cast<uint4*>(static_cast<uint8_t*>(p.ws) + bwd_workspace<NK>(p.B, p.T, p.H, cus));
     hipLaunchKernelGGL(wkv7_bwd_prep<NK>, dim3(nchunk, BH), dim3(64), 0, p.stream, p.T, p.H, r, w, k, a, b,
-                       static_cast<uint8_t*>(p.ws));
+                       static_cast<uint8_t*>(p.ws), mats);
     const float* const hbuf = scan_back<NK, bf16_t>(p.T, p.H, BH, 0, p.dsT, dy, p.ds0, p.ws, cus, p.stream);
     const int jobs = nchunk * BH, per_xcd = (jobs + 7) / 8;
     hipLaunchKernelGGL(wkv7_bwd_chunk<NK>, dim3(8 * per_xcd), dim3(4 * NK), 0, p.stream, p.T, p.H, BH, per_xcd, r, w, k,
-                       v, a, b, dy, p.ckpt, hbuf, static_cast<bf16_t*>(p.dr), static_cast<bf16_t*>(p.dw),
+                       v, a, b, dy, p.ckpt, hbuf, mats, static_cast<bf16_t*>(p.dr), static_cast<bf16_t*>(p.dw),
                        static_cast<bf16_t*>(p.dk), static_cast<bf16_t*>(p.dv), static_cast<bf16_t*>(p.da),
                        static_cast<bf16_t*>(p.db));
 }
