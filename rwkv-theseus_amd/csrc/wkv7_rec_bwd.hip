@@ -808,25 +808,44 @@ __global__ __launch_bounds__(64) void gdn_bwd_prep(int Tn, int H, int qk_norm, c
     }
 }
 
-struct GdnChunkLds {
-    SplitPlane<BNK> K, R;   // k, r = q / sqrt(N) [t][j], written by the key owners
-    SplitPlane<BNK> SA, Q;  // [t][i], written by the value-row owners
-    float gam[BC], gm1[BC], beta[BC];
+// The value rows' operands V and dY [t][i]: bf16 as given (exact), fp32 split.
+template <typename TI> struct RowPlane {
+    static constexpr int HALVES = sizeof(TI) == 2 ? 1 : 2;
+    uint16_t x[HALVES][BC][BNK + 8];
+    __device__ __forceinline__ const uint16_t* hi() const { return &x[0][0][0]; }
+    __device__ __forceinline__ const uint16_t* lo() const { return HALVES == 2 ? &x[HALVES - 1][0][0] : nullptr; }
+};
+template <typename TI> struct GdnChunkLds {
+    union {
+        struct {
+            SplitPlane<BNK> K, R;  // k, q as given [t][j], written by the key owners
+        };
+        uint16_t st[BNK * BNK];    // (then) the states, one half after another
+    };
+    SplitPlane<BNK> SA, Q;         // [t][i], written by the value-row owners
+    RowPlane<TI> V, dY;
+    uint4 mat[MATS][64];           // the chunk's matrices, then the masked Gram matrices, packed
+    float gam[BC], gm1[BC], beta[BC], fk[BC], fq[BC];  // (fk, fq: the norm factors)
     float csum[BTJ][BNK];
     float pv[BTJ][BC], pd[BTJ][BC], pk[BTJ][BC];  // per wave and token: sum v dV', sum dlogd, sum k dB
     float nk[BTJ][BC], nq[BTJ][BC];  // with qk_norm: sum k^2, sum q^2; then sum k dk, sum q dq of the normalised
 };
 
+// As wkv7_bwd_chunk, but for the chunk's matrices, which waves 0..2 form here (from two Gram
+// matrices over the keys; the inverse by one wave, not by all eight), and with the exact bf16
+// operands' zero lo parts left out.  One lane of 2048 tokens and 32 heads: 364 -> 300 us (the
+// states, inputs and outputs at the rate of a copy: 130).  128 registers with 15 spilled; the
+// inverse left out is 3 %, S_end's rows left out 9 %; other orders of the first loads or of
+// the matrices spill 13 to 20 and measure within 3 %.
 template <typename TI>
-__global__ __launch_bounds__(512) void gdn_bwd_chunk(int Tn, int H, int BH, int per_xcd, int qk_norm,
-                                                     const TI* __restrict__ q,
-                                                     const TI* __restrict__ k, const TI* __restrict__ v,
-                                                     const float* __restrict__ g, const float* __restrict__ beta,
-                                                     const TI* __restrict__ dy, const float* __restrict__ ckpt,
-                                                     const float* __restrict__ hbuf, TI* __restrict__ dq,
-                                                     TI* __restrict__ dk, TI* __restrict__ dv, float* __restrict__ dg,
-                                                     float* __restrict__ dbeta) {
-    __shared__ __attribute__((aligned(16))) GdnChunkLds sm;
+__global__ __launch_bounds__(512, sizeof(TI) == 2 ? 4 : 2) void gdn_bwd_chunk(
+    int Tn, int H, int BH, int per_xcd, int qk_norm, const TI* __restrict__ q, const TI* __restrict__ k,
+    const TI* __restrict__ v, const float* __restrict__ g, const float* __restrict__ beta, const TI* __restrict__ dy,
+    const float* __restrict__ ckpt, const float* __restrict__ hbuf, TI* __restrict__ dq, TI* __restrict__ dk,
+    TI* __restrict__ dv, float* __restrict__ dg, float* __restrict__ dbeta) {
+    constexpr bool EXACT = sizeof(TI) == 2;  // (k, q, v and dY without a lo part)
+    constexpr int CLB = BNK + 8;
+    __shared__ __attribute__((aligned(16))) GdnChunkLds<TI> sm;
     const int nchunk = (Tn + BC - 1) / BC;
     const int job = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if (job >= nchunk * BH) return;  // (whole workgroup)
@@ -864,24 +883,53 @@ __global__ __launch_bounds__(512) void gdn_bwd_chunk(int Tn, int H, int BH, int 
     };
     rows(Hm, hr);
     rows(Se, sr);
-    // k and r of the wave's keys in D layout ([t][col], t = 4q4 + e)
-    f32x4_t kD, rD;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const int t = 4 * q4 + e;
-        const bool ok = t < L;
-        const long o = at_tok(ok ? t : 0) + col;  // (clamped: every lane loads)
-        const float k_ = io<TI>::ld(k, o), q_ = io<TI>::ld(q, o);
-        kD[e] = keep(lane_mask(ok), k_);
-        rD[e] = keep(lane_mask(ok), q_) * rs;
+    {  // V and dY: four elements per thread, rows past the chunk's end zero
+        const int t = tid / (BNK / 4), cv = 4 * (tid % (BNK / 4));
+        const uint32_t m = lane_mask(t < L);
+        const long o = at_tok(t < L ? t : 0) + cv;
+        auto put_row = [&](RowPlane<TI>& P, const TI* x) {
+            if constexpr (EXACT) {
+                const uint2 u = *reinterpret_cast<const uint2*>(x + o);
+                *reinterpret_cast<uint2*>(&P.x[0][t][cv]) = make_uint2(u.x & m, u.y & m);
+            } else {
+                const float4 f = keep4(m, ld4f(x + o));
+                uint2 hi, lo;
+                pack4(f32x4_t{f.x, f.y, f.z, f.w}, hi, lo);
+                *reinterpret_cast<uint2*>(&P.x[0][t][cv]) = hi;
+                *reinterpret_cast<uint2*>(&P.x[RowPlane<TI>::HALVES - 1][t][cv]) = lo;
+            }
+        };
+        put_row(sm.V, v), put_row(sm.dY, dy);
     }
-    // (with qk_norm the planes hold k and r as given: their products are scaled below)
-    put_split(sm.K, kD, lane, wv), put_split(sm.R, rD, lane, wv);
-    if (qk_norm) {
+    // an input's column of the wave in D layout ([t][col], t = 4q4 + e), zero past the chunk's end
+    auto tile = [&](const TI* x) {
+        int u = q4;
+        asm volatile("" : "+v"(u));  // (opaque: a second reading is not merged with the first and held)
+        f32x4_t o;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const float sk = row_sum16(kD[e] * kD[e]), sq = row_sum16(rD[e] * rD[e]);
-            if (r16 == 0) sm.nk[wv][4 * q4 + e] = sk, sm.nq[wv][4 * q4 + e] = sq;
+            const int t = 4 * u + e;
+            const float f = io<TI>::ld(x, at_tok(t < L ? t : 0) + col);  // (clamped: every lane loads)
+            o[e] = keep(lane_mask(t < L), f);
+        }
+        return o;
+    };
+    // (the planes hold k and q as given: their products are scaled below)
+    {
+        const f32x4_t kD = tile(k), qD = tile(q);
+        if constexpr (EXACT) {
+            const int tr = 4 * q4 + (lane & 3), cv = 16 * wv + 4 * ((lane >> 2) & 3);
+            *reinterpret_cast<uint2*>(&sm.K.h[tr][cv]) = quad_rows_bf16(kD, lane);
+            *reinterpret_cast<uint2*>(&sm.R.h[tr][cv]) = quad_rows_bf16(qD, lane);
+        } else {
+            put_split(sm.K, kD, lane, wv), put_split(sm.R, qD, lane, wv);
+        }
+        if (qk_norm) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float sk = row_sum16(kD[e] * kD[e]), sq = row_sum16(qD[e] * qD[e]);
+                if (r16 == 0) sm.nk[wv][4 * q4 + e] = sk, sm.nq[wv][4 * q4 + e] = sq;
+            }
         }
     }
 #pragma unroll
@@ -899,60 +947,84 @@ __global__ __launch_bounds__(512) void gdn_bwd_chunk(int Tn, int H, int BH, int 
     for (int ks = 0; ks < BKS; ks++) pack8(sr[ks], Sh[ks], Sl[ks]);
     __syncthreads();
 
-    // token scalars: rows rr = 4q4 + e, column token cc = r16
-    const int cc = r16;
-    float gr[4], gm1r[4], br[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) gr[e] = sm.gam[4 * q4 + e], gm1r[e] = sm.gm1[4 * q4 + e], br[e] = sm.beta[4 * q4 + e];
-    const float gc = sm.gam[cc], gm1c = sm.gm1[cc], bc = sm.beta[cc], gL = sm.gam[BC - 1];
-    // the norm factors x * rsqrt(sum x^2 + 1e-6) of rows rr and column token cc (r = q / sqrt(N))
-    float nkr[4] = {1.f, 1.f, 1.f, 1.f}, nqr[4] = {1.f, 1.f, 1.f, 1.f}, nkc = 1.f;
+    // the norm factors x * rsqrt(sum x^2 + 1e-6) of column token r16, and of rows 4q4 + e by shuffle
+    float fk = 1.f, fq = 1.f;
     if (qk_norm) {
-        float sk = 0.f;
+        float sk = 0.f, sq = 0.f;
 #pragma unroll
-        for (int u = 0; u < BTJ; u++) sk += sm.nk[u][cc];
-        nkc = __frsqrt_rn(sk + 1e-6f);
+        for (int u = 0; u < BTJ; u++) sk += sm.nk[u][r16], sq += sm.nq[u][r16];
+        fk = __frsqrt_rn(sk + 1e-6f), fq = __frsqrt_rn(sq + 1e-6f);
+    }
+    if (wv == 0 && q4 == 0) sm.fk[r16] = fk, sm.fq[r16] = fq;
+    auto put_mat = [&](int i, const f32x4_t& x) {
+        const Pk p = pk(x);
+        sm.mat[i][lane] = cat(p.h, p.l);
+    };
+    auto mat = [&](int i) {
+        const uint4 m = sm.mat[i][lane];
+        return Pk{make_uint2(m.x, m.y), make_uint2(m.z, m.w)};
+    };
+    // the chunk's matrices, element [rr][cc] (rr = 4q4 + e, cc = r16): wave 0 the inverse, 1 Aak, 2 Brb and Brk
+    if (wv < 3) {
+        f32x4_t G = zero4();  // k_rr . k_cc; wave 2: q_rr . k_cc
+        const SplitPlane<BNK>& X = wv == 2 ? sm.R : sm.K;
+#pragma unroll
+        for (int ks = 0; ks < BKS; ks++) {
+            uint4 xh, xl, kh, kl;
+            get_split(X, lane, ks, xh, xl), get_split(sm.K, lane, ks, kh, kl);
+            G = EXACT ? mma32(G, xh, kh) : mm3(G, xh, xl, kh, kl);
+        }
+        const int cc = r16;
+        const float gc = sm.gam[cc], gm1c = sm.gm1[cc], bc = sm.beta[cc];
+        float gr[4], gm1r[4], br[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            float a = 0.f, b = 0.f;
+            gr[e] = sm.gam[4 * q4 + e], gm1r[e] = sm.gm1[4 * q4 + e], br[e] = sm.beta[4 * q4 + e];
+            G[e] *= (wv == 2 ? rs * __shfl(fq, 4 * q4 + e) : __shfl(fk, 4 * q4 + e)) * fk;
+        }
+        f32x4_t a, b;
+        if (wv == 0) {
+            f32x4_t Ti, TiT;
 #pragma unroll
-            for (int u = 0; u < BTJ; u++) a += sm.nk[u][4 * q4 + e], b += sm.nq[u][4 * q4 + e];
-            nkr[e] = __frsqrt_rn(a + 1e-6f), nqr[e] = __frsqrt_rn(b * (float)BNK + 1e-6f);
-            kD[e] *= nkr[e], rD[e] *= nqr[e];
+            for (int e = 0; e < 4; e++) {
+                const int rr = 4 * q4 + e;
+                a[e] = cc < rr ? -bc * G[e] * __expf(gm1r[e] - gm1c) : 0.f;
+                b[e] = rr < cc ? -br[e] * G[e] * __expf(gm1c - gm1r[e]) : 0.f;
+            }
+            tri_inverse(a, b, lane, Ti, TiT);
+            put_mat(MAT_TI, Ti), put_mat(MAT_TIT, TiT);
+        } else if (wv == 1) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int rr = 4 * q4 + e;
+                a[e] = cc < rr ? G[e] * __expf(gm1r[e] - gc) : 0.f;
+                b[e] = rr < cc ? G[e] * __expf(gm1c - gr[e]) : 0.f;
+            }
+            put_mat(MAT_AAK, a), put_mat(MAT_AAKT, b);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int rr = 4 * q4 + e;
+                a[e] = cc <= rr ? -bc * G[e] * __expf(gr[e] - gm1c) : 0.f;
+                b[e] = cc <= rr ? G[e] * __expf(gr[e] - gc) : 0.f;
+            }
+            put_mat(MAT_BRB, a), put_mat(MAT_BRK, b);
         }
     }
-    // Gram matrices over the keys and the wave's products k S0^T, k H^T
-    f32x4_t KK = zero4(), RK = zero4(), kS = zero4(), kH = zero4();
+    // the wave's products k S0^T, k H^T
+    f32x4_t P1 = zero4(), kH = zero4();
 #pragma unroll
     for (int ks = 0; ks < BKS; ks++) {
-        uint4 kh, kl, rh, rl;
-        get_split(sm.K, lane, ks, kh, kl), get_split(sm.R, lane, ks, rh, rl);
-        KK = mm3(KK, kh, kl, kh, kl);
-        RK = mm3(RK, rh, rl, kh, kl);  // r_rr . k_cc
-        kS = mm3(kS, kh, kl, Sh[ks], Sl[ks]);
-        kH = mm3(kH, kh, kl, Hh[ks], Hl[ks]);
+        uint4 kh, kl;
+        get_split(sm.K, lane, ks, kh, kl);
+        P1 = mma32(mma32(P1, kh, Sh[ks]), kh, Sl[ks]);
+        kH = mma32(mma32(kH, kh, Hh[ks]), kh, Hl[ks]);
+        if constexpr (!EXACT) P1 = mma32(P1, kl, Sh[ks]), kH = mma32(kH, kl, Hh[ks]);
     }
-    f32x4_t Aab, AabT, Aak, Brb, Brk, P1, P2, P3;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const int rr = 4 * q4 + e;
-        KK[e] *= nkr[e] * nkc, RK[e] *= nqr[e] * nkc, kS[e] *= nkr[e], kH[e] *= nkr[e];
-        Aab[e] = cc < rr ? -bc * KK[e] * __expf(gm1r[e] - gm1c) : 0.f;
-        AabT[e] = rr < cc ? -br[e] * KK[e] * __expf(gm1c - gm1r[e]) : 0.f;
-        Aak[e] = cc < rr ? KK[e] * __expf(gm1r[e] - gc) : 0.f;
-        Brb[e] = cc <= rr ? -bc * RK[e] * __expf(gr[e] - gm1c) : 0.f;
-        Brk[e] = cc <= rr ? RK[e] * __expf(gr[e] - gc) : 0.f;
-        P1[e] = kS[e] * __expf(gm1r[e]);
-        P2[e] = kH[e] * (-br[e] * __expf(gL - gm1r[e]));
-        P3[e] = kH[e] * __expf(gL - gr[e]);
-    }
-    f32x4_t Ti, TiT;
-    tri_inverse(Aab, AabT, lane, Ti, TiT);
-    const Pk pAak = pk(Aak), pBrb = pk(Brb), pBrk = pk(Brk), pTi = pk(Ti), pTiT = pk(TiT);
-    const Pk pAakT = pk(transpose16(Aak, lane));
+    __syncthreads();  // the matrices, the norm factors; (the key planes are read)
 
     auto put = [&](TI* dst, const f32x4_t& x) {
-        if constexpr (sizeof(TI) == 2) {
+        if constexpr (EXACT) {
             const int tr = 4 * q4 + (lane & 3);
             const uint2 qv = quad_rows_bf16(x, lane);  // (cross-lane: every lane takes part)
             if (tr < L) *reinterpret_cast<uint2*>(dst + at_tok(tr) + 16 * wv + 4 * ((lane >> 2) & 3)) = qv;
@@ -963,85 +1035,115 @@ __global__ __launch_bounds__(512) void gdn_bwd_chunk(int Tn, int H, int BH, int 
         }
     };
     // ---- SA, Q, dV' for the wave's value columns ----
-    f32x4_t vraw, vD, dyD;
+    {
+        const float gL = sm.gam[BC - 1];
+        f32x4_t P2, P3, vD, br;
+        const f32x4_t vraw = tile(v), dyD = tile(dy);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float gre = sm.gam[4 * q4 + e], gm1e = sm.gm1[4 * q4 + e], f = sm.fk[4 * q4 + e];
+            br[e] = sm.beta[4 * q4 + e];
+            P1[e] *= f * __expf(gm1e);
+            P2[e] = kH[e] * f * (-br[e] * __expf(gL - gm1e));
+            P3[e] = kH[e] * f * __expf(gL - gre);
+            vD[e] = br[e] * vraw[e];
+        }
+        const Pk pV = pk(vD), pdY = pk(dyD);
+        const f32x4_t SA = mm16s(mat(MAT_TIT), pk(P1 + mm16s(mat(MAT_AAKT), pV)));
+        const f32x4_t Q = mm16s(mat(MAT_TI), pk(P2 + mm16s(mat(MAT_BRB), pdY)));
+        const f32x4_t dVp = P3 + mm16s(mat(MAT_AAK), pk(Q)) + mm16s(mat(MAT_BRK), pdY);
+        put_split(sm.SA, SA, lane, wv), put_split(sm.Q, Q, lane, wv);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float s = row_sum16(vraw[e] * dVp[e]);
+            if (r16 == 0) sm.pv[wv][4 * q4 + e] = s;
+        }
+        put(dv, br * dVp);
+    }
+    // ---- the products over the value rows (V as given: V' = beta V of its rows below) ----
+    f32x4_t VH = zero4(), SAH = zero4(), dYS = zero4(), QS = zero4();
+    auto turn = [&](const uint4 (&x)[BKS], bool first) {
+        if (!first) __syncthreads();  // (the half before is read)
+#pragma unroll
+        for (int ks = 0; ks < BKS; ks++) put_state<BNK>(sm.st, x[ks], irow, ks, q4);
+        __syncthreads();  // (the first also: SA, Q, csum, pv; the matrices are read)
+    };
+    // acc += X m, acc2 += Y m (`low`: m is a lo half)
+    auto over_rows = [&](const RowPlane<TI>& X, const SplitPlane<BNK>& Y, bool low, f32x4_t& acc, f32x4_t& acc2) {
+#pragma unroll
+        for (int ks = 0; ks < BKS; ks++) {
+            const uint4 m = get_state<BNK>(sm.st, ks, wv, lane);
+            acc = mma32(acc, fragp(X.hi(), CLB, r16, 32 * ks, lane), m);
+            if (!EXACT && !low) acc = mma32(acc, fragp(X.lo(), CLB, r16, 32 * ks, lane), m);
+            acc2 = mma32(acc2, fragp(&Y.h[0][0], CLB, r16, 32 * ks, lane), m);
+            if (!low) acc2 = mma32(acc2, fragp(&Y.l[0][0], CLB, r16, 32 * ks, lane), m);
+        }
+    };
+    turn(Hh, true), over_rows(sm.V, sm.SA, false, VH, SAH);
+    turn(Hl, false), over_rows(sm.V, sm.SA, true, VH, SAH);
+    turn(Sh, false), over_rows(sm.dY, sm.Q, false, dYS, QS);
+    turn(Sl, false), over_rows(sm.dY, sm.Q, true, dYS, QS);
+
+    // ---- the intra-chunk matrices' masked transposes, shared out over waves 0..5: element
+    // [rr][cc] of the sums X_rr . Y_cc over the value rows ----
+    //   0 (Q, V')   1 (dY, V')   2 (Q, SA)   3 (dY, SA)   4 (SA, dY) + (V', dY)   5 (SA, Q) + (V', Q)
+    if (wv < 6) {
+        const int cc = r16;
+        const float gc = sm.gam[cc], gm1c = sm.gm1[cc], bc = sm.beta[cc];
+        float gr[4], gm1r[4], br[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) gr[e] = sm.gam[4 * q4 + e], gm1r[e] = sm.gm1[4 * q4 + e], br[e] = sm.beta[4 * q4 + e];
+        auto gram = [&](const uint16_t* xh, const uint16_t* xl, const uint16_t* yh, const uint16_t* yl) {
+            f32x4_t G = zero4();
+#pragma unroll
+            for (int ks = 0; ks < BKS; ks++) {
+                const uint4 X = fragp(xh, CLB, r16, 32 * ks, lane), Y = fragp(yh, CLB, r16, 32 * ks, lane);
+                G = mma32(G, X, Y);
+                if (yl) G = mma32(G, X, fragp(yl, CLB, r16, 32 * ks, lane));
+                if (xl) G = mma32(G, fragp(xl, CLB, r16, 32 * ks, lane), Y);
+            }
+            return G;
+        };
+        const bool tok = wv == 5 || (wv < 4 && wv % 2 == 0);  // with Q, else with dY
+        const uint16_t *yh = tok ? &sm.Q.h[0][0] : sm.dY.hi(), *yl = tok ? &sm.Q.l[0][0] : sm.dY.lo();
+        f32x4_t M;
+        if (wv < 4) {
+            const bool sa = wv >= 2;
+            M = gram(yh, yl, sa ? &sm.SA.h[0][0] : sm.V.hi(), sa ? &sm.SA.l[0][0] : sm.V.lo());
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int d = 4 * q4 + e - cc;
+                // triu_s: e^{gm1_rr - gam_cc}, triu: e^{gam_rr - gam_cc}
+                const float f = (sa ? 1.f : bc) * __expf((tok ? gm1r[e] : gr[e]) - gc);
+                M[e] = d >= (tok ? 1 : 0) ? M[e] * f : 0.f;
+            }
+        } else {
+            const f32x4_t S = gram(&sm.SA.h[0][0], &sm.SA.l[0][0], yh, yl), V = gram(sm.V.hi(), sm.V.lo(), yh, yl);
+            const float gcol = tok ? gm1c : gc;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int d = cc - (4 * q4 + e);
+                M[e] = d >= (tok ? 1 : 0) ? br[e] * (V[e] * __expf(gcol - gr[e]) - S[e] * __expf(gcol - gm1r[e])) : 0.f;
+            }
+        }
+        put_mat(wv, M);
+    }
+    // ---- dq, dk and the token sums for the wave's keys ----
+    float gr[4], gm1r[4], br[4], nkr[4], nqr[4];
+    const float gL = sm.gam[BC - 1];
+    f32x4_t kD = tile(k), rD = tile(q);
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         const int t = 4 * q4 + e;
-        const long o = at_tok(t < L ? t : 0) + col;
-        const float v_ = io<TI>::ld(v, o), y_ = io<TI>::ld(dy, o);
-        vraw[e] = keep(lane_mask(t < L), v_);
-        vD[e] = br[e] * vraw[e];
-        dyD[e] = keep(lane_mask(t < L), y_);
+        gr[e] = sm.gam[t], gm1r[e] = sm.gm1[t], br[e] = sm.beta[t], nkr[e] = sm.fk[t], nqr[e] = sm.fq[t];
+        kD[e] *= nkr[e], rD[e] *= rs * nqr[e];
+        VH[e] *= br[e];
     }
-    const Pk pV = pk(vD), pdY = pk(dyD);
-    const f32x4_t SA = mm16s(pTiT, pk(P1 + mm16s(pAakT, pV)));
-    const f32x4_t Q = mm16s(pTi, pk(P2 + mm16s(pBrb, pdY)));
-    const f32x4_t dVp = P3 + mm16s(pAak, pk(Q)) + mm16s(pBrk, pdY);
-    put_split(sm.SA, SA, lane, wv), put_split(sm.Q, Q, lane, wv);
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const float s = row_sum16(vraw[e] * dVp[e]);
-        if (r16 == 0) sm.pv[wv][4 * q4 + e] = s;
-    }
-    put(dv, f32x4_t{br[0] * dVp[0], br[1] * dVp[1], br[2] * dVp[2], br[3] * dVp[3]});
-#pragma unroll
-    for (int ks = 0; ks < BKS; ks++)
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int i = 32 * ks + (e < 4 ? 4 * q4 + e : 16 + 4 * q4 + e - 4);
-            hr[ks][e] = Hm[(long)i * BNK + col];
-            sr[ks][e] = S0[(long)i * BNK + col];
-        }
-#pragma unroll
-    for (int ks = 0; ks < BKS; ks++) pack8(hr[ks], Hh[ks], Hl[ks]), pack8(sr[ks], Sh[ks], Sl[ks]);
-    __syncthreads();  // SA, Q, csum, pv
-
-    // ---- dq, dk and the token sums for the wave's keys ----
-    f32x4_t VH = zero4(), SAH = zero4(), dYS = zero4(), QS = zero4();
-    f32x4_t Gqv = zero4(), Gyv = zero4(), Gqs = zero4(), Gys = zero4();
-    const bool tv = r16 < L;
-#pragma unroll
-    for (int ks = 0; ks < BKS; ks++) {
-        float fv[8], fy[8];
-        {
-            const long o = at_tok(tv ? r16 : 0) + 32 * ks + 4 * q4;
-            const uint32_t m = lane_mask(tv);
-            const float4 v0 = keep4(m, ld4f(v + o)), v1 = keep4(m, ld4f(v + o + 16));
-            const float4 y0 = keep4(m, ld4f(dy + o)), y1 = keep4(m, ld4f(dy + o + 16));
-            fv[0] = v0.x, fv[1] = v0.y, fv[2] = v0.z, fv[3] = v0.w, fv[4] = v1.x, fv[5] = v1.y, fv[6] = v1.z, fv[7] = v1.w;
-            fy[0] = y0.x, fy[1] = y0.y, fy[2] = y0.z, fy[3] = y0.w, fy[4] = y1.x, fy[5] = y1.y, fy[6] = y1.z, fy[7] = y1.w;
-#pragma unroll
-            for (int e = 0; e < 8; e++) fv[e] *= bc;  // V' = beta v (the lane's token r16)
-        }
-        uint4 sh, sl, qh, ql, vh, vl, yh, yl;
-        get_split(sm.SA, lane, ks, sh, sl), get_split(sm.Q, lane, ks, qh, ql);
-        pack8(fv, vh, vl), pack8(fy, yh, yl);
-        VH = mm3(VH, vh, vl, Hh[ks], Hl[ks]);
-        SAH = mm3(SAH, sh, sl, Hh[ks], Hl[ks]);
-        dYS = mm3(dYS, yh, yl, Sh[ks], Sl[ks]);
-        QS = mm3(QS, qh, ql, Sh[ks], Sl[ks]);
-        Gqv = mm3(Gqv, qh, ql, vh, vl);  // Q_rr . V'_cc
-        Gyv = mm3(Gyv, yh, yl, vh, vl);  // dY_rr . V'_cc
-        Gqs = mm3(Gqs, qh, ql, sh, sl);  // Q_rr . SA_cc
-        Gys = mm3(Gys, yh, yl, sh, sl);  // dY_rr . SA_cc
-    }
-    const f32x4_t Gvq = transpose16(Gqv, lane), Gvy = transpose16(Gyv, lane);
-    const f32x4_t Gsq = transpose16(Gqs, lane), Gsy = transpose16(Gys, lane);
-    f32x4_t M1, M2, M3, M4, M56, M78;  // transposes, element [rr][cc]
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const int rr = 4 * q4 + e;
-        M1[e] = rr > cc ? Gqv[e] * __expf(gm1r[e] - gc) : 0.f;
-        M2[e] = rr >= cc ? Gyv[e] * __expf(gr[e] - gc) : 0.f;
-        M3[e] = rr > cc ? Gqs[e] * __expf(gm1r[e] - gc) : 0.f;
-        M4[e] = rr >= cc ? Gys[e] * __expf(gr[e] - gc) : 0.f;
-        M56[e] = rr <= cc ? -br[e] * Gsy[e] * __expf(gc - gm1r[e]) + Gvy[e] * __expf(gc - gr[e]) : 0.f;
-        M78[e] = rr < cc ? -br[e] * Gsq[e] * __expf(gm1c - gm1r[e]) + Gvq[e] * __expf(gm1c - gr[e]) : 0.f;
-    }
+    __syncthreads();  // the Gram matrices
     const Pk pkD = pk(kD), prD = pk(rD);
-    const f32x4_t tK = mm16s(pk(M1), pkD) + mm16s(pk(M2), prD);
-    const f32x4_t tB = mm16s(pk(M3), pkD) + mm16s(pk(M4), prD);
-    const f32x4_t tR = mm16s(pk(M56), pkD), tA = mm16s(pk(M78), pkD);
+    const f32x4_t tK = mm16s(mat(0), pkD) + mm16s(mat(1), prD);
+    const f32x4_t tB = mm16s(mat(2), pkD) + mm16s(mat(3), prD);
+    const f32x4_t tR = mm16s(mat(4), pkD), tA = mm16s(mat(5), pkD);
     f32x4_t gK, gB, gR, gA, egb;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
