@@ -90,7 +90,7 @@ const char* theseus_wkv7_error_string(int status);
 /* Which kernel family theseus_wkv7_forward / _backward use for these sizes
  * (a theseus_wkv7_family value), or minus a status code for invalid sizes.
  * The step-serial kernels are exact but run one step at a time (config 2:
- * ~0.12 M tokens/s against ~9 M on the chunked kernels); callers can warn or
+ * 1.56 M tokens/s against 10.2 M on the chunked kernels); callers can warn or
  * refuse when a call would fall back to them.  No counterpart in the
  * reference (its kernel is step-serial for every call, kernels/wkv7_state.cu:81-92). */
 int theseus_wkv7_kernel_family(int B, int T, int H, int N, int dtype);
@@ -127,7 +127,9 @@ long long theseus_wkv7_checkpoint_count(int T);
  * need for these sizes and dtype on the current device (0 when none).  The
  * chunked kernels use it when B*H heads outnumber the device's CUs: heads are
  * then cut between workgroups, which hand the carried state over through it;
- * the step-serial backward replays each 16-step segment into it.  For few
+ * the step-serial backward keeps dL/dS at every 16-step segment's end in it;
+ * the chunk-record kernels their records, states and the segments of their
+ * scans.  For few
  * heads (chunked kernels, 2*B*H <= CUs, T > 112) the forward size also covers
  * the time-split forward: a forward without saved states given that much cuts
  * every head's steps into k = min(4, CUs / (B*H)) segments that run at once,
@@ -143,8 +145,8 @@ size_t theseus_wkv7_forward_workspace_size(int B, int T, int H, int N, int dtype
 size_t theseus_wkv7_backward_workspace_size(int B, int T, int H, int N, int dtype);
 /* The workspace with which a forward runs fastest, at least theseus_wkv7_forward_workspace_size:
  * more for calls whose few heads leave CUs idle.  saved_states: whether ckpt is given.
- *  - bf16, N = 64 with saved states and few heads (n = ceil(T/16) > 16 chunks,
- *    (CUs/4 - B*H) n > 600): the chunk records of the two-launch form and its time split
+ *  - bf16, N = 64 with saved states and few heads (n = ceil(T/16) > 28 chunks,
+ *    B*H <= CUs/4, (3 CUs/10 - B*H) n > 760): the chunk records of the two-launch form and its time split
  *    (the saved states' order does not depend on it);
  *  - bf16, N = 128: the buffers of up to 9 time segments. */
 size_t theseus_wkv7_forward_best_workspace_size(int B, int T, int H, int N, int dtype, int saved_states);

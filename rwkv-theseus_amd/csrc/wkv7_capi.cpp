@@ -101,18 +101,21 @@ static bool split_ok(const Fwd& p) {
 // the chunked kernels' time (1.55 us a chunk forward, 2.8 backward, one workgroup per head
 // and the other CUs idle: 4.35 n + 12 us for both, n chunks a head, whatever the heads), so the
 // chunk-record kernels take it, whose scans carry less per chunk, are cut in time and leave
-// the rest to every chunk at once (about 50 + 0.053 B H n us on 256 CUs).  The two meet at
-// B H = 82 - 717 / n; the line is drawn a fifth below.  Forward + backward in us, chunked
-// against records: T=272 8 heads 83 / 64, 40 heads 86 / 89; T=512 20 heads 144 / 96; T=1021
-// 40 heads 276 / 177, 80 heads 280 / 321; T=4096 40 heads 1034 / 647.  The saved states are
+// the rest to every chunk at once.  Forward + backward in us, chunked against records: T=272
+// 20 heads 84 / 79, 32 heads 86 / 83, 40 heads 87 / 86; T=512 50 heads 148 / 128; T=1021 55
+// heads 280 / 216, 64 heads 279 / 240; T=2048 60 heads 532 / 465, 64 heads 530 / 480, 72 heads
+// 535 / 545 (the scans then have four segments, not five), 80 heads 540 / 586.  The line lies
+// at CUs/4 heads, lower for short calls, and at 28 chunks: the records' eleven launches take
+// the host 125 us through autograd, the chunked kernels' four 100 (T=272 8 heads 124 against
+// 101, T=400 44 heads 124 against 119, T=512 52 heads 128 against 147).  The saved states are
 // the chunked kernels' (tiled), so each direction decides by itself: the forward when the
 // workspace holds the records (forward_workspace_best), the backward by its own size.
 static bool rec64_shape(int B, int T, int H, int N, int dtype, int flags) {
     if (!chunk_ok(B, T, H, N, dtype, flags) || (long long)B * H > 65535 ||
         wkv7_rec_workspace(1, T, 1, N) >= (1ull << 32))
         return false;
-    const long long n = (T + kCkptInterval - 1) / kCkptInterval, room = cu_count() / 4 - (long long)B * H;
-    return n > 16 && room > 0 && room * n > 600;
+    const long long n = (T + kCkptInterval - 1) / kCkptInterval, cus = cu_count(), BH = (long long)B * H;
+    return n > 28 && BH <= cus / 4 && (3 * cus / 10 - BH) * n > 760;
 }
 static bool rec64_ok(const Fwd& p) {
     return p.ckpt && rec64_shape(p.B, p.T, p.H, p.N, p.dtype, p.flags) && p.ws &&
@@ -138,8 +141,8 @@ void launch_backward(const Bwd& p) {
     else if (rec_shape(p.B, p.T, p.H, p.N, p.dtype, p.flags)) launch_wkv7_rec_backward(p, cu_count());
     else launch_seq_backward(p);
 }
-// The chunked kernels' handoffs; the step-serial backward replays each
-// 16-step segment into its workspace (its forward needs none).
+// The chunked kernels' handoffs; the step-serial backward keeps dL/dS at every segment's
+// end and the segments' sums in its workspace (its forward needs none).
 size_t forward_workspace(int B, int T, int H, int N, int dtype, int flags) {
     return chunk_ok(B, T, H, N, dtype, flags) ? chunk_forward_workspace(B, T, H, cu_count()) : 0;
 }
