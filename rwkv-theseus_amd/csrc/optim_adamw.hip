@@ -13,8 +13,8 @@
 //   adamw:       every element's update with g = grad * (grad_scale * clip),
 //                reading the factor from device memory.
 // HBM per parameter: the gradient twice (4 + 4 B), param / moments read and
-// written (24 B): 32 B; the update alone needs 28 B.  The update walks the chunks
-// backwards, so it starts on the gradients that the norm pass read last while the
+// written (24 B): 32 B; the update alone needs 28 B.  Past L2_BYTES of gradients the
+// update walks the chunks backwards, so it starts on the gradients that the norm pass read last while the
 // 256 MB memory-side cache still holds them.
 //
 // The tensor list travels in kernel arguments (32 tensors per launch, under
@@ -40,6 +40,9 @@ constexpr int BATCH = 32;  // tensors per launch
 // (forwards, all non-temporal) -> now: 107.9 M parameters 640 -> 613 us, 69.5 M 413 -> 389,
 // 39.6 M 240 -> 224, 18 M 117 -> 114, below 10 M equal (bound by the call); with every gradient
 // loaded ordinarily the norm pass itself costs 78 instead of 75 us and the update gains nothing.
+// Up to L2_BYTES, what the eight L2s hold together, the update walks forwards behind
+// non-temporal loads (the update at 2.9 M parameters 25.5 us, backwards 27.6; at 5 M 32.8 and
+// 32.5; at 20 M 103.5 and 93.8).
 typedef float vf4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float4 ld_nt(const float4* p) {
     const vf4 t = __builtin_nontemporal_load(reinterpret_cast<const vf4*>(p));
@@ -68,7 +71,7 @@ struct Batch {
 static_assert(sizeof(Batch) < 4096, "kernel arguments");
 
 static long long chunks_of(long long n) { return (n + CHUNK - 1) / CHUNK; }
-constexpr long long KEEP_BYTES = 192ll << 20;
+constexpr long long KEEP_BYTES = 192ll << 20, L2_BYTES = 32ll << 20;
 
 // the tensor of this workgroup's chunk, and the chunk's first element and length
 struct Where {
@@ -76,11 +79,15 @@ struct Where {
     long long start;
     int len;
 };
-__device__ __forceinline__ Where locate(const Batch& bt, bool back) {
-    const int b = blockIdx.x;
+template <bool BACK = false> __device__ __forceinline__ Where locate(const Batch& bt) {
+    int b = blockIdx.x;
+    if constexpr (BACK) {  // each eight permuted so that chunk c of a launch stays on XCD c % 8, whose L2 may hold its gradients
+        const int total = gridDim.x;
+        if (b < (total & ~7)) b = (b & ~7) | ((total - 1 - b) & 7);
+    }
     int i = 0;
     while (i + 1 < bt.count && bt.chunk0[i + 1] <= b) i++;
-    const int k = back ? bt.chunk0[i + 1] - 1 - b : b - bt.chunk0[i];
+    const int k = BACK ? bt.chunk0[i + 1] - 1 - b : b - bt.chunk0[i];
     const long long start = (long long)k * CHUNK;
     const long long rem = bt.t[i].n - start;
     return Where{i, start, (int)(rem < CHUNK ? rem : CHUNK)};
@@ -102,7 +109,7 @@ __device__ __forceinline__ double block_sum(double x, double* red) {
 
 __global__ __launch_bounds__(THREADS) void grad_sumsq(Batch bt, double* __restrict__ partial) {
     __shared__ double red[THREADS / 64];
-    const Where w = locate(bt, false);
+    const Where w = locate(bt);
     const float* g = bt.t[w.i].g + w.start;
     double acc = 0.0;
     auto sum4 = [&](const float4& x) {
@@ -163,10 +170,10 @@ __device__ __forceinline__ void adamw_one(float& p, float g, float& m, float& v,
     p -= t.step_size * (m / denom);
 }
 
-__global__ __launch_bounds__(THREADS) void adamw(Batch bt, Hyper h, const float* __restrict__ result) {
+template <bool BACK> __global__ __launch_bounds__(THREADS) void adamw(Batch bt, Hyper h, const float* __restrict__ result) {
     if (h.skip_nonfinite && result[2] != 0.0f) return;
     const float mult = result[1];
-    const Where w = locate(bt, true);
+    const Where w = locate<BACK>(bt);
     const TensorArg& t = bt.t[w.i];
     float* p = t.p + w.start;
     const float* g = t.g + w.start;
@@ -255,8 +262,10 @@ int theseus_adamw_step(const theseus_adamw_tensor* tensors, int ntensors, float 
         return THESEUS_WKV7_ERR_WORKSPACE;
     double* partial = static_cast<double*>(workspace);
     optim::Batch bt;
-    const long long keep = nchunks - optim::KEEP_BYTES / (optim::CHUNK * (long long)sizeof(float));
-    bt.keep_from = keep > 0 ? (int)keep : 0;
+    constexpr long long CHUNK_BYTES = optim::CHUNK * (long long)sizeof(float);
+    const long long keep = nchunks - optim::KEEP_BYTES / CHUNK_BYTES;
+    const bool back = nchunks > optim::L2_BYTES / CHUNK_BYTES;
+    bt.keep_from = !back ? (int)nchunks : keep > 0 ? (int)keep : 0;
     int next = 0;
     long long base = 0;
     while (norm && optim::next_batch(tensors, ntensors, next, base, bt))
@@ -267,9 +276,9 @@ int theseus_adamw_step(const theseus_adamw_tensor* tensors, int ntensors, float 
     const optim::Hyper h{beta1, beta2, eps, skip_nonfinite};
     next = 0;
     base = 0;
-    while (optim::next_batch(tensors, ntensors, next, base, bt, true))
-        hipLaunchKernelGGL(optim::adamw, dim3(bt.chunk0[bt.count]), dim3(optim::THREADS), 0, stream, bt, h,
-                           result);
+    while (optim::next_batch(tensors, ntensors, next, base, bt, back))
+        hipLaunchKernelGGL(back ? optim::adamw<true> : optim::adamw<false>, dim3(bt.chunk0[bt.count]),
+                           dim3(optim::THREADS), 0, stream, bt, h, result);
     return hipGetLastError() == hipSuccess ? THESEUS_WKV7_OK : THESEUS_WKV7_ERR_LAUNCH;
 }
 

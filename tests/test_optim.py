@@ -202,11 +202,11 @@ def test_fused_step_is_deterministic():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("count, size", [(1, 16384 * 3200 + 5), (70, 16384 * 47 + 3), (33, 16385)],
-                         ids=["one-past-the-kept", "three-launches-past-the-kept", "all-kept"])
+@pytest.mark.parametrize("count, size", [(1, 16384 * 3200 + 5), (70, 16384 * 47 + 3), (33, 16384 * 16 + 1), (32, 16384 * 16)],
+                         ids=["one-past-the-kept", "three-launches-past-the-kept", "all-kept", "forwards"])
 def test_update_in_reverse_order_reads_every_chunk_once(count, size):
-    """The norm keeps the last 192 MB of gradients (3072 chunks) cached and the update walks
-    from the last chunk: past that line, with more than one launch, and within it, every
+    """Past 512 chunks the norm keeps the last 192 MB of gradients (3072 chunks) cached and the
+    update walks from the last chunk: past that line, with more than one launch, within it, and forwards, every
     element gets exactly one step (the first step moves each parameter by lr * g / (|g| + eps *
     sqrt(bias)), i.e. by lr to 1e-3 for |g| >= 1e-2 at eps 1e-8) and the norm is the sum over
     all (sizes not multiples of 4, so the second tensor on is not 16-byte aligned in `flat`)."""
