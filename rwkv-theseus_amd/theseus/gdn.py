@@ -146,9 +146,8 @@ def patch_transformers(module):
     (cu_seqlens): without gradients for K == V <= 128 (the teacher's forward, on the
     chunked kernels for 64 and 128), with gradients for K == V == 128 (the chunked forward
     and backward); any other call goes to the function that was there -- with gradients
-    at other head sizes, transformers' own chunked torch function (37 ms forward+backward
-    at B=1, T=2048, H=32, K=V=128 on MI355X) beats the step-serial backward.  Returns the
-    previous pair."""
+    at other head sizes, transformers' own chunked torch function.  Returns the previous
+    pair."""
     old = (module.torch_chunk_gated_delta_rule, module.torch_recurrent_gated_delta_rule)
 
     def route(ours, theirs):
