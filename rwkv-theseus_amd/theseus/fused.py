@@ -188,9 +188,13 @@ def native_layer(m):
 def pack_params(params, C):
     """The C-element parameters as float32 rows [n, C] in one launch (bf16 or float32 ones; others
     are converted first): a call's own copies, the kernels' inputs without gradients."""
+    n, dev = len(params), params[0].device
+    for p in params:  # (the kernel reads C elements of each)
+        if p.numel() != C or p.device != dev:
+            raise RuntimeError(f"pack_params: expected parameters of {C} elements on {dev}, got {tuple(p.shape)} "
+                               f"on {p.device}")
     src = [p.detach() if p.dtype in (torch.float32, torch.bfloat16) else p.detach().float() for p in params]
     src = [p if p.is_contiguous() else p.contiguous() for p in src]
-    n, dev = len(src), src[0].device
     out = torch.empty(n, C, dtype=torch.float32, device=dev)
     ptrs = (ctypes.c_void_p * n)(*[p.data_ptr() for p in src])
     dts = (ctypes.c_int * n)(*[0 if p.dtype == torch.bfloat16 else 1 for p in src])
@@ -200,7 +204,7 @@ def pack_params(params, C):
 
 
 def _vec(p, C):
-    if p.dtype == torch.float32 and p.dim() == 1 and not p.requires_grad and p.is_contiguous():
+    if p.dtype == torch.float32 and p.shape == (C,) and not p.requires_grad and p.is_contiguous():
         return p  # (a row of pack_params)
     if p.dtype == torch.float32:
         return p.detach().reshape(C).contiguous()
@@ -208,9 +212,14 @@ def _vec(p, C):
 
 
 def _coef_matrix(coefs, C):
-    if isinstance(coefs, torch.Tensor):  # (rows of pack_params)
-        return coefs
-    return _cached("coefs", tuple(coefs), lambda: torch.stack([_vec(c, C) for c in coefs]).contiguous())
+    if (isinstance(coefs, torch.Tensor) and coefs.dtype == torch.float32 and coefs.shape == (6, C)
+            and coefs.is_contiguous()):
+        cf = coefs  # (rows of pack_params)
+    else:
+        cf = _cached("coefs", tuple(coefs), lambda: torch.stack([_vec(c, C) for c in coefs]).contiguous())
+    if cf.shape != (6, C):
+        raise RuntimeError(f"shift_lerp: expected six coefficients of {C} elements, got {tuple(cf.shape)}")
+    return cf
 
 
 def _shift_lerp_fwd(x, shift, coefs):
@@ -218,6 +227,8 @@ def _shift_lerp_fwd(x, shift, coefs):
     x = x.contiguous()
     shift = shift.to(x.dtype).contiguous()
     cf = _coef_matrix(coefs, C)
+    if cf.device != x.device:
+        raise RuntimeError(f"shift_lerp: coefficients on {cf.device}, x on {x.device}")
     outs = [torch.empty_like(x) for _ in range(6)]
     arr = (ctypes.c_void_p * 6)(*[o.data_ptr() for o in outs])
     with torch.cuda.device(x.device):
@@ -299,6 +310,8 @@ def _kk_fwd(k, za, a0, k_k, k_a, N, dtype, zw=None, w0=None):
     k = k.to(torch.bfloat16).contiguous()
     zs = za.to(torch.bfloat16).contiguous()
     a0v, kk_, ka = _vec(a0, C), _vec(k_k, C), _vec(k_a, C)
+    if zw is not None and (zw.shape[-1] != C or zw.numel() != k.numel()):
+        raise RuntimeError(f"kk_kmod_w: expected a decay input like k {tuple(k.shape)}, got {tuple(zw.shape)}")
     kw, aw, bw = (torch.empty((B, T, C // N, N), dtype=torch.bfloat16, device=k.device) for _ in range(3))
     args = (B, T, C, _p(k), _p(zs), _p(a0v), _p(kk_), _p(ka), _p(kw), _p(aw), _p(bw))
     outs = (kw, aw, bw)
