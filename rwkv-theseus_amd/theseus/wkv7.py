@@ -29,6 +29,7 @@ from functools import lru_cache
 from pathlib import Path
 
 import torch
+from torch.autograd import forward_ad
 
 DECAY_SCALE = 0.6065306597126334  # e^{-1/2} (theseus/wkv7.py:19)
 LIB_PATH = Path(__file__).resolve().parent / "libtheseus_wkv7.so"
@@ -443,10 +444,13 @@ def _native_module():
 
 
 def _native(*xs):
-    """The native functions when they cover a call: plain tensors, no functorch transform (the
-    Python functions say there what they do not support)."""
+    """The native functions when they cover a call: plain tensors; no functorch transform and no
+    forward-mode level (the Python functions say there what they do not support); no
+    torch.jit.trace (which records a Python function as a node that runs it again, but of a
+    native one only the torch operators inside, the outputs' empty_like without the kernel)."""
     m = _native_module()
-    if m is None or torch._C._are_functorch_transforms_active():
+    if (m is None or torch._C._are_functorch_transforms_active() or torch._C._get_tracing_state() is not None
+            or forward_ad._current_level >= 0):
         return None
     return m if all(type(x) in (torch.Tensor, torch.nn.Parameter) for x in xs) else None
 

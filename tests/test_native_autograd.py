@@ -23,6 +23,11 @@ def test_calls_that_stay_with_python():
     seen = []
     torch.func.vmap(lambda t: (seen.append(W._native(t)), t)[1])(torch.zeros(2, 3))
     assert seen == [None]
+    torch.jit.trace(lambda t: (seen.append(W._native(t)), t * 2)[1], torch.zeros(2), check_trace=False)
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(W._native(x))
+    assert seen == [None] * len(seen) and len(seen) >= 3
+    assert W._native(x) is not None
 
 
 def _case(B, T, H, N, dtype):
@@ -113,3 +118,33 @@ def test_checks_streams_hooks_and_family(monkeypatch):
     monkeypatch.setenv("THESEUS_WKV7_STRICT", "1")
     with pytest.raises(RuntimeError, match="step-serial kernels"):
         W.wkv7(*[x.float() for x in a[:6]], a[6])
+
+
+@pytest.mark.gpu
+def test_traced_calls_run_the_kernels():
+    """torch.jit.trace of calls with gradients: the traced function replays the operator."""
+    xs, _, _ = _case(1, 40, 2, 64, torch.bfloat16)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    B, T, H, N = 1, 40, 2, 128
+    gs = [rnd(B, T, H, N) * N ** -.5 for _ in range(3)] + [-rnd(B, T, H).exp(), rnd(B, T, H).sigmoid(), rnd(B, H, N, N)]
+
+    def delta_rule(*a):
+        return G.gated_delta_rule(*a, output_final_state=True, use_qk_l2norm_in_kernel=True)
+
+    for f, args in ((lambda *a: W.wkv7(*a), xs), (delta_rule, gs)):
+        args = tuple(a.requires_grad_() for a in args)
+        traced = torch.jit.trace(f, args, check_trace=False)
+        other = tuple((a.detach() * .5).requires_grad_() for a in args)
+        for a in (args, other):
+            assert all(torch.equal(p, q) for p, q in zip(traced(*a), f(*a)))
+
+
+@pytest.mark.gpu
+def test_forward_mode_is_refused_by_the_python_functions():
+    xs, _, _ = _case(1, 40, 2, 64, torch.bfloat16)
+    xs = [x.requires_grad_() for x in xs]
+    with torch.autograd.forward_ad.dual_level():
+        r = torch.autograd.forward_ad.make_dual(xs[0], torch.ones_like(xs[0]))
+        with pytest.raises(NotImplementedError, match="jvp"):
+            W.wkv7(r, *xs[1:])
