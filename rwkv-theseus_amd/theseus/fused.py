@@ -29,6 +29,7 @@ import contextlib
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
 
 from .wkv7 import extension
 
@@ -265,8 +266,8 @@ class _ShiftLerp(torch.autograd.Function):
 
 
 def shift_lerp(x, shift, coefs):
-    """coefs: the six parameters, or (without gradients) their rows of ``pack_params``."""
-    if isinstance(coefs, torch.Tensor) or not _needs_grad(x, shift, *coefs):  # (no autograd node)
+    """coefs: the six parameters, or one [6, C] tensor (``pack_params``' rows without a copy)."""
+    if _direct(x, shift, *((coefs,) if isinstance(coefs, torch.Tensor) else coefs)):  # (no autograd node)
         return tuple(_shift_lerp_fwd(x, shift, coefs)[1])
     return _ShiftLerp.apply(x, shift, *coefs)
 
@@ -303,6 +304,15 @@ def add_param(z, p):
 
 def _needs_grad(*ts):
     return torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in ts)
+
+
+def _direct(*ts):
+    """Whether a call may go past its autograd function: no gradient wanted, and nothing on that only
+    the function answers -- a forward-mode level or a functorch transform (it refuses both, where
+    the bare kernel would drop the tangent) or torch.jit.trace (which records it as a node that
+    runs again, where the bare kernel leaves nothing behind)."""
+    return not (_needs_grad(*ts) or forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
+                or torch._C._are_functorch_transforms_active())
 
 
 def _kk_fwd(k, za, a0, k_k, k_a, N, dtype, zw=None, w0=None):

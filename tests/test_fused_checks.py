@@ -59,3 +59,16 @@ def test_decay_input_like_k(shape):
     v = torch.ones(C)
     with pytest.raises(RuntimeError, match="decay input like k"):
         fused.kk_kmod_w(k, k, v, v, v, torch.zeros(shape, dtype=torch.bfloat16), v, 64, torch.bfloat16)
+
+
+def test_direct_calls():
+    """A call goes past its autograd function only when nothing that the function answers is on."""
+    x, p, seen = torch.ones(2), torch.ones(2, requires_grad=True), []
+    assert fused._direct(x, x) and not fused._direct(x, p)
+    with torch.no_grad():
+        assert fused._direct(x, p)
+        torch.jit.trace(lambda t: (seen.append(fused._direct(t)), t * 2)[1], x, check_trace=False)
+        torch.func.vmap(lambda t: (seen.append(fused._direct(t)), t)[1])(x)
+        with torch.autograd.forward_ad.dual_level():
+            seen.append(fused._direct(x))
+    assert seen == [False] * len(seen) and len(seen) >= 3

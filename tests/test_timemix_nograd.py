@@ -74,3 +74,44 @@ def test_layer_without_gradients_equals_the_layer_with(dtype):
     # (7 chunks: below the time split, which only calls without saved states take)
     assert torch.equal(out, ref) and not out.requires_grad
     assert torch.equal(st["wkv"], st2["wkv"])
+
+
+def _shift_case(C=256):
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x, shift = torch.randn(1, 40, C, generator=g, device="cuda").to(bf), torch.randn(1, C, generator=g, device="cuda").to(bf)
+    return x, shift, torch.rand(6, C, generator=g, device="cuda")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, bf, torch.float64])
+def test_coefficient_tensor_keeps_its_gradients(dtype):
+    """Six parameters or one [6, C] tensor of them, of any type: the same mixes and gradients."""
+    x, shift, c = _shift_case()
+    c = c.to(dtype).requires_grad_()
+    rows = [r.detach().reshape(1, 1, -1).requires_grad_() for r in c]
+    got, want = fused.shift_lerp(x, shift, c), fused.shift_lerp(x, shift, rows)
+    dys = [torch.full_like(x, i + 1) for i in range(6)]
+    gc, gr = torch.autograd.grad(got, c, dys)[0], torch.autograd.grad(want, rows, dys)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert torch.equal(gc, torch.cat(gr, 1)[0])
+    with torch.no_grad():
+        assert all(torch.equal(a, b) for a, b in zip(fused.shift_lerp(x, shift, c), want))
+
+
+def test_shift_lerp_leaves_to_its_function_what_only_that_answers():
+    x, shift, c = _shift_case()
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda x, s, c: fused.shift_lerp(x, s, c), (x, shift, c), check_trace=False)
+        assert all(torch.equal(a, b) for a, b in zip(traced(2 * x, shift, c), fused.shift_lerp(2 * x, shift, c)))
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(NotImplementedError, match="jvp"):
+        fused.shift_lerp(torch.autograd.forward_ad.make_dual(x, x), shift, c)
+    with pytest.raises(RuntimeError, match="functorch"):
+        torch.func.vmap(lambda x, s: fused.shift_lerp(x, s, c))(x[None], shift[None])
+
+
+@pytest.mark.parametrize("dtype", [bf, torch.float32])
+def test_layer_refuses_a_tangent(dtype):
+    m = TimeMix(256, 2, 6, backend="cuda").cuda().to(dtype).requires_grad_(False)
+    x = torch.randn(1, 40, 256, device="cuda", dtype=bf)
+    with torch.autocast("cuda", dtype=bf), torch.autograd.forward_ad.dual_level():
+        with pytest.raises(NotImplementedError, match="jvp"):
+            m(torch.autograd.forward_ad.make_dual(x, x))
