@@ -209,8 +209,7 @@ class TimeMix(nn.Module):
             from . import fused
             coefs = [getattr(self, "x_" + n) for n in "rwkvag"]
             vecs = (self.w0, self.a0, self.k_k, self.k_a, self.r_k, self.ln_x.weight, self.ln_x.bias)
-            nograd = not (torch.is_grad_enabled() and (x.requires_grad or state["shift"].requires_grad
-                                                       or any(p.requires_grad for p in self.parameters())))
+            nograd = fused._direct(x, state["shift"], *coefs, *vecs)
             if nograd and fused._store is None and any(p.dtype != torch.float32 for p in (*coefs, *vecs)):
                 # the kernels' float32 parameters, made for this call in one launch (a serving
                 # loop's store keeps its own copies)

@@ -115,3 +115,29 @@ def test_layer_refuses_a_tangent(dtype):
     with torch.autocast("cuda", dtype=bf), torch.autograd.forward_ad.dual_level():
         with pytest.raises(NotImplementedError, match="jvp"):
             m(torch.autograd.forward_ad.make_dual(x, x))
+
+
+@pytest.mark.parametrize("dtype", [bf, torch.float32])
+@pytest.mark.parametrize("name", ["w0", "a0", "x_r", "k_k"])
+def test_gradient_of_a_tensor_in_a_parameter_s_place(name, dtype):
+    """A layer whose parameters need no gradient, one of them replaced by a tensor that does (a
+    generated one): the gradient that the parameter itself would get."""
+    torch.manual_seed(0)
+    m = TimeMix(256, 2, 6, backend="cuda")
+    with torch.no_grad():
+        for n, p in m.named_parameters():
+            if n in ("w1", "a1", "g1", "output.weight"):
+                p.normal_(0, .05)
+    m = m.cuda().to(dtype)
+    x = torch.randn(2, 100, 256, device="cuda", dtype=bf)  # (200 rows: past the few-row products)
+
+    def grad(of):
+        with torch.autocast("cuda", dtype=bf):
+            out, _ = m(x)
+        return torch.autograd.grad(out, of, torch.ones_like(out))[0]
+
+    want = grad(getattr(m, name))
+    t = getattr(m, name).detach().clone().requires_grad_()
+    delattr(m.requires_grad_(False), name)
+    setattr(m, name, t)
+    assert torch.equal(grad(t), want) and want.abs().max() > 0
