@@ -94,7 +94,8 @@ __global__ __launch_bounds__(W) void seq_forward(
         S[e] = keep(lane_mask(ok), s0[bh * NN + (ok ? i * ei + (j0 + e) * ej : 0)]);
     }
     // the 16 steps of a segment, loaded raw a segment ahead (clamped addresses, masked when
-    // they go to LDS: steps past the end get d = 1 and zeros, which leave the state as it is)
+    // they go to LDS: steps past the end get d = 1 and zeros, which leave the state as it is,
+    // with S a taken as zero there: an infinite state times a's zeros is not)
     float raw[5][M], rawv[MV];
     auto load = [&](int t0) {
 #pragma unroll
@@ -150,7 +151,7 @@ __global__ __launch_bounds__(W) void seq_forward(
             const float4 k4 = *reinterpret_cast<const float4*>(&vec[buf][2][u][j0]);
             const float4 r4 = *reinterpret_cast<const float4*>(&vec[buf][0][u][j0]);
             const float vi = vrow[buf][u][rl];
-            const float sa = row_lanes_sum<G>(dot4(S, a4));
+            const float sa = keep(t0 + u < Tn ? ~0u : 0u, row_lanes_sum<G>(dot4(S, a4)));
             S[0] = S[0] * d4.x + (sa * b4.x + vi * k4.x);
             S[1] = S[1] * d4.y + (sa * b4.y + vi * k4.y);
             S[2] = S[2] * d4.z + (sa * b4.z + vi * k4.z);
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(W) void seq_grad_scan(
             const float4 a4 = *reinterpret_cast<const float4*>(&vec[buf][2][u][j0]);
             const float dyi = vrow[buf][u][rl];
             g[0] += dyi * r4.x, g[1] += dyi * r4.y, g[2] += dyi * r4.z, g[3] += dyi * r4.w;
-            const float q = row_lanes_sum<G>(dot4(g, b4));
+            const float q = keep(c * CKPT + u < Tn ? ~0u : 0u, row_lanes_sum<G>(dot4(g, b4)));  // (as the forward's S a)
             g[0] = g[0] * d4.x + q * a4.x;
             g[1] = g[1] * d4.y + q * a4.y;
             g[2] = g[2] * d4.z + q * a4.z;
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(seq_bwd_lanes<NP>()) void seq_backward(
             const float4 a4 = *reinterpret_cast<const float4*>(&sm.a[u][j0]);
             const float dyi = sm.dy[u][i], vi = sm.v[u][i], sa = sm.sa[u][rl];
             g[0] += dyi * r4.x, g[1] += dyi * r4.y, g[2] += dyi * r4.z, g[3] += dyi * r4.w;
-            const float q = row_lanes_sum<G>(dot4(g, b4));
+            const float q = keep(t0 + u < Tn ? ~0u : 0u, row_lanes_sum<G>(dot4(g, b4)));  // (as seq_grad_scan's)
             const float dvi = row_lanes_sum<G>(dot4(g, k4));
             if (u % G == G - 1 || u == CKPT - 1) dvs[u / G] = dvi;
             else dvs[u / G] = kg == u % G ? dvi : dvs[u / G];

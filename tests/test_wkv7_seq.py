@@ -103,3 +103,33 @@ def test_infinite_inputs_stay_in_their_columns():
         ref = [*O.forward(*arr, s0), *O.backward(*arr, s0, dy, dsT)]
     for name, g, r in zip(NAMES, got, ref):
         assert np.array_equal(np.isfinite(g.double().cpu().numpy()), np.isfinite(r)), name
+
+
+@pytest.mark.filterwarnings("ignore::RuntimeWarning")
+@pytest.mark.parametrize("T", [1, 3, 16, 17, 31])
+@pytest.mark.parametrize("N", [32, 64, 128])
+def test_infinities_in_the_last_segment(N, T):
+    """The steps past the end of a sequence leave an infinite state (an infinite key at the last
+    step) and an infinite dL/dsT as they are: the float64 oracle's pattern of finite values, and
+    the finite ones at their usual bar."""
+    ext = W.extension()
+    inp = wkv7_inputs(1, T, 2, N, seed=3, dtype=torch.float32, s0_std=.3, with_dsT=True)
+    inf = {n: x.clone() for n, x in inp.items() if torch.is_tensor(x)}
+    inf["k"][0, T - 1, 0, 7] = float("inf")
+    inf["dsT"][0, 0, 3, 5] = float("inf")
+
+    def run(a, dsT):
+        xs, s0, dy = [a[n] for n in "rwkvab"], a["s0"], inp["dy"]
+        y, sT, saved = ext.forward(*[x.cuda() for x in (*xs, s0)], True)
+        got = [y, sT, *ext.backward(*[x.cuda() for x in xs], saved, dy.cuda(), dsT.cuda())]
+        arr = [x.double().numpy() for x in (*xs, s0)]
+        with np.errstate(all="ignore"):
+            ref = [*O.forward(*arr), *O.backward(*arr, dy.double().numpy(), dsT.double().numpy())]
+        return [g.double().cpu().numpy() for g in got], ref
+
+    for part, (got, ref) in ((slice(0, 2), run(inf, inp["dsT"])), (slice(2, 9), run(inp, inf["dsT"]))):
+        for name, g, r in zip(NAMES[part], got[part], ref[part]):
+            ok = np.isfinite(r)
+            assert np.array_equal(np.isfinite(g), ok) and ok.any(), name
+            assert rel_l2(g[ok], r[ok]) <= FP32_BAR, name
+        assert not np.isfinite(ref[1 if part.start == 0 else 8]).all()
