@@ -55,19 +55,23 @@ struct Dims {
     std::vector<int64_t> saved() const { return {B, H, (int64_t)theseus_wkv7_checkpoint_count(T), N, N}; }
     int family() const { return theseus_wkv7_kernel_family(B, T, H, N, dt); }
 };
+bool env_is_1(const char* name) {
+    const char* e = std::getenv(name);
+    return e && std::strcmp(e, "1") == 0;
+}
 // Extension._warn_fallback: a warning (or, THESEUS_WKV7_STRICT=1, an error) when a call runs
-// on the step-serial kernels without having asked for them
+// on the step-serial kernels without having asked for them.  The warning names the caller of
+// theseus.wkv7.wkv7 (three frames up: this function, wkv7, the caller).
 void warn_fallback(const Dims& d, int family) {
     if (family != THESEUS_WKV7_FAMILY_FP32 && family != THESEUS_WKV7_FAMILY_HEAD_SIZE &&
         family != THESEUS_WKV7_FAMILY_SIZE)
         return;
     py::gil_scoped_acquire gil;
-    py::module_::import("theseus.wkv7").attr("extension")().attr("_warn_fallback")(d.B, d.T, d.H, d.N, d.dt);
+    py::module_::import("theseus.wkv7").attr("extension")().attr("_warn_fallback")(d.B, d.T, d.H, d.N, d.dt, 3);
 }
 // THESEUS_WKV7_CHECK_WAITS=1 (Extension._check_waits)
 void check_waits() {
-    const char* e = std::getenv("THESEUS_WKV7_CHECK_WAITS");
-    if (!e || std::strcmp(e, "1") != 0) return;
+    if (!env_is_1("THESEUS_WKV7_CHECK_WAITS")) return;
     unsigned int n = 0;
     raise_status(theseus_wkv7_wait_timeouts(&n, 1), "theseus_wkv7");
     TORCH_CHECK(n == 0, "theseus_wkv7: ", n,
@@ -132,7 +136,8 @@ struct Wkv7 : torch::autograd::Function<Wkv7> {
         variable_list o(7);
         for (int i = 0; i < 6; i++) o[i] = at::empty_like(r);
         o[6] = at::empty({d.B, d.H, d.N, d.N}, saved.options());
-        warn_fallback(d, family);
+        // (the forward of these sizes has warned, and the engine's thread has no caller to name)
+        if (env_is_1("THESEUS_WKV7_STRICT")) warn_fallback(d, family);
         const size_t need = theseus_wkv7_backward_workspace_size(d.B, d.T, d.H, d.N, d.dt);
         const Tensor ws = scratch(need, r);
         raise_status(theseus_wkv7_backward(d.B, d.T, d.H, d.N, d.dt, ptr(r), ptr(s[1]), ptr(s[2]), ptr(s[3]), ptr(s[4]),

@@ -161,7 +161,7 @@ class Extension:
         """theseus_wkv7_family code of a call (0: chunked MFMA kernels)."""
         return int(self.lib.theseus_wkv7_kernel_family(B, T, H, N, dtype))
 
-    def _warn_fallback(self, B, T, H, N, dt):
+    def _warn_fallback(self, B, T, H, N, dt, stacklevel=4):
         """Say so when a call runs on the step-serial kernels (exact, but one step at a
         time: 6.6x slower than the chunked kernels at B=4, T=2048, H=80).  THESEUS_WKV7_STRICT=1
         turns the warning into an error; THESEUS_WKV7_FAMILY=seq (an explicit request)
@@ -173,7 +173,7 @@ class Extension:
                f"(B={B} T={T} H={H} N={N}); bf16 with N=64 or N=128 runs on the chunked MFMA kernels")
         if os.environ.get("THESEUS_WKV7_STRICT", "") == "1":
             raise RuntimeError(msg)
-        warnings.warn(msg, RuntimeWarning, stacklevel=4)
+        warnings.warn(msg, RuntimeWarning, stacklevel=stacklevel)
 
     def _layout(self, B, T, H, N, dt, flags):
         """Order of the saved states a forward writes: "tiled" on the chunked kernels

@@ -1,6 +1,8 @@
 """theseus._native: the operator's autograd functions as native torch nodes against the Python
 functions that they stand in for (the same kernels, so the same bits), their checks, and the
 calls that stay with the Python functions."""
+import warnings
+
 import pytest
 import torch
 
@@ -148,3 +150,24 @@ def test_forward_mode_is_refused_by_the_python_functions():
         r = torch.autograd.forward_ad.make_dual(xs[0], torch.ones_like(xs[0]))
         with pytest.raises(NotImplementedError, match="jvp"):
             W.wkv7(r, *xs[1:])
+
+
+@pytest.mark.gpu
+def test_fallback_warning_names_the_caller(monkeypatch):
+    """A float32 call warns once, at the line that calls the operator, with gradients and without;
+    its backward does not warn again (strict mode still refuses there)."""
+    xs, dy, _ = _case(1, 5, 2, 64, torch.float32)
+    for grad in (True, False):
+        a = [x.clone().requires_grad_(grad) for x in xs]
+        with warnings.catch_warnings(record=True) as seen:
+            warnings.simplefilter("always")
+            y, _ = W.wkv7(*a)
+        assert [w.filename for w in seen] == [__file__] and "step-serial" in str(seen[0].message)
+        if grad:
+            with warnings.catch_warnings():
+                warnings.simplefilter("error")
+                torch.autograd.grad(y, a, dy, retain_graph=True)
+            monkeypatch.setenv("THESEUS_WKV7_STRICT", "1")
+            with pytest.raises(RuntimeError, match="step-serial"):
+                torch.autograd.grad(y, a, dy)
+            monkeypatch.delenv("THESEUS_WKV7_STRICT")
