@@ -67,6 +67,15 @@ def l2norm(x, dim=-1, eps=1e-6):
     return x * torch.rsqrt((x * x).sum(dim=dim, keepdim=True) + eps)
 
 
+def _kept(x, io, normalised):
+    """x as the kernels take it and the backward keeps it.  A program may change a bfloat16
+    query, key or value in place after the call (and a float32 query or key that is
+    normalised), as after transformers' functions, which compute from float32 copies: those
+    get a copy, unless autograd forbids such changes anyway (leaves that need gradients)."""
+    y = x.to(io).contiguous()
+    return y.clone() if y is x and (normalised or io != torch.float32) and not (x.is_leaf and x.requires_grad) else y
+
+
 def gated_delta_rule(query, key, value, g, beta, initial_state=None, output_final_state=False,
                      use_qk_l2norm_in_kernel=False):
     """query, key [B,T,H,K]; value [B,T,H,V]; g, beta [B,T,H]; initial_state [B,H,K,V]
@@ -97,7 +106,8 @@ def gated_delta_rule(query, key, value, g, beta, initial_state=None, output_fina
         # take bf16 or fp32 q/k/v as they are and normalise q and k themselves (float32 inside)
         io = query.dtype if query.dtype == key.dtype == value.dtype and query.dtype in (torch.bfloat16, torch.float32) \
             else torch.float32
-        q, k, v = (x.to(io).contiguous() for x in (query, key, value))
+        q, k, v = (_kept(x, io, copied) for x, copied in (
+            (query, use_qk_l2norm_in_kernel), (key, use_qk_l2norm_in_kernel), (value, False)))
         gf, bf = g.float().contiguous(), beta.float().contiguous()
         native = _native(q, k, v, gf, bf, s0)
         o, sT = (_GDN.apply if native is None else native.gdn)(q, k, v, gf, bf, s0, use_qk_l2norm_in_kernel)

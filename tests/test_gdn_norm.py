@@ -60,3 +60,22 @@ def test_training_pair_with_normalisation(B, T, H, dtype):
             bar = max(bar, 1.25 * rel_l2(plain[3].grad, b))
         assert a.dtype == (dtype if name in ("o", "dq", "dk", "dv") else torch.float32)
         assert rel_l2(a, b) <= bar, (name, rel_l2(a, b))
+
+
+@pytest.mark.parametrize("dtype,norm,changed", [(torch.bfloat16, True, (0, 1, 2)), (torch.bfloat16, False, (0, 1, 2)),
+                                                (torch.float32, True, (0, 1)), (torch.float16, True, (0, 1, 2))])
+def test_inputs_changed_in_place_after_the_call(dtype, norm, changed):
+    """What the call computed from copies before it normalised inside the kernels may still be
+    changed between the call and its backward; the gradients are of the values at the call."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    B, T, H, N = 1, 33, 2, 128
+    leaves = [rnd(B, T, H, N).to(dtype).requires_grad_() for _ in range(3)]
+    rest, do, grads = [-rnd(B, T, H).exp(), rnd(B, T, H).sigmoid()], rnd(B, T, H, N).to(dtype), []
+    for change in (False, True):
+        qkv = [x * 1 for x in leaves]
+        o, _ = G.chunk_gated_delta_rule(*qkv, *rest, use_qk_l2norm_in_kernel=norm)
+        for i in changed if change else ():
+            qkv[i].mul_(2)
+        grads.append(torch.autograd.grad(o, leaves, do))
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
