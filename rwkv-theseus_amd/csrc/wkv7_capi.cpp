@@ -109,13 +109,22 @@ static bool split_ok(const Fwd& p) {
 // the host 125 us through autograd, the chunked kernels' four 100 (T=272 8 heads 124 against
 // 101, T=400 44 heads 124 against 119, T=512 52 heads 128 against 147).  The saved states are
 // the chunked kernels' (tiled), so each direction decides by itself: the forward when the
-// workspace holds the records (forward_workspace_best), the backward by its own size.
+// workspace holds the records (forward_workspace_best), the backward likewise.  Their records and
+// dL/dS (23 KB forward, 35 KB backward per chunk and head, where the chunked kernels need
+// nothing) are bounded: past 1 GiB the chunked kernels keep the call (40 heads: from some
+// 12000 tokens).
+constexpr size_t kRec64WorkspaceBytes = (size_t)1 << 30;
 static bool rec64_shape(int B, int T, int H, int N, int dtype, int flags) {
     if (!chunk_ok(B, T, H, N, dtype, flags) || (long long)B * H > 65535 ||
         wkv7_rec_workspace(1, T, 1, N) >= (1ull << 32))
         return false;
     const long long n = (T + kCkptInterval - 1) / kCkptInterval, cus = cu_count(), BH = (long long)B * H;
-    return n > 28 && BH <= cus / 4 && (3 * cus / 10 - BH) * n > 760;
+    return n > 28 && BH <= cus / 4 && (3 * cus / 10 - BH) * n > 760 &&
+           wkv7_rec_bwd_workspace(B, T, H, N, (int)cus) <= kRec64WorkspaceBytes;
+}
+static bool rec64_ok(const Bwd& p) {
+    return rec64_shape(p.B, p.T, p.H, p.N, p.dtype, p.flags) && p.ws &&
+           p.ws_bytes >= wkv7_rec_bwd_workspace(p.B, p.T, p.H, p.N, 0);
 }
 static bool rec64_ok(const Fwd& p) {
     return p.ckpt && rec64_shape(p.B, p.T, p.H, p.N, p.dtype, p.flags) && p.ws &&
@@ -136,7 +145,7 @@ void launch_forward(const Fwd& p) {
     else launch_seq_forward(p);
 }
 void launch_backward(const Bwd& p) {
-    if (rec64_shape(p.B, p.T, p.H, p.N, p.dtype, p.flags)) launch_wkv7_rec_backward(p, cu_count());
+    if (rec64_ok(p)) launch_wkv7_rec_backward(p, cu_count());
     else if (chunk_ok(p.B, p.T, p.H, p.N, p.dtype, p.flags)) launch_chunk_backward(p, cu_count());
     else if (rec_shape(p.B, p.T, p.H, p.N, p.dtype, p.flags)) launch_wkv7_rec_backward(p, cu_count());
     else launch_seq_backward(p);
@@ -163,6 +172,11 @@ size_t backward_workspace(int B, int T, int H, int N, int dtype, int flags) {
     if (rec64_shape(B, T, H, N, dtype, flags)) return wkv7_rec_bwd_workspace(B, T, H, N, cu_count());
     if (chunk_ok(B, T, H, N, dtype, flags)) return chunk_backward_workspace(B, T, H, cu_count());
     if (rec_shape(B, T, H, N, dtype, flags)) return wkv7_rec_bwd_workspace(B, T, H, N, cu_count());
+    return seq_backward_workspace(B, T, H, N);
+}
+size_t backward_workspace_least(int B, int T, int H, int N, int dtype, int flags) {
+    if (chunk_ok(B, T, H, N, dtype, flags)) return chunk_backward_workspace(B, T, H, cu_count());
+    if (rec_shape(B, T, H, N, dtype, flags)) return wkv7_rec_bwd_workspace(B, T, H, N, 0);
     return seq_backward_workspace(B, T, H, N);
 }
 
@@ -263,11 +277,12 @@ int theseus_wkv7_backward_ex(int B, int T, int H, int N, int dtype, int flags, c
     if (!r || !w || !k || !v || !a || !b || !ckpt || !dy || !dr || !dw || !dk || !dv || !da ||
         !db || !ds0)
         return THESEUS_WKV7_ERR_NULL;
-    const size_t need = wkv7::backward_workspace(B, T, H, N, dtype, flags);
+    const size_t need = wkv7::backward_workspace_least(B, T, H, N, dtype, flags);
     if (workspace_bytes < need || (need && !workspace)) return THESEUS_WKV7_ERR_WORKSPACE;
     wkv7::Bwd p{B, T, H, N, dtype, r, w, k, v, a, b, ckpt, dy, dsT,
                 dr, dw, dk, dv, da, db, ds0, workspace, stream};
     p.flags = flags;
+    p.ws_bytes = workspace_bytes;
     wkv7::launch_backward(p);
     return launch_status();
 }
@@ -359,10 +374,11 @@ int theseus_gdn_backward_ex(int B, int T, int H, int N, int dtype, int qk_l2norm
     if (dtype != THESEUS_WKV7_BF16 && dtype != THESEUS_WKV7_FP32) return THESEUS_WKV7_ERR_DTYPE;
     if (!q || !k || !v || !g || !beta || !ckpt || !dout || !dq || !dk || !dv || !dg || !dbeta || !ds0)
         return THESEUS_WKV7_ERR_NULL;
-    if (!workspace || workspace_bytes < wkv7::gdn_backward_workspace(B, T, H, wkv7::cu_count())) return THESEUS_WKV7_ERR_WORKSPACE;
+    if (!workspace || workspace_bytes < wkv7::gdn_backward_workspace(B, T, H, 0)) return THESEUS_WKV7_ERR_WORKSPACE;
     wkv7::GdnBwd p{B, T, H, N, dtype, q, k, v, g, beta, ckpt, dout, dsT, dq, dk, dv, dg, dbeta, ds0, workspace, stream};
     p.cus = wkv7::cu_count();
     p.qk_norm = qk_l2norm ? 1 : 0;
+    p.ws_bytes = workspace_bytes;
     wkv7::launch_gdn_backward(p);
     return launch_status();
 }

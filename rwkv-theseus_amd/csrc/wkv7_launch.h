@@ -37,6 +37,7 @@ struct Bwd {
     void* ws;
     hipStream_t stream;
     int flags = 0;
+    size_t ws_bytes = 0;  // bytes at ws (at least backward_workspace_least)
 };
 
 struct Dec {
@@ -105,8 +106,9 @@ struct GdnBwd {
     hipStream_t stream;
     int cus = 0;  // CUs the reverse scan's time split may fill
     int qk_norm = 0;
+    size_t ws_bytes = 0;  // bytes at ws (at least gdn_backward_workspace with cus = 0)
 };
-size_t gdn_backward_workspace(int B, int T, int H, int cus);
+size_t gdn_backward_workspace(int B, int T, int H, int cus);  // (cus = 0: the least, no time split)
 void launch_gdn_backward(const GdnBwd& p);
 // the operand records (the least a call needs); with the time split's buffers when it
 // applies (gdn_split_segments >= 2)
@@ -126,8 +128,8 @@ size_t wkv7_rec_workspace_fast(int B, int T, int H, int N, int cus);
 size_t wkv7_rec_train_workspace(int B, int T, int H, int N, int cus);
 void launch_wkv7_rec_forward(const Fwd& p, int cus);
 // Its backward (wkv7_rec_bwd.hip), every chunk at once from the saved states: a workspace
-// of wkv7_rec_bwd_workspace bytes (the scan's records, dL/dS at every chunk's end, the
-// reverse scan's time split).
+// of wkv7_rec_bwd_workspace bytes (the scan's records, dL/dS at every chunk's end, the chunks'
+// matrices, the reverse scan's time split; cus = 0: the least, without the split).
 size_t wkv7_rec_bwd_workspace(int B, int T, int H, int N, int cus);
 void launch_wkv7_rec_backward(const Bwd& p, int cus);
 
@@ -140,6 +142,8 @@ size_t forward_workspace(int B, int T, int H, int N, int dtype, int flags = 0);
 size_t forward_workspace_fast(int B, int T, int H, int N, int dtype, int flags = 0);
 // forward_workspace, or more where a forward (with saved states or without) runs faster given more
 size_t forward_workspace_best(int B, int T, int H, int N, int dtype, bool saved);
+// what a backward runs fastest with, and what it accepts
 size_t backward_workspace(int B, int T, int H, int N, int dtype, int flags = 0);
+size_t backward_workspace_least(int B, int T, int H, int N, int dtype, int flags = 0);
 
 }  // namespace wkv7

@@ -1216,34 +1216,41 @@ __global__ __launch_bounds__(512, sizeof(TI) == 2 ? 4 : 2) void gdn_bwd_chunk(
 
 }  // namespace
 
-// Workspace: the scan's records, H = dL/dS at every chunk's end, the time split's buffers.
+// Workspace: the scan's records, H = dL/dS at every chunk's end, (WKV7) the chunks' matrices, and
+// the time split's buffers (cus = 0: without them).
 template <int NK> static size_t bwd_records(size_t chunks) { return (chunks * BwdRec<NK>::BYTES + 255) / 256 * 256; }
-template <int NK> static size_t bwd_workspace(int B, int T, int H, int cus) {
+static size_t mats_bytes(size_t chunks) { return chunks * MATS * 64 * sizeof(uint4); }
+template <int NK> static size_t split_at(size_t chunks, bool mats) {
+    return bwd_records<NK>(chunks) + chunks * NK * NK * sizeof(float) + (mats ? mats_bytes(chunks) : 0);
+}
+template <int NK> static size_t bwd_workspace(int B, int T, int H, int cus, bool mats) {
     const int n = (T + BC - 1) / BC;
     const size_t BH = (size_t)B * H;
-    return bwd_records<NK>(BH * n) + BH * n * NK * NK * sizeof(float) +
-           resume_bytes(BH, NK, resume_segments(BH, NK, n, cus));
+    return split_at<NK>(BH * n, mats) + resume_bytes(BH, NK, resume_segments(BH, NK, n, cus));
 }
-// (WKV7: and the chunks' matrices behind them)
 size_t wkv7_rec_bwd_workspace(int B, int T, int H, int N, int cus) {
-    const size_t mats = (size_t)B * H * ((T + BC - 1) / BC) * MATS * 64 * sizeof(uint4);
-    return mats + (N == 64 ? bwd_workspace<64>(B, T, H, cus) : bwd_workspace<128>(B, T, H, cus));
+    return N == 64 ? bwd_workspace<64>(B, T, H, cus, true) : bwd_workspace<128>(B, T, H, cus, true);
 }
-// The reverse scan over the records at ws, in one pass or in time segments.
+// The reverse scan over the records at ws, in one pass or in as many time segments as cus and
+// the ws_bytes behind the records, H and (mats) matrices allow.
 template <int NK, typename TI>
 static const float* scan_back(int T, int H, int BH, int kv, const float* dsT, const void* dy, float* ds0, void* ws,
-                              int cus, hipStream_t stream) {
-    const int n = (T + BC - 1) / BC, k = resume_segments(BH, NK, n, cus);
+                              size_t ws_bytes, bool mats, int cus, hipStream_t stream) {
+    const int n = (T + BC - 1) / BC;
+    const size_t chunks = (size_t)BH * n, at = split_at<NK>(chunks, mats);
+    int k = resume_segments(BH, NK, n, cus);
+    while (k >= 4 && at + resume_bytes(BH, NK, k) > ws_bytes) k--;
+    if (k < 4) k = 1;
     const int rgs = k < 2 ? NK / 64 : scan_groups(BH, NK, k - 1, cus), lanes = 4 * NK / rgs;
     const uint8_t* const recs = static_cast<const uint8_t*>(ws);
-    float* const hbuf = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + bwd_records<NK>((size_t)BH * n));
+    float* const hbuf = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + bwd_records<NK>(chunks));
     const TI* const y = static_cast<const TI*>(dy);
     if (k < 2) {
         hipLaunchKernelGGL((wkv7_bwd_scan<NK, TI, SCAN_ALL>), dim3(BH * rgs), dim3(lanes), 0, stream, T, H, BH, kv, dsT, y,
                            ds0, hbuf, recs, ScanSplit{});
         return hbuf;
     }
-    const ScanSplit sp = resume_split(BH, NK, n, k, hbuf + (size_t)BH * n * NK * NK);
+    const ScanSplit sp = resume_split(BH, NK, n, k, reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + at));
     hipLaunchKernelGGL((wkv7_bwd_scan<NK, TI, SCAN_ENDS>), dim3((k - 1) * BH * rgs), dim3(lanes), 0, stream, T, H, BH, kv,
                        dsT, y, ds0, hbuf, recs, sp);
     hipLaunchKernelGGL((scan_chain<NK>), dim3(BH, NK / 16), dim3(4 * NK), 0, stream, BH, k - 2, kv, sp, nullptr);
@@ -1258,11 +1265,11 @@ template <int NK> static void launch_rec_bwd(const Bwd& p, int cus) {
                  *k = static_cast<const bf16_t*>(p.k), *v = static_cast<const bf16_t*>(p.v),
                  *a = static_cast<const bf16_t*>(p.a), *b = static_cast<const bf16_t*>(p.b),
                  *dy = static_cast<const bf16_t*>(p.dy);
-    uint4* const mats =
-        reinterpret_cast<uint4*>(static_cast<uint8_t*>(p.ws) + bwd_workspace<NK>(p.B, p.T, p.H, cus));
+    uint4* const mats = reinterpret_cast<uint4*>(static_cast<uint8_t*>(p.ws) + split_at<NK>((size_t)BH * nchunk, false));
     hipLaunchKernelGGL(wkv7_bwd_prep<NK>, dim3(nchunk, BH), dim3(64), 0, p.stream, p.T, p.H, r, w, k, a, b,
                        static_cast<uint8_t*>(p.ws), mats);
-    const float* const hbuf = scan_back<NK, bf16_t>(p.T, p.H, BH, 0, p.dsT, dy, p.ds0, p.ws, cus, p.stream);
+    const float* const hbuf = scan_back<NK, bf16_t>(p.T, p.H, BH, 0, p.dsT, dy, p.ds0, p.ws, p.ws_bytes, true, cus,
+                                                  p.stream);
     const int jobs = nchunk * BH, per_xcd = (jobs + 7) / 8;
     hipLaunchKernelGGL(wkv7_bwd_chunk<NK>, dim3(8 * per_xcd), dim3(4 * NK), 0, p.stream, p.T, p.H, BH, per_xcd, r, w, k,
                        v, a, b, dy, p.ckpt, hbuf, mats, static_cast<bf16_t*>(p.dr), static_cast<bf16_t*>(p.dw),
@@ -1274,7 +1281,7 @@ void launch_wkv7_rec_backward(const Bwd& p, int cus) {
     else launch_rec_bwd<128>(p, cus);
 }
 
-size_t gdn_backward_workspace(int B, int T, int H, int cus) { return bwd_workspace<BNK>(B, T, H, cus); }
+size_t gdn_backward_workspace(int B, int T, int H, int cus) { return bwd_workspace<BNK>(B, T, H, cus, false); }
 
 template <typename TI>
 static void launch_gdn_bwd(const GdnBwd& p) {
@@ -1283,7 +1290,8 @@ static void launch_gdn_bwd(const GdnBwd& p) {
              *dout = static_cast<const TI*>(p.dout);
     hipLaunchKernelGGL(gdn_bwd_prep<TI>, dim3(nchunk, BH), dim3(64), 0, p.stream, p.T, p.H, p.qk_norm, q, k,
                        p.g, p.beta, static_cast<uint8_t*>(p.ws));
-    const float* const hbuf = scan_back<BNK, TI>(p.T, p.H, BH, 1, p.dsT, dout, p.ds0, p.ws, p.cus, p.stream);
+    const float* const hbuf = scan_back<BNK, TI>(p.T, p.H, BH, 1, p.dsT, dout, p.ds0, p.ws, p.ws_bytes, false, p.cus,
+                                             p.stream);
     const int jobs = nchunk * BH, per_xcd = (jobs + 7) / 8;
     hipLaunchKernelGGL(gdn_bwd_chunk<TI>, dim3(8 * per_xcd), dim3(512), 0, p.stream, p.T, p.H, BH, per_xcd,
                        p.qk_norm, q, k, v, p.g, p.beta, dout, p.ckpt, hbuf, static_cast<TI*>(p.dq), static_cast<TI*>(p.dk),

@@ -292,3 +292,20 @@ def test_gdn_abi_exported_bound_and_validated():
     assert lib.theseus_gdn_backward(1, 4, 1, 64, 1, *[None] * 14, None, 0, None) == 1
     assert lib.theseus_gdn_backward(1, 4, 1, 128, 5, *[None] * 14, None, 0, None) == 2
     assert lib.theseus_gdn_backward(1, 4, 1, 128, 1, *[None] * 14, None, 0, None) == 3
+
+
+def test_few_heads_training_workspace_is_bounded(monkeypatch):
+    """N = 64 training with few heads on the chunk-record kernels stays within 1 GiB each way;
+    longer calls keep the chunked kernels, which need nothing."""
+    monkeypatch.setenv("THESEUS_WKV7_CUS", "256")
+    lib, seen = W.extension().lib, set()
+    for H in (1, 8, 40, 64):
+        for T in (1021, 4096, 8192, 12288, 32768, 65536, 131072):
+            f = lib.theseus_wkv7_forward_best_workspace_size(1, T, H, 64, 0, 1)
+            b = lib.theseus_wkv7_backward_workspace_size(1, T, H, 64, 0)
+            plain = lib.theseus_wkv7_forward_workspace_size(1, T, H, 64, 0)
+            assert b <= 2 ** 30 and (f == plain or f <= 2 ** 30) and (b > 0) == (f > plain or f >= 22784 * H * T // 16)
+            seen.add(b > 0)
+    assert seen == {False, True}
+    assert lib.theseus_wkv7_backward_workspace_size(1, 65536, 40, 64, 0) == 0
+    assert lib.theseus_wkv7_backward_workspace_size(1, 8192, 40, 64, 0) > 0

@@ -89,3 +89,33 @@ def test_few_heads_at_the_ends_of_the_decay_range(mode):
             assert np.all(np.abs(g.detach().double().cpu().numpy() - r) <= 2e-2 + 2.0 ** -7 * np.abs(r))
         else:
             _check(name, g, r, torch.bfloat16)
+
+
+@pytest.mark.parametrize("N", [64, 128])
+def test_backward_by_the_workspace_it_is_given(N, monkeypatch):
+    """The backward takes what a call brings: nothing at N = 64 (the chunked kernels), the records
+    and dL/dS alone (one pass), fewer segments than the most, all of them."""
+    monkeypatch.setenv("THESEUS_WKV7_CUS", "256")
+    B, T, H = 1, 600, 3
+    lib, ext, n = W.extension().lib, W.extension(), 38
+    inp = wkv7_inputs(B, T, H, N, seed=9, dtype=torch.bfloat16, s0_std=.1, with_dsT=True)
+    xs, s0, dy, dsT = [inp[i].cuda() for i in "rwkvab"], inp["s0"].cuda(), inp["dy"].cuda(), inp["dsT"].cuda()
+    saved = ext.forward(*xs, s0, True)[2]
+    best = lib.theseus_wkv7_backward_workspace_size(B, T, H, N, 0)
+    record = {64: 12544, 128: 25088}[N] + 4 * N * N + 6 * 1024
+    least, state = B * H * n * record, B * H * N * N * 4
+    assert best == least + 15 * state  # (9 segments)
+    ref = ext.backward(*xs, saved, dy, dsT)
+    p = lambda t: t.data_ptr()  # noqa: E731
+    for size in ([0] if N == 64 else []) + [least, least + 5 * state, best]:
+        grads = [torch.empty_like(x) for x in xs] + [torch.empty_like(s0)]
+        ws = torch.empty((max(size, 1),), dtype=torch.uint8, device="cuda")
+        assert lib.theseus_wkv7_backward(B, T, H, N, 0, *map(p, (*xs, saved, dy, dsT, *grads)), p(ws) if size else None,
+                                         size, torch.cuda.current_stream().cuda_stream) == 0
+        for name, a, b in zip(NAMES[2:], grads, ref):
+            if size == best:
+                assert torch.equal(a, b), name
+            assert rel_l2(a, b) <= (1e-5 if name == "ds0" else 3e-3), (size, name)
+    if N == 128:  # (nothing else reads its saved states)
+        assert lib.theseus_wkv7_backward(B, T, H, N, 0, *map(p, (*xs, saved, dy, dsT, *grads)), p(ws), least - 1,
+                                         torch.cuda.current_stream().cuda_stream) == 4
