@@ -759,7 +759,7 @@ static void scan_records(int B, int T, int H, int kv, const float* s0, TO* o, fl
     const size_t rec_bytes = (records<PK>(B, T, H, NK) + 255) / 256 * 256;
     float* const base = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + rec_bytes);  // buffers after the records
     if (ckpt) {
-        int k = resume_segments(BH, NK, nchunk, cus);
+        int k = resume_segments(BH, NK, nchunk, cus, false);
         while (k >= 4 && rec_bytes + resume_bytes(BH, NK, k) > ws_bytes) k--;
         if (k >= 4) {
             const ScanSplit sp = resume_split(BH, NK, nchunk, k, base);
@@ -832,7 +832,7 @@ void launch_wkv7_rec_forward(const Fwd& p, int cus) {
 template <bool PK> static size_t train_workspace(int B, int T, int H, int N, int cus) {
     const size_t BH = (size_t)B * H;
     return (records<PK>(B, T, H, N) + 255) / 256 * 256 +
-           resume_bytes(BH, N, resume_segments(BH, N, (T + GC - 1) / GC, cus));
+           resume_bytes(BH, N, resume_segments(BH, N, (T + GC - 1) / GC, cus, false));
 }
 size_t wkv7_rec_train_workspace(int B, int T, int H, int N, int cus) { return train_workspace<true>(B, T, H, N, cus); }
 size_t gdn_train_workspace(int B, int T, int H, int N, int cus) { return train_workspace<false>(B, T, H, N, cus); }

@@ -1226,7 +1226,7 @@ template <int NK> static size_t split_at(size_t chunks, bool mats) {
 template <int NK> static size_t bwd_workspace(int B, int T, int H, int cus, bool mats) {
     const int n = (T + BC - 1) / BC;
     const size_t BH = (size_t)B * H;
-    return split_at<NK>(BH * n, mats) + resume_bytes(BH, NK, resume_segments(BH, NK, n, cus));
+    return split_at<NK>(BH * n, mats) + resume_bytes(BH, NK, resume_segments(BH, NK, n, cus, true));
 }
 size_t wkv7_rec_bwd_workspace(int B, int T, int H, int N, int cus) {
     return N == 64 ? bwd_workspace<64>(B, T, H, cus, true) : bwd_workspace<128>(B, T, H, cus, true);
@@ -1238,7 +1238,7 @@ static const float* scan_back(int T, int H, int BH, int kv, const float* dsT, co
                               size_t ws_bytes, bool mats, int cus, hipStream_t stream) {
     const int n = (T + BC - 1) / BC;
     const size_t chunks = (size_t)BH * n, at = split_at<NK>(chunks, mats);
-    int k = resume_segments(BH, NK, n, cus);
+    int k = resume_segments(BH, NK, n, cus, true);
     while (k >= 4 && at + resume_bytes(BH, NK, k) > ws_bytes) k--;
     if (k < 4) k = 1;
     const int rgs = k < 2 ? NK / 64 : scan_groups(BH, NK, k - 1, cus), lanes = 4 * NK / rgs;

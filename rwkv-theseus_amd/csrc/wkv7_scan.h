@@ -131,13 +131,40 @@ __global__ __launch_bounds__(4 * NK) void scan_chain(int BH, int steps, int kv, 
 inline int scan_groups(long BH, int N, int segments, int cus) {
     return N / 64 > 1 && segments * BH * (N / 64) <= cus ? N / 64 : 1;
 }
-// Segments of the split with saved states: k - 1 workgroups per head in each launch, one per
-// CU, at most 9 segments of at least 4 chunks; worth it from 4 segments on (2 n / k ticks and
-// two more launches against n ticks).
-inline int resume_segments(long BH, int, int nchunk, int cus) {
-    const long k = cus / BH + 1;
-    const int fit = (int)(k < 9 ? k : 9), s = nchunk / 4 < fit ? nchunk / 4 : fit;
-    return s >= 4 ? s : 1;
+// Segments of the split with saved states (1: one pass), at most 9 of at least 4 chunks each:
+// k - 1 workgroups per head and row group in each of its two launches, one per CU.  A split
+// costs 2 n / k ticks, a chain of k - 2 steps and two more launches against n ticks, and its
+// ticks are longer than one pass's: all of a head's rows in one workgroup where N/64 row groups
+// per segment do not fit the CUs (128 keys: 4 to 5.5 us a tick against 2.2 with two groups,
+// one pass 1.5 to 2), and more records and states through memory at once.  So at 128 keys it is
+// cut as far as both row groups fit, and further only from 96 chunks on, where fewer chunks per
+// segment weigh more.  Forward with saved states | backward, whole calls at B = 1 in us, one
+// pass / k segments (MI355X, 256 CUs):
+//   heads   16 chunks              24                     48                      64                      128
+//    8      56/4: 53 | 59/4: 61    73/6: 61 | 73/6: 67    124/9: 83 | 123/9: 96   155/9: 86 | 149/9: 102  284/9: 124 | 279/9: 160
+//    32     60/4: 60 | 77/4: 80    77/5: 68 | 105/5: 101  132/5: 103 | 187/5: 176 171/5: 126 | 249/5: 233 370/9: 240 | 481/9: 422
+//    40     60/4: 68 | 90/4: 100   78/4: 88 | 118/4: 128  137/4: 127 | 218/4: 225 188/4: 168 | 290/4: 285 409/7: 293 | 562/7: 526
+//    56     63/4: 87 | 106/4: 126  84/5: 100 | 147/5: 169 160/5: 167 | 278/5: 303 236/5: 210 | 365/5: 384 460/5: 372 | 703/5: 694
+//    85     70/4: 104 | 142/4: 173 94/4: 135 | 206/4: 245 228/4: 228 | 385/4: 418 297/4: 287 | 501/4: 532 552/4: 533 | 932/4: 999
+// (32 heads, 48 chunks: one group's 9 segments 116 | 191.)  The backward, whose own work beside
+// the scan is larger, starts a little later.  The gated delta rule's calls lie within 3 % of
+// these lines.  At 64 keys (one row group always, and calls of more than 28 chunks only) every
+// split pays: 29 chunks 47/7: 36 | 43/7: 38 at 8 heads, 55/6: 47 | 69/6: 67 at 48.
+inline int resume_segments(long BH, int N, int nchunk, int cus, bool back) {
+    auto fit = [&](long groups) {
+        const long k = cus / (groups * BH) + 1, m = k < 9 ? k : 9;
+        return (int)(nchunk / 4 < m ? nchunk / 4 : m);
+    };
+    const int one = fit(1);  // with one workgroup per head and segment
+    if (N == 64) return one >= 4 && nchunk > 28 ? one : 1;
+    if (nchunk >= 96) return one >= (back ? 5 : 4) ? one : 1;
+    const int all = fit(N / 64);  // with every row group
+    const long room = cus / (N / 64 * BH) + 1;  // (before the chunks' and the most segments' limits)
+    if (room >= 4) {
+        const int from = room >= 9 ? 16 : room >= 5 ? 20 : 48;
+        return all >= 4 && nchunk >= from + (back ? room == 4 ? 16 : 4 : 0) ? all : 1;
+    }
+    return !back && nchunk >= 64 && one >= 4 ? one : 1;
 }
 // Chunks of segment 0 and of each later one: the first launch takes max(m0, 4/3 m) ticks
 // (two states on one record), the second m.

@@ -309,3 +309,30 @@ def test_few_heads_training_workspace_is_bounded(monkeypatch):
     assert seen == {False, True}
     assert lib.theseus_wkv7_backward_workspace_size(1, 65536, 40, 64, 0) == 0
     assert lib.theseus_wkv7_backward_workspace_size(1, 8192, 40, 64, 0) > 0
+
+
+def test_backward_record_scans_are_cut_where_it_pays(monkeypatch):
+    """Time segments of the reverse record scan at 128 keys on 256 CUs (1: one pass), read from the
+    workspace sizes, on both sides of every line of the rule; never more workgroups than CUs,
+    never a segment of less than four chunks."""
+    monkeypatch.setenv("THESEUS_WKV7_CUS", "256")
+    lib = W.extension().lib
+
+    def segments(H, n):
+        state, ks = H * 128 * 128 * 4, set()
+        for size, chunk in ((lib.theseus_wkv7_backward_workspace_size(1, 16 * n, H, 128, 0), 25088 + 65536 + 6144),
+                            (lib.theseus_gdn_backward_workspace_size(1, 16 * n, H, 128), 25088 + 65536)):
+            states, rest = divmod(size - H * n * chunk, state)  # 1 + 2 (k - 2) of them
+            assert rest == 0
+            ks.add((states - 1) // 2 + 2 if states else 1)
+        assert len(ks) == 1
+        return ks.pop()
+
+    for H, n, k in [(8, 19, 1), (8, 20, 5), (8, 64, 9), (16, 20, 5), (17, 23, 1), (17, 24, 6), (32, 23, 1), (32, 24, 5),
+                    (32, 95, 5), (32, 96, 9), (33, 63, 1), (40, 64, 4), (40, 96, 7), (43, 95, 1), (64, 96, 5),
+                    (65, 256, 1), (128, 256, 1)]:
+        assert segments(H, n) == k, (H, n)
+    for H in range(1, 140):
+        for n in (1, 7, 8, 16, 19, 20, 28, 47, 48, 64, 96, 200):
+            k = segments(H, n)
+            assert k == 1 or 4 <= k <= 9 and (k - 1) * H <= 256 and 4 * k <= n
