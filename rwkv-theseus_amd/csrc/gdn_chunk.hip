@@ -709,8 +709,9 @@ static size_t records(int B, int T, int H, int N) {
     return (size_t)B * H * ((T + GC - 1) / GC) * rec;
 }
 size_t gdn_forward_workspace(int B, int T, int H, int N) { return records<false>(B, T, H, N); }
-// Segments of the time-split scan: with at least 8 chunks, as many as fit one workgroup
-// per CU (B*H*N/64 per segment), at most 4, each with at least one chunk; 1 = no split.
+// Segments whose buffers the plain workspace sizes hold: with at least 8 chunks, one workgroup
+// per CU (B*H*N/64 per segment), at most 4, each with at least one chunk.  A call uses as many of
+// them as tiles_segments says.
 int gdn_split_segments(int B, int T, int H, int N, int cus) {
     const int n = (T + GC - 1) / GC, per = B * H * (N / 64);
     if (n < 8 || per < 1) return 1;
@@ -726,17 +727,36 @@ static size_t tiles_workspace(int B, int T, int H, int N, int k) {
     const size_t recs = (records<PK>(B, T, H, N) + 255) / 256 * 256;
     return recs + BH * ((2 * k - 1) * NN + 2 * (k - 1) * m * GC * N) * sizeof(float);
 }
-// As many segments as one workgroup of all of a head's rows per CU allows, at most 8; the
-// default workspace size holds the buffers of gdn_split_segments of them.
-static int tiles_segments(int B, int T, int H, int cus) {
-    const int n = (T + GC - 1) / GC;
-    return n < 8 ? 1 : max(1, min(min(8, cus / (B * H)), n));
+// Segments of the split without saved states (SCAN_TILES; 1: one pass), at most 8, one
+// workgroup per CU.  It replaces n ticks by n / k longer ones, k - 1 chain steps of 3 us, the
+// fix-up of the outputs and two launches, so short calls and many heads stay in one pass.  The
+// gated delta rule at B = 1 in us, one pass / k segments:
+//   keys heads   8 chunks     16            24            48            64             128
+//   128   16     28/8: 45     42/4: 45      57/6: 51      96/8: 63      121/8: 71      228/8: 96
+//   128   32     30/8: 50     46/4: 46      59/4: 54      100/4: 74     129/4: 87      251/8: 149
+//   128   40     32/6: 61     47/3: 56      59/3: 67      102/3: 90     133/3: 105     270/6: 195
+//   128   64     34/4: 54     47/4: 66      64/4: 76      114/4: 114    149/4: 145     318/4: 261
+//   128   128    37/2: 62     57/2: 83      78/2: 104     170/2: 189    221/2: 243     422/2: 469
+//    64   32     20/8: 26     31/4: 31      41/6: 35      67/8: 41      82/8: 46       153/8: 66
+//    64   85     25/3: 32     36/3: 37      43/3: 43      74/3: 63      96/3: 77       202/3: 160
+// So from 20 chunks on (64 keys and few heads: 16), at least 4 chunks a segment; at 128 keys as
+// many as leave room for both row groups, from 96 chunks on as many as one of all rows allows.
+static int tiles_segments(int B, int T, int H, int N, int cus) {
+    const int n = (T + GC - 1) / GC, BH = B * H;
+    const int one = min(8, cus / BH), all = min(8, cus / (N / 64 * BH));
+    if (n < (N == 64 && BH <= cus / 16 ? 16 : 20)) return 1;
+    if (N == 64) return one >= 4 ? min(one, n / 4) : n >= 48 ? max(1, one) : 1;
+    if (n >= 96) return one >= 4 ? one : 1;
+    if (all >= 4) return min(all, n / 4);
+    if (n < 48) return 1;
+    return all == 3 ? 3 : one >= 4 ? one : 1;
 }
 size_t gdn_forward_workspace_fast(int B, int T, int H, int N, int cus) {
-    return tiles_workspace<false>(B, T, H, N, tiles_segments(B, T, H, cus));
+    return tiles_workspace<false>(B, T, H, N, tiles_segments(B, T, H, N, cus));
 }
 size_t wkv7_rec_workspace_fast(int B, int T, int H, int N, int cus) {
-    return tiles_workspace<true>(B, T, H, N, tiles_segments(B, T, H, cus));
+    return max(tiles_workspace<true>(B, T, H, N, tiles_segments(B, T, H, N, cus)),
+               tiles_workspace<true>(B, T, H, N, gdn_split_segments(B, T, H, N, cus)));
 }
 size_t gdn_forward_workspace_split(int B, int T, int H, int N, int cus) {
     return tiles_workspace<false>(B, T, H, N, gdn_split_segments(B, T, H, N, cus));
@@ -772,7 +792,7 @@ static void scan_records(int B, int T, int H, int kv, const float* s0, TO* o, fl
             return;
         }
     }
-    int k = ckpt ? 1 : tiles_segments(B, T, H, cus);
+    int k = ckpt ? 1 : tiles_segments(B, T, H, NK, cus);
     while (k >= 2 && tiles_workspace<PK>(B, T, H, NK, k) > ws_bytes) k--;
     if (k < 2) {
         const int rgs = gdn_row_groups(NK);

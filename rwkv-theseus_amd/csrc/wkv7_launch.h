@@ -110,8 +110,8 @@ struct GdnBwd {
 };
 size_t gdn_backward_workspace(int B, int T, int H, int cus);  // (cus = 0: the least, no time split)
 void launch_gdn_backward(const GdnBwd& p);
-// the operand records (the least a call needs); with the time split's buffers when it
-// applies (gdn_split_segments >= 2)
+// the operand records (the least a call needs); with the buffers of gdn_split_segments time
+// segments
 size_t gdn_forward_workspace(int B, int T, int H, int N);
 size_t gdn_forward_workspace_split(int B, int T, int H, int N, int cus);
 // with the buffers of as many segments as help, without and with saved states

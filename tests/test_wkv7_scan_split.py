@@ -31,7 +31,11 @@ def test_saved_state_split_against_one_pass(N, B, T, H, cus, monkeypatch):
 @pytest.mark.parametrize("saved,N,H,n,split", [
     (True, 128, 8, 15, False), (True, 128, 8, 16, True), (True, 128, 17, 19, False), (True, 128, 17, 20, True),
     (True, 128, 33, 47, False), (True, 128, 33, 48, True), (True, 128, 43, 63, False), (True, 128, 43, 64, True),
-    (True, 128, 86, 100, False), (True, 64, 20, 28, False), (True, 64, 20, 29, True), (True, 64, 86, 40, False)])
+    (True, 128, 86, 100, False), (True, 64, 20, 28, False), (True, 64, 20, 29, True), (True, 64, 86, 40, False)] + [
+    (False, *case) for case in [(128, 8, 19, False), (128, 8, 20, True), (128, 33, 47, False), (128, 33, 48, True),
+                                         (128, 43, 47, False), (128, 43, 48, True), (128, 65, 100, False),
+                                         (64, 16, 15, False), (64, 16, 16, True), (64, 17, 19, False), (64, 17, 20, True),
+                                         (64, 80, 47, False), (64, 80, 48, True), (64, 129, 50, False)]])
 def test_forward_split_where_it_pays(saved, N, H, n, split, monkeypatch):
     """The forward, with saved states or without, given its best workspace, against the same
     records in one pass (a workspace of the records alone): the same bits where the rule keeps
