@@ -6,6 +6,8 @@ include/theseus_wkv7.h is looked up, and argument validation is exercised
 """
 import ctypes
 import re
+import shutil
+import subprocess
 from pathlib import Path
 
 import pytest
@@ -336,3 +338,20 @@ def test_backward_record_scans_are_cut_where_it_pays(monkeypatch):
         for n in (1, 7, 8, 16, 19, 20, 28, 47, 48, 64, 96, 200):
             k = segments(H, n)
             assert k == 1 or 4 <= k <= 9 and (k - 1) * H <= 256 and 4 * k <= n
+
+
+@pytest.mark.skipif(shutil.which("make") is None, reason="needs make")
+def test_the_c_library_builds_without_torch():
+    """The default target leaves theseus._native out where Python has no torch, and `make lib` does
+    anywhere (dry runs: every command is printed, none is run)."""
+    def commands(*args):
+        r = subprocess.run(["make", "-n", "-B", "-C", str(ROOT / "rwkv-theseus_amd" / "csrc"), *args], text=True,
+                           capture_output=True, timeout=120)
+        assert r.returncode == 0, r.stderr
+        return r.stdout
+
+    for args in (("PYTHON=false",), ("lib",)):
+        out = commands(*args)
+        assert "libtheseus_wkv7.so" in out and "torch_bind" not in out and "_native.so" not in out
+    out = commands()
+    assert "torch_bind" in out and f"_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)} " in out
