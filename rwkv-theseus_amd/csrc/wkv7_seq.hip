@@ -29,6 +29,7 @@
 #include "wkv7_common.h"
 #include "wkv7_io.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace wkv7 {
@@ -72,12 +73,12 @@ __device__ __forceinline__ float one_or(uint32_t m, float x) {  // x where the m
 // ---------------------------------------------------------------------------
 template <typename T, int NP, int MODE, int W>
 __global__ __launch_bounds__(W) void seq_forward(
-    int Tn, int H, int N, int kv, int blocks, const T* __restrict__ r, const T* __restrict__ w,
+    int Tn, int H, int N, int kv, int bh0, int blocks, const T* __restrict__ r, const T* __restrict__ w,
     const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ a,
     const T* __restrict__ b, const float* s0, T* __restrict__ y,
     float* sT, float* __restrict__ ckpt) {
     constexpr int G = NP / 4, RB = W / G, M = CKPT * NP / W, MV = (CKPT * RB + W - 1) / W, YR = (CKPT + G - 1) / G;
-    const int bh = blockIdx.x / blocks, row0 = (blockIdx.x - bh * blocks) * RB;
+    const int hd = blockIdx.x / blocks, bh = bh0 + hd, row0 = (blockIdx.x - hd * blocks) * RB;
     const int bb = bh / H, h = bh - bb * H, tid = threadIdx.x;
     const int kg = tid % G, rl = tid / G, i = row0 + rl, j0 = 4 * kg;
     const bool row = i < N;
@@ -184,11 +185,11 @@ __global__ __launch_bounds__(W) void seq_forward(
 // ---------------------------------------------------------------------------
 template <typename T, int NP, int MODE, int W>
 __global__ __launch_bounds__(W) void seq_grad_scan(
-    int Tn, int H, int N, int kv, int blocks, int c0, int c1, const T* __restrict__ r, const T* __restrict__ w,
+    int Tn, int H, int N, int kv, int bh0, int blocks, int c0, int c1, const T* __restrict__ r, const T* __restrict__ w,
     const T* __restrict__ a, const T* __restrict__ b, const T* __restrict__ dy, const float* gin, float* gout,
     float* __restrict__ hbuf) {
     constexpr int G = NP / 4, RB = W / G, M = CKPT * NP / W, MV = (CKPT * RB + W - 1) / W;
-    const int bh = blockIdx.x / blocks, row0 = (blockIdx.x - bh * blocks) * RB;
+    const int hd = blockIdx.x / blocks, bh = bh0 + hd, row0 = (blockIdx.x - hd * blocks) * RB;
     const int bb = bh / H, h = bh - bb * H, tid = threadIdx.x;
     const int kg = tid % G, rl = tid / G, i = row0 + rl, j0 = 4 * kg;
     const bool row = i < N;
@@ -289,7 +290,7 @@ static_assert(sizeof(SeqBwdLds<32>) <= 163840 && sizeof(SeqBwdLds<64>) <= 163840
               "LDS of a CU");
 template <typename T, int NP, int MODE>
 __global__ __launch_bounds__(seq_bwd_lanes<NP>()) void seq_backward(
-    int Tn, int H, int N, int c0, int nseg, const T* __restrict__ r, const T* __restrict__ w,
+    int Tn, int H, int N, int bh0, int c0, int nseg, const T* __restrict__ r, const T* __restrict__ w,
     const T* __restrict__ k, const T* __restrict__ v, const T* __restrict__ a,
     const T* __restrict__ b, const float* __restrict__ ckpt, const T* __restrict__ dy,
     T* __restrict__ dr, T* __restrict__ dw, T* __restrict__ dk, T* __restrict__ dv, T* __restrict__ da,
@@ -299,7 +300,7 @@ __global__ __launch_bounds__(seq_bwd_lanes<NP>()) void seq_backward(
     constexpr int M = CKPT * NP / W, YR = (CKPT + G - 1) / G;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     Lds& sm = *reinterpret_cast<Lds*>(lds_raw);
-    const int bh = blockIdx.x / nseg, cw = blockIdx.x - bh * nseg, c = c0 + cw;
+    const int hd = blockIdx.x / nseg, bh = bh0 + hd, cw = blockIdx.x - hd * nseg, c = c0 + cw;
     const int bb = bh / H, h = bh - bb * H, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int kg = tid % G, rl = tid / G, j0 = 4 * kg, t0 = c * CKPT;
     const long NN = (long)N * N, ncp = ckpt_count(Tn);
@@ -329,8 +330,8 @@ __global__ __launch_bounds__(seq_bwd_lanes<NP>()) void seq_backward(
         }
     }
     __syncthreads();
-    // columns [5][NP] of a step (dr, dw, dk, db, da), summed over the waves by five (WAVES = 4:
-    // all) of them in turn; each column's lane is the same in every pass
+    // columns [5][NP] of a step (dr, dw, dk, db, da), summed over the waves by LW of them (2 of 4,
+    // 5 of 16, all 8 at NP = 32, 64, 128) in turn; each column's lane is the same in every pass
     auto columns = [&](int u, int pass, const float (&part)[WAVES][5 * NP]) {
         constexpr int LW = 5 * NP / 64 > WAVES ? WAVES : 5 * NP / 64;  // waves at work per step
         const int first = (u * LW) % WAVES, slot = (wave - first + WAVES) % WAVES;
@@ -481,6 +482,11 @@ template <typename F> void by_width(int BH, int NP, F&& f) {
     if (NP > 32 && BH >= 256) f(std::integral_constant<int, 1024>());
     else f(std::integral_constant<int, 256>());
 }
+// f(first head, heads) in as few launches as the grid takes: at most 2^32 - 1 lanes along x.
+template <typename F> void by_heads(int BH, int lanes_per_head, F&& f) {
+    const unsigned most = 0xffffffffu / (unsigned)lanes_per_head;
+    for (unsigned h = 0, n; h < (unsigned)BH; h += n) f((int)h, n = std::min((unsigned)BH - h, most));
+}
 template <typename F> void by_shape(int N, int dtype, int flags, F&& f) {
     auto mode = [&](auto t, auto np) {
         if (flags & FLAG_DECAY_EXP) f(t, np, std::integral_constant<int, MODE_EXP>());
@@ -504,10 +510,12 @@ void launch_seq_forward(const Fwd& p) {
         by_width(p.B * p.H, NP, [&](auto width) {
             constexpr int W = decltype(width)::value, WW = NP == 32 ? 256 : W, RB = 4 * WW / NP;
             const int blocks = (p.N + RB - 1) / RB;
-            hipLaunchKernelGGL((seq_forward<T, NP, MODE, WW>), dim3((unsigned)(p.B * p.H * blocks)), dim3(WW), 0,
-                               p.stream, p.T, p.H, p.N, (p.flags & FLAG_STATE_KV) ? 1 : 0, blocks, (const T*)p.r,
-                               (const T*)p.w, (const T*)p.k, (const T*)p.v, (const T*)p.a, (const T*)p.b, p.s0,
-                               (T*)p.y, p.sT, p.ckpt);
+            by_heads(p.B * p.H, blocks * WW, [&](int bh0, unsigned heads) {
+                hipLaunchKernelGGL((seq_forward<T, NP, MODE, WW>), dim3(heads * blocks), dim3(WW), 0, p.stream, p.T,
+                                   p.H, p.N, (p.flags & FLAG_STATE_KV) ? 1 : 0, bh0, blocks, (const T*)p.r,
+                                   (const T*)p.w, (const T*)p.k, (const T*)p.v, (const T*)p.a, (const T*)p.b, p.s0,
+                                   (T*)p.y, p.sT, p.ckpt);
+            });
         });
     });
 }
@@ -531,15 +539,19 @@ void launch_seq_backward(const Bwd& p) {
                 constexpr int W = decltype(width)::value, WW = NP == 32 ? 256 : W, RB = 4 * WW / NP;
                 // (every padded row runs: the segment kernel reads hbuf's padding too)
                 const int blocks = NP / RB;
-                hipLaunchKernelGGL((seq_grad_scan<T, NP, MODE, WW>), dim3((unsigned)(BH * blocks)), dim3(WW), 0,
-                                   p.stream, p.T, p.H, p.N, kv, blocks, c0, c1, (const T*)p.r, (const T*)p.w,
-                                   (const T*)p.a, (const T*)p.b, (const T*)p.dy, c1 == nseg ? p.dsT : p.ds0, p.ds0,
-                                   (float*)p.ws);
+                by_heads(BH, blocks * WW, [&](int bh0, unsigned heads) {
+                    hipLaunchKernelGGL((seq_grad_scan<T, NP, MODE, WW>), dim3(heads * blocks), dim3(WW), 0, p.stream,
+                                       p.T, p.H, p.N, kv, bh0, blocks, c0, c1, (const T*)p.r, (const T*)p.w,
+                                       (const T*)p.a, (const T*)p.b, (const T*)p.dy, c1 == nseg ? p.dsT : p.ds0,
+                                       p.ds0, (float*)p.ws);
+                });
             });
-            hipLaunchKernelGGL((seq_backward<T, NP, MODE>), dim3((unsigned)(BH * (c1 - c0))), dim3(Lds::W),
-                               sizeof(Lds), p.stream, p.T, p.H, p.N, c0, c1 - c0, (const T*)p.r, (const T*)p.w,
-                               (const T*)p.k, (const T*)p.v, (const T*)p.a, (const T*)p.b, p.ckpt, (const T*)p.dy,
-                               (T*)p.dr, (T*)p.dw, (T*)p.dk, (T*)p.dv, (T*)p.da, (T*)p.db, (const float*)p.ws);
+            by_heads(BH, (c1 - c0) * Lds::W, [&](int bh0, unsigned heads) {
+                hipLaunchKernelGGL((seq_backward<T, NP, MODE>), dim3(heads * (c1 - c0)), dim3(Lds::W), sizeof(Lds),
+                                   p.stream, p.T, p.H, p.N, bh0, c0, c1 - c0, (const T*)p.r, (const T*)p.w,
+                                   (const T*)p.k, (const T*)p.v, (const T*)p.a, (const T*)p.b, p.ckpt, (const T*)p.dy,
+                                   (T*)p.dr, (T*)p.dw, (T*)p.dk, (T*)p.dv, (T*)p.da, (T*)p.db, (const float*)p.ws);
+            });
         }
     });
 }

@@ -107,6 +107,24 @@ def test_infinite_inputs_stay_in_their_columns():
 
 
 @pytest.mark.filterwarnings("ignore::RuntimeWarning")
+def test_more_heads_than_one_launch_takes():
+    """16777296 heads at 256 lanes each are more lanes than a grid has (2^32 - 1): the same bits as
+    from two calls of half the heads."""
+    H, N, T, ext = 2 ** 23 + 40, 4, 2, W.extension()
+    g = torch.Generator(device="cuda").manual_seed(6)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    xs, s0, dy, dsT = [rnd(2, T, H, N) for _ in range(6)], rnd(2, H, N, N), rnd(2, T, H, N), rnd(2, H, N, N)
+
+    def run(b):
+        y, sT, saved = ext.forward(*[x[b] for x in xs], s0[b], True)
+        return y, sT, *ext.backward(*[x[b] for x in xs], saved, dy[b], dsT[b])
+
+    whole, halves = run(slice(0, 2)), [run(slice(0, 1)), run(slice(1, 2))]
+    for name, a, *bs in zip(NAMES, whole, *halves):
+        assert all(torch.equal(a[i:i + 1], b) for i, b in enumerate(bs)), name
+
+
+@pytest.mark.filterwarnings("ignore::RuntimeWarning")
 @pytest.mark.parametrize("T", [1, 3, 16, 17, 31])
 @pytest.mark.parametrize("N", [32, 64, 128])
 def test_infinities_in_the_last_segment(N, T):
