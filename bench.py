@@ -285,7 +285,7 @@ def bench_gdn(args, cfg):
     with the layers' in-kernel q/k L2 norm, through theseus.gdn: the forward on the chunked
     MFMA kernels (theseus_gdn_forward: gdn_prep, gdn_scan), forward+backward on the chunked
     kernels too (theseus_gdn_forward_train with saved states, theseus_gdn_backward:
-    gdn_bwd_prep, wkv7_bwd_scan, gdn_bwd_chunk; float32 operands as transformers computes);
+    gdn_bwd_prep, wkv7_bwd_scan, gdn_bwd_chunk; float32 inside as transformers computes);
     beside transformers' torch_chunk_gated_delta_rule (its torch fallback, the function the
     reference's teacher runs without FLA) and the step-serial forward of the same call."""
     import inspect
@@ -376,7 +376,7 @@ def bench_gdn(args, cfg):
         "vs_baseline": None, "dtype": "bf16 I/O, fp32 compute", "data": "synthetic",
         "config": {"workload": "gdn_forward", "B": B, "T": T, "H": H, "K": N, "V": N,
                    "kernels": "forward: chunked MFMA GDN (gdn_prep + gdn_scan); fwd+bwd: the same with saved "
-                              "states, then gdn_bwd_prep + wkv7_bwd_scan + gdn_bwd_chunk (float32 operands)"},
+                              "states, then gdn_bwd_prep + wkv7_bwd_scan + gdn_bwd_chunk"},
         "ms_by_impl": {k2: round(v2, 4) for k2, v2 in ms.items()},
         "speedup_vs_transformers_torch_chunk": round(ms["transformers_torch_chunk_fwd"] / ms["ours_fwd"], 2),
         "speedup_fwd_bwd_vs_transformers_torch_chunk": round(ms["transformers_torch_chunk_fwd_bwd"] /

@@ -34,9 +34,11 @@ typedef struct ihipStream_t* hipStream_t;
  *   N = 64 or 128 (else THESEUS_WKV7_ERR_SHAPE); workspace of
  *   theseus_gdn_forward_workspace_size bytes (every 16-step chunk's operands,
  *   42 KB per chunk at N = 128, and, with few heads -- B*H*N/64 workgroups at
- *   most half the CUs, T > 112 -- the buffers of the time-split scan, which
- *   cuts each head's chunks into k = min(4, CUs / (B*H*N/64)) segments run at
- *   once; a workspace of just the operand records runs the one-pass scan, to
+ *   most half the CUs, T > 112 -- the buffers of min(4, CUs / (B*H*N/64)) time
+ *   segments, one workgroup per CU, which the scan runs at once: up to that many
+ *   where cutting a head pays, from 16 to 96 chunks on by head size and heads,
+ *   and up to 8 given theseus_gdn_forward_best_workspace_size of theseus_gdn_ex.h;
+ *   a workspace of just the operand records runs the one-pass scan, to
  *   float32 rounding the same), not shared with a call that can run at the
  *   same time.  Replaces the forward of transformers' torch_chunk_gated_delta_rule
  *   (chunk_size is not used) and torch_recurrent_gated_delta_rule. */
@@ -50,8 +52,9 @@ size_t theseus_gdn_forward_workspace_size(int B, int T, int H, int N);
 /* The forward of a call that needs gradients: as theseus_gdn_forward with q and k used as
  * given (a layer that normalises them does so before, differentiably), and also the saved
  * states ckpt [B,H,ceil(T/16)+1,N,N] float32 (the state after steps 0, 16, 32, ... and the
- * final one, in the library's own [value][key] order) for theseus_gdn_backward; the scan
- * runs in one pass (no time split).  Replaces the forward of transformers'
+ * final one, in the library's own [value][key] order) for theseus_gdn_backward.  Few heads
+ * and many chunks: the scan runs in up to 9 time segments, as many as the workspace holds
+ * (theseus_gdn_forward_best_workspace_size; the operand records alone run one pass).  Replaces the forward of transformers'
  * torch_chunk_gated_delta_rule under autograd (theseus/hf_model.py:37-48 keeps it for
  * such calls). */
 int theseus_gdn_forward_train(int B, int T, int H, int N, int dtype, const void* q, const void* k,
@@ -63,9 +66,11 @@ int theseus_gdn_forward_train(int B, int T, int H, int N, int dtype, const void*
  * caller's stream: q, k, v, g, beta and ckpt as that forward had them, dout [B,T,H,N] in
  * dtype, dsT [B,H,key,value] float32 (may be NULL: zero); writes dq, dk, dv [B,T,H,N] in
  * dtype, dg, dbeta [B,T,H] float32 and ds0 [B,H,key,value] float32.  Workspace of
- * theseus_gdn_backward_workspace_size bytes (24.5 KB of scan records and a 64 KB float32
- * dL/dS per 16-step chunk and head), not shared with a call that can run at the same
- * time.  Replaces the backward of transformers' torch_chunk_gated_delta_rule. */
+ * theseus_gdn_backward_workspace_size bytes, not shared with a call that can run at the same
+ * time: 24.5 KB of scan records and a 64 KB float32 dL/dS per 16-step chunk and head, which
+ * a call needs (else THESEUS_WKV7_ERR_WORKSPACE), and with few heads and many chunks
+ * 2k - 3 states of 64 KB per head for k <= 9 time segments of the reverse scan (given fewer,
+ * it runs in fewer, or in one pass).  Replaces the backward of transformers' torch_chunk_gated_delta_rule. */
 int theseus_gdn_backward(int B, int T, int H, int N, int dtype, const void* q, const void* k,
                          const void* v, const float* g, const float* beta, const float* ckpt,
                          const void* dout, const float* dsT, void* dq, void* dk, void* dv,

@@ -128,11 +128,11 @@ long long theseus_wkv7_checkpoint_count(int T);
  * chunked kernels use it when B*H heads outnumber the device's CUs: heads are
  * then cut between workgroups, which hand the carried state over through it;
  * the step-serial backward keeps dL/dS at every 16-step segment's end in it;
- * the chunk-record kernels their records, states and the segments of their
- * scans.  For few
- * heads (chunked kernels, 2*B*H <= CUs, T > 112) the forward size also covers
- * the time-split forward: a forward without saved states given that much cuts
- * every head's steps into k = min(4, CUs / (B*H)) segments that run at once,
+ * the chunk-record kernels their records, states and the time segments of
+ * their scans (a backward given less than its size runs in fewer segments, or, at
+ * N = 64, on the chunked kernels).  For few heads (chunked kernels, 2*B*H <= CUs,
+ * T > 112) the forward size also covers the time-split forward: a forward without
+ * saved states given that much cuts every head's steps into k = min(4, CUs / (B*H)) segments that run at once,
  * one workgroup each, and chains them with a fix-up kernel; it agrees with
  * the one-pass kernels to float32 rounding.  Given less (none is needed at
  * such sizes) it runs the one-pass kernels.  The split's buffers are
@@ -146,9 +146,9 @@ size_t theseus_wkv7_backward_workspace_size(int B, int T, int H, int N, int dtyp
 /* The workspace with which a forward runs fastest, at least theseus_wkv7_forward_workspace_size:
  * more for calls whose few heads leave CUs idle.  saved_states: whether ckpt is given.
  *  - bf16, N = 64 with saved states and few heads (n = ceil(T/16) > 28 chunks,
- *    B*H <= CUs/4, (3 CUs/10 - B*H) n > 760): the chunk records of the two-launch form and its time split
- *    (the saved states' order does not depend on it);
- *  - bf16, N = 128: the buffers of up to 9 time segments. */
+ *    B*H <= CUs/4, (3 CUs/10 - B*H) n > 760, at most 1 GiB each way): the chunk records of the
+ *    two-launch form and its time split (the saved states' order does not depend on it);
+ *  - bf16, N = 128: the buffers of up to 9 time segments with saved states, 8 without. */
 size_t theseus_wkv7_forward_best_workspace_size(int B, int T, int H, int N, int dtype, int saved_states);
 
 /* Forward recurrence.  Replaces wkv_forward (kernels/wkv7_state.cpp:16-25)

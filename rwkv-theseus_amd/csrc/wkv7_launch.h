@@ -88,9 +88,10 @@ struct Gdn {
     hipStream_t stream;
     size_t ws_bytes = 0;  // bytes at ws: the time-split scan runs when they cover its buffers
     int cus = 0;          // CUs the time split may spread the segments over (0: no split)
-    float* ckpt = nullptr;  // saved states for gdn backward ([value][key], every 16 steps + final); no split
+    float* ckpt = nullptr;  // saved states for gdn backward ([value][key], every 16 steps + final)
 };
-// Its backward for N = 128 (wkv7_rec_bwd.hip): q, k and qk_norm as the forward had them, dout [B,T,H,N] and the gradients of q, k, v in dtype; g, beta and their
+// Its backward for N = 128 (wkv7_rec_bwd.hip): q, k and qk_norm as the forward had them,
+// dout [B,T,H,N] and the gradients of q, k, v in dtype; g, beta and their
 // gradients [B,T,H] float32; dsT (may be null) and ds0 [B,H,key,value]; the forward's
 // saved states; a workspace of gdn_backward_workspace bytes.
 struct GdnBwd {

@@ -1,4 +1,5 @@
-// WKV7 backward for head size 128 (bf16) on the matrix cores, every chunk at once.
+// WKV7 backward (bf16, head size 128, and 64 with few heads) and the gated delta rule's (head
+// size 128) on the matrix cores, every chunk at once.
 //
 // The chunk form of the recurrence (kernels/wkv7_state.cu:12-79; operands A~, R~, B-, K-,
 // B^, K^, Aab, Aak, Brb, Brk, Ti, P, P2 as in wkv7_chunk_fwd.hip, decays per key) gives,
@@ -21,12 +22,13 @@
 // Three kernels.  wkv7_bwd_prep (one wave per chunk, all at once) writes each chunk's
 // record for the scan: B^ as the K=32 A operand over the keys, [P | P2] per 16-key tile
 // as the A operand of the K=32 update, e^{gL} per key.  wkv7_bwd_scan walks each head's
-// chunks backwards (one workgroup per 64 value rows of H, fp32 in registers, records
+// chunks backwards (fp32 H in registers, one wave per 16 of its value rows; a workgroup holds
+// 64 rows, or all of a head's where time segments fill the CUs that way; records
 // double-buffered in LDS by DMA as gdn_scan's), storing H at every chunk's end in the
-// workspace and the first chunk's start as ds0.  wkv7_bwd_chunk then forms every
-// chunk's gradients independently (eight waves; wave w owns value rows 16w..16w+15 for
-// SA, Q, dV and keys 16w..16w+15 for dK, dB, dR, dA, dw), with the chunk's matrices from
-// wkv7_bwd_prep.
+// workspace and the first chunk's start as ds0, in one pass or cut in time (wkv7_scan.h).
+// wkv7_bwd_chunk then forms every chunk's gradients independently (N/16 waves; wave w owns
+// value rows 16w..16w+15 for SA, Q, dV and keys 16w..16w+15 for dK, dB, dR, dA, dw), with the
+// chunk's matrices from wkv7_bwd_prep (the gated delta rule's gdn_bwd_chunk forms its own).
 #include "wkv7_launch.h"
 #include "wkv7_scan.h"
 
@@ -197,12 +199,13 @@ __global__ __launch_bounds__(64, NK == 64 ? 4 : 3) void wkv7_bwd_prep(int Tn, in
 }
 
 // ---------------------------------------------------------------------------
-// Each head's chunks backwards: workgroup rg * BH + bh, four waves, wave wv of group rg
-// keeps value rows i_own = 16 (4 rg + wv) + r16 of H as Ht[tj][e] = H[i_own][16tj + 4q4 + e].
+// Each head's chunks backwards: workgroup (segment * RGS + rg) * BH + bh of NW waves (4, or
+// N/16: all of a head's rows), wave wv of row group rg keeps value rows
+// i_own = 16 (NW rg + wv) + r16 of H as Ht[tj][e] = H[i_own][16tj + 4q4 + e].
 // Per chunk: H is stored (the chunk kernel's H_end), U^T = B^ H^T over the keys, then
 // H^T <- e^{gL} o H^T + [P^T | P2^T] [U^T; dY] on the K=32 instruction.  dY of dtype TI;
 // dsT (may be null) and ds0 [key][value] when kv (GDN's layout), else [value][key]; H in
-// the workspace always [value][key].
+// the workspace always [value][key].  MODE: the time split's launches (ScanMode).
 // ---------------------------------------------------------------------------
 template <int NK, typename TI, ScanMode MODE>
 __global__ __launch_bounds__(4 * NK) void wkv7_bwd_scan(int Tn, int H, int BH, int kv, const float* __restrict__ dsT,
